@@ -31,8 +31,8 @@ sys.path.insert(0, ROOT)
 METRIC = "slices/s at 2048^2 x1500 proj, FP32 vs FP16 at rel-L2 vs FP64; HBM GB/s"
 HBM_PEAK_GBS = 8000.0
 ISO_CHUNKS = 16  # chunks of the untimed one-stream breakdown pass
-KERNELS = ['k_pre_means', 'k_pre_rows', 'k_fw_rows', 'k_fw_cols', 'k_fw_xsum', 'k_fw_syn_cols',
-           'k_fw_syn_rows', 'k_pre_log_swap', 'k_flt_weights', 'k_flt_rows', 'k_flt_prepare',
+KERNELS = ['k_pre_means', 'k_pre_rows', 'k_fw_project', 'k_fw_detector', 'k_fw_apply',
+           'k_pre_log_swap', 'k_flt_weights', 'k_flt_rows', 'k_flt_prepare',
            'k_fr_prep', 'k_fr_filtprep',
            'k_fr_gscale', 'k_fr_grid_x3', 'k_fr_grid16', 'k_fr_grid_reduce', 'k_fr_rowfft',
            'k_fr_colfft', 'k_pre_median', 'k_pre_dezinger', 'k_ti_mean', 'k_ti_conv', 'k_ti_add',
@@ -89,43 +89,27 @@ def parse():
     return ap.parse_args()
 
 
-def fw_levels(a, L=32):
-    """Band shapes (H, W, Ho, Wo, Hs, Ws) of the sym16 Fourier-wavelet levels."""
-    H, W = a.nproj + a.nproj // 8, a.n
-    out = []
+def fw_terms(a, L=32, sigma=1.0):
+    """Terms of the sym16 stripe removal: the kept cosines and sines of the
+    notch of each level."""
+    H, terms = a.nproj + a.nproj // 8, 0
     for _ in range(a.fw_level):
-        Ho, Wo = (H + L - 1) // 2, (W + L - 1) // 2
-        out.append((H, W, Ho, Wo, 2 * Ho - L + 2, 2 * Wo - L + 2))
-        H, W = Ho, Wo
-    return out
+        H = (H + L - 1) // 2
+        for q in range(H // 2 + 1):
+            y = (-H + 2 * ((q + H // 2) % H) + 1) / 2
+            if np.exp(-y * y / (2 * sigma * sigma)) >= 1e-9:
+                terms += 1 if q == 0 or 2 * q == H else 2
+    return terms
 
 
 def fw_bytes(name, a):
-    """Mean external I/O per launch of a Fourier-wavelet kernel (one launch per
-    level and chunk, levels launched equally often; correction form: the
-    column analysis writes ll only, the column synthesis reads the
-    correction of the level below, the last pass reads the raw counts and
-    writes the sinograms at storage precision)."""
-    ch = a.chunk
+    """External I/O per launch of a Fourier-wavelet kernel: the counts into the
+    angle contraction (FP64 sums out), the sums to three bfloat16 parts, the
+    counts to the sinograms at storage precision."""
     r = 4 if a.dtype == 'float32' else 2
-    per = []
-    for k, (H, W, Ho, Wo, Hs, Ws) in enumerate(fw_levels(a)):
-        if name == 'k_fw_rows':      # read the rows (level 0: uint16 counts), write lo+hi
-            rd = 2 * a.nproj * a.n if k == 0 else 4 * H * W
-            per.append(ch * (rd + 4 * 2 * H * Wo))
-        elif name == 'k_fw_cols':    # read lo+hi, write ll
-            per.append(4 * ch * (2 * H * Wo + Ho * Wo))
-        elif name == 'k_fw_syn_cols':  # read the correction of the level below, write lo+hi
-            rd = 0 if k == len(fw_levels(a)) - 1 else Ho * Wo
-            per.append(4 * ch * (rd + 2 * Hs * Wo))
-        elif name == 'k_fw_syn_rows':  # read lo+hi (last: + counts), write the correction / sinograms
-            if k == 0:
-                per.append(ch * (4 * 2 * Hs * Wo + 2 * a.nproj * a.n + r * a.nproj * a.n))
-            else:
-                per.append(4 * ch * (2 * Hs * Wo + Hs * Ws))
-        else:
-            return None
-    return sum(per) // len(per)
+    sino, rows = a.chunk * a.nproj * a.n, a.chunk * fw_terms(a) * a.n
+    return {'k_fw_project': 2 * sino + 8 * rows, 'k_fw_detector': (8 + 6) * rows,
+            'k_fw_apply': 6 * rows + (2 + r) * sino}.get(name)
 
 
 def algorithmic_bytes(name, a, s):
@@ -494,8 +478,8 @@ def bench_steps(a):
     torch.cuda.synchronize()
     _lib.prof_enable(False)
     kern = {}
-    for k in ('k_ph_rows_fwd', 'k_ph_cols', 'k_ph_rows_inv', 'k_pre_log_swap', 'k_fw_rows',
-              'k_fr_grid_x3', 'k_pre_rows'):
+    for k in ('k_ph_rows_fwd', 'k_ph_cols', 'k_ph_rows_inv', 'k_pre_log_swap', 'k_fw_project',
+              'k_fw_detector', 'k_fw_apply', 'k_fr_grid_x3', 'k_pre_rows'):
         ms, cnt = _lib.prof_read(k)
         if cnt:
             kern[k] = {'avg_ms': round(ms / cnt, 5), 'launches': cnt, 'total_ms': round(ms, 3)}

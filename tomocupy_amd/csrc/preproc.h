@@ -31,29 +31,40 @@ struct VoBufs {
   }
 };
 
-// One level of the Fourier-wavelet stripe removal: analysis input H x W,
-// bands Ho x Wo; the notch keeps nk angular frequencies of the stripe band.
-struct FwLevel {
-  int H = 0, W = 0, Ho = 0, Wo = 0;
-  int nk = 0;
-  int KM = 8;   // notch frequencies a kernel instance holds (8, 16 or 32 >= nk)
-  int R = 8;    // output rows per wave of the column analysis
-  int nrb = 0;  // row blocks of the column analysis
-  DevBuf tw;    // (nk, Ho) float2: cos/sin(2 pi k t / Ho)
-  DevBuf gk;    // (nk,) float: c_k g_k / Ho
-  DevBuf ll;    // (nz, Ho, Wo): low band = input of the next level
-  DevBuf part;  // (nz, nrb, KM, Wo) float2: partial notch DFTs of the stripe band
-  DevBuf X;     // (nz, KM, Wo) float2: notch coefficients, kept until the synthesis
+// Tables and scratch of the Fourier-wavelet stripe removal (stripe.hip),
+// (re)built when the settings change.
+struct FwPlan {
+  std::string name;  // wavelet; empty: nothing built
+  int level = 0;
+  double sigma = 0.0;
+  int R = 0, Rp = 0;    // terms, padded to the matrix products' 32
+  int steps = 0;        // 32-angle steps of an angle group
+  int Pt = 0, Pa = 0;   // padded angles of T and of A
+  int nPad = 0;         // padded columns of B
+  int len = 0;          // longest band along the detector
+  size_t lds = 0;       // k_fw_detector: its two rows; glob: they do not fit
+  bool glob = false;
+  DevBuf terms, T, TS, A;  // see k_fw_tables
+  DevBuf P, B, row;             // see k_fw_project, k_fw_detector
+  void release() {
+    name.clear();
+    for (DevBuf *b : {&terms, &T, &TS, &A, &P, &B, &row}) b->release();
+  }
 };
 
-// dark/flat correction of one count (proc_functions.py:67-74): flat0 =
-// flat mean (or the linear interpolation v of the two halves' means,
-// :62-66) * float32(1 + 1e-5) - dark0; result (x - dark0) / flat0
+// flat0 of a mean flat fa and a mean dark d0: fa * float32(1 + 1e-5) - d0
+// (proc_functions.py:71-72)
+__device__ __forceinline__ float flat0(float fa, float d0) {
+  const float eps = 1.0f + 1e-5f;
+  return fa * eps - d0;
+}
+
+// dark/flat correction of one count (proc_functions.py:67-74): flat0 of the
+// flat mean (or of the linear interpolation v of the two halves' means,
+// :62-66); result (x - dark0) / flat0
 __device__ __forceinline__ float darkflat(float x, float d0, float fa, float fb, float v,
                                           int flat_linear) {
-  const float eps = 1.0f + 1e-5f;  // float32(1 + 1e-5), proc_functions.py:71
-  float f0 = flat_linear ? (1.0f - v) * fa + v * fb : fa;
-  f0 = f0 * eps - d0;
+  const float f0 = flat0(flat_linear ? (1.0f - v) * fa + v * fb : fa, d0);
   return (x - d0) / f0;
 }
 
@@ -75,13 +86,7 @@ int pre_launch_means(tomo_pre_plan *P, const uint16_t *dark, const uint16_t *fla
 struct tomo_pre_plan {
   int64_t nproj = 0, nz = 0, n = 0, ndark = 0, nflat = 0;
   tomo::DevBuf dark0, flatA, flatB;
-  // Fourier-wavelet scratch, (re)built when the settings change
-  std::string fw_name;
-  int fw_levels = 0;
-  double fw_sigma = 0.0;
-  int fw_L = 0;
-  std::vector<tomo::FwLevel> lv;
-  tomo::DevBuf rowlo, rowhi, synlo, synhi, syn[2];
+  tomo::FwPlan fw;
   tomo::DevBuf outl;  // medians of pre_remove_outliers, allocated on first use
   tomo::DevBuf ti;    // column means and corrections of pre_remove_stripe_ti (first use)
   tomo::VoBufs vo;    // scratch of pre_remove_all_stripe (first use)

@@ -372,19 +372,7 @@ extern "C" void pre_destroy(tomo_pre_plan *P) {
   P->dark0.release();
   P->flatA.release();
   P->flatB.release();
-  for (auto &l : P->lv) {
-    l.tw.release();
-    l.gk.release();
-    l.ll.release();
-    l.part.release();
-    l.X.release();
-  }
-  P->rowlo.release();
-  P->rowhi.release();
-  P->synlo.release();
-  P->synhi.release();
-  P->syn[0].release();
-  P->syn[1].release();
+  P->fw.release();
   P->outl.release();
   P->ti.release();
   P->vo.release();
