@@ -1,4 +1,5 @@
 // Status handling, version string and FFT plan construction for libtomohip.
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstring>
@@ -6,6 +7,7 @@
 #include <mutex>
 #include <string>
 #include <tuple>
+#include <utility>
 
 #include "common.h"
 #include "fft_lds.h"
@@ -32,12 +34,11 @@ size_t max_lds_per_block() {
   return (size_t)v;
 }
 
-int FftPlan::radices(int N, FftDesc &d) {
+int FftPlan::radices(int N, FftRule &d) {
   TOMO_REQUIRE(fft_size_ok(N) && N <= 16384,
                "FFT length %d is not <= 16384 with prime factors <= %d", N, kFftMaxPrime);
   d.N = N;
   d.nr = 0;
-  d.tw = nullptr;
   int m = N;
   // radix 16 first (fewest passes), then 8, 4, 2, then 3s, 5s, 7s, then the
   // larger primes
@@ -53,9 +54,100 @@ int FftPlan::radices(int N, FftDesc &d) {
   return TOMO_OK;
 }
 
+namespace {
+
+// Vector instructions per element of a run-time pass: the butterfly, plus
+// loads, stores, twiddles and the index split.
+double rt_cost(int R) {
+  static const double f[21] = {0,  0, 3,  4.5, 4,  6.5, 6,  10, 6,  8,  8.5,
+                               15, 8, 18, 12,  10, 9.5, 24, 10, -1, 9.5};
+  return 11.0 + 24.0 / R + f[R];
+}
+
+}  // namespace
+
+void fft_rt_radices(int N, FftDesc &d) {
+  d.N = N;
+  d.nr = 0;
+  // primes above kFftRegPrime first (odd radices: no bank conflicts)
+  int m = N;
+  for (int p = kFftMaxPrime; p > kFftRegPrime; --p)
+    while (m % p == 0) {
+      bool prime = true;
+      for (int q = 2; q * q <= p; ++q) prime &= p % q != 0;
+      if (!prime) break;
+      d.r[d.nr++] = p;
+      m /= p;
+    }
+  // best[v]: the cheapest passes of the divisor v of m whose butterflies keep
+  // within 1024 threads
+  const int fixed = d.nr;
+  std::map<int, std::pair<double, int>> best;  // cost, radix taken
+  best[1] = {0.0, 1};
+  for (int v = 2; v <= m; ++v) {
+    if (m % v) continue;
+    std::pair<double, int> b{1e30, 0};
+    for (int R = 2; R <= kFftRtVals; ++R) {
+      if (R == 19 || v % R) continue;
+      if (N / R > 1024 * rt_maxb(R)) continue;
+      const auto it = best.find(v / R);
+      if (it == best.end()) continue;
+      const double c = it->second.first + rt_cost(R);
+      if (c < b.first) b = {c, R};
+    }
+    if (b.second) best[v] = b;
+  }
+  for (int v = m; v > 1;) {
+    const auto it = best.find(v);
+    if (it == best.end()) {  // not reached for the sizes the callers accept
+      d.nr = 0;
+      return;
+    }
+    d.r[d.nr++] = it->second.second;
+    v /= it->second.second;
+  }
+  // odd radices first, then the even ones whose stride-R writes meet the most
+  // banks (2 mod 4, then 4 mod 8, ...)
+  std::sort(d.r + fixed, d.r + d.nr, [](int a, int b) {
+    const int la = a & -a, lb = b & -b;
+    return la != lb ? la < lb : a > b;
+  });
+}
+
 int FftPlan::init(int N) {
-  int rc = radices(N, d);
+  int rc = radices(N, rule);
   if (rc) return rc;
+  fft_rt_radices(N, d);
+  TOMO_REQUIRE(d.nr > 0 && fft_rt_threads(d, 0) > 0, "FFT length %d has no run-time plan", N);
+  std::vector<float> mat;
+  size_t off[3] = {0, 0, 0};
+  int np = 0;
+  for (int i = 0; i < d.nr; ++i) {
+    const int p = d.r[i];
+    if (p <= kFftRtVals && p != 19) continue;
+    TOMO_REQUIRE(np < 3, "FFT length %d has more than three prime factors above %d", N,
+                 kFftRegPrime);
+    const int h = (p - 1) / 2, hp = rt_prime_cols(p);
+    off[np] = mat.size();
+    if (np > 0 && d.r[np - 1] == p) {
+      off[np] = off[np - 1];
+    } else {
+      mat.resize(mat.size() + (size_t)2 * h * hp, 0.f);
+      for (int j = 1; j <= h; ++j)
+        for (int q = 1; q <= h; ++q) {
+          const double ang = 2.0 * M_PI * (double)((j * q) % p) / (double)p;
+          float *e = &mat[off[np] + 2 * ((size_t)(j - 1) * hp + q - 1)];
+          e[0] = (float)std::cos(ang);
+          e[1] = (float)std::sin(ang);
+        }
+    }
+    ++np;
+  }
+  if (!mat.empty()) {
+    if ((rc = pm.alloc(sizeof(float) * mat.size()))) return rc;
+    TOMO_HIP(hipMemcpy(pm.p, mat.data(), sizeof(float) * mat.size(), hipMemcpyHostToDevice));
+    for (int i = 0; i < np; ++i) d.pm[i] = pm.as<float>() + off[i];
+  }
   std::vector<float2> h(N);
   for (int k = 0; k < N; ++k) {
     double a = -2.0 * M_PI * (double)k / (double)N;

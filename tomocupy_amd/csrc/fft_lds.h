@@ -1,8 +1,6 @@
 // LDS-resident Stockham autosort FFT for sizes N <= 16384 whose prime factors
 // are at most kFftMaxPrime (per transform), executed cooperatively by a
-// workgroup on 2^lgH interleaved transforms held in LDS.  Radices 2, 3, 4, 5,
-// 7, 8, 11, 13, 16 and 17 run as butterflies in registers; any other prime p
-// runs as a direct length-p DFT per output (fft_pass_gen).
+// workgroup on 2^lgH interleaved transforms held in LDS.
 //
 // Pass with radix R and current sub-transform length Ns (1, R1, R1*R2, ...):
 //   for j in [0, N/R):  k = j mod Ns
@@ -14,34 +12,59 @@
 // Twiddles come from a per-size table W_N^k = exp(-2 pi i k/N) computed on the
 // host in FP64; the inverse transform uses their conjugates.  Unnormalised in
 // both directions.
+//
+// Two forms: sizes 2^k 3^a 5^b of with_static_size() have everything constant
+// at compile time (lds_fft_c); any other size runs passes of radix 2..18, 20
+// and larger primes chosen at plan time (lds_fft).
 #pragma once
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 
 namespace tomo {
 
 constexpr int kFftMaxRadices = 16;
-constexpr int kFftEPT = 16;  // complex elements staged per thread per pass (max)
+constexpr int kFftEPT = 16;  // complex elements staged per thread per pass (compiled sizes)
 constexpr int kFftMaxPrime = 127;  // largest prime factor of a transform length
+constexpr int kFftRegPrime = 17;   // larger primes run wave-uniform (rt_pass_prime)
+constexpr int kFftRtVals = 20;     // values a thread holds in a run-time pass of small radix
 
+// A run-time plan: the passes in order and the tables they read.
 struct FftDesc {
   int N;
   int nr;
   int r[kFftMaxRadices];
-  const float2 *tw;  // device, N entries
+  const float2 *tw;    // device, N entries
+  const float *pm[3];  // cosine/sine matrices of the primes above kFftRegPrime, in pass order
 };
 
-// Host-side plan: radix sequence + device twiddle table.
+// The radix sequence of the compiled sizes; for every size the sequence by
+// which widths are accepted (fft_threads).
+struct FftRule {
+  int N;
+  int nr;
+  int r[kFftMaxRadices];
+};
+
+// Host-side plan: radix sequence + device tables.
 struct FftPlan {
   FftDesc d{};
-  DevBuf tw;
+  FftRule rule{};
+  DevBuf tw, pm;
   int init(int N);  // N <= 16384, prime factors <= kFftMaxPrime
-  // the radix sequence of init() alone (no device memory, no HIP call)
-  static int radices(int N, FftDesc &d);
+  // the rule's radix sequence alone (no device memory, no HIP call)
+  static int radices(int N, FftRule &r);
+  void release() {
+    tw.release();
+    pm.release();
+  }
 };
+
+// The passes of a run-time plan for length N (no HIP call).
+void fft_rt_radices(int N, FftDesc &d);
 
 template <int DIR>
 __device__ __forceinline__ float2 mul_i(float2 a) {
@@ -186,6 +209,13 @@ __device__ __forceinline__ int lds_pad(int i) { return i + (i >> 4); }
 // LDS elements needed for a padded transform of length N.
 __host__ __device__ inline int lds_padded_len(int N) { return N + (N >> 4); }
 
+// LDS index of element i of a transform: compiled size (NS > 0) or run-time
+// size (NS = 0).
+template <int NS>
+__device__ __forceinline__ int lidx(int i) {
+  return NS > 0 ? lds_pad(i) : i;
+}
+
 // a[r] *= w^r for r = 1..R-1 with w = W_N^base (conjugated for the inverse).
 // Powers of two of w come from the FP64-built table; the others are products
 // of at most three of them (relative error a few float32 ulps).
@@ -239,241 +269,389 @@ __device__ __forceinline__ void twiddle(float2 *a, const float2 *__restrict__ tw
   }
 }
 
-template <int R, int DIR, int EPT>
-__device__ __forceinline__ void fft_pass(float2 *buf, int N, int Ns, const float2 *tw, int lgH,
-                                         int tid, int nt) {
-  constexpr int MAXB = EPT / R;
-  const int H = 1 << lgH;
-  const int nbPer = N / R;
-  const int nb = nbPer << lgH;
-  const int twstep = N / (Ns * R);
-  const bool pow2 = (Ns & (Ns - 1)) == 0;
-  const int lgNs = pow2 ? __ffs(Ns) - 1 : 0;
-  const float invNs = 1.0f / (float)Ns;
-  // j -> (j / Ns, j % Ns); shifts when Ns is a power of two (all passes before
-  // the radix-3 ones), otherwise a float-reciprocal quotient with correction
-  auto split = [&](int j, int &jq, int &k) {
-    if (pow2) {
-      jq = j >> lgNs;
-      k = j & (Ns - 1);
-    } else {
-      jq = (int)((float)j * invNs);
-      k = j - jq * Ns;
-      if (k < 0) { jq -= 1; k += Ns; }
-      if (k >= Ns) { jq += 1; k -= Ns; }
-    }
+// ---- transforms of a run-time size -------------------------------------------
+// What bounds them: vector instructions, so the passes are few (radices up to
+// 20: three for the 2n of a detector) and their index arithmetic small: one
+// index split per butterfly, inputs at a uniform stride, no bank padding (an
+// odd radix goes first where there is one; its writes, R apart, then fall on
+// different banks).  Each pass sits behind a call, so a kernel's register
+// demand is its largest pass's; pointers carry their address space (a generic
+// one would turn every table read into a FLAT access).  The call's convention
+// spends 87 registers on the 64 a pass needs (5 waves per SIMD); inlined, the
+// switch spilled.  n = 2448 (2n = 17 18 16), 8 slices x 1500 angles, us, row
+// pass / column pass / filter and spectrum: 378 / 528 / 349, against 1211 /
+// 1123 / 1065 with radices 16, 2, 3, 3, 17 and per-element index arithmetic.
+
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) f2v *LdsPtr;
+typedef const __attribute__((address_space(1))) f2v *TabPtr;
+typedef const __attribute__((address_space(4))) float *ScalarPtr;
+
+__device__ __forceinline__ float2 ldf2(LdsPtr p) {
+  const f2v v = *p;
+  return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ float2 ldf2(TabPtr p) {
+  const f2v v = *p;
+  return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ void stf2(LdsPtr p, float2 v) { *p = f2v{v.x, v.y}; }
+
+// cos and sin(2 pi m / R) at compile time (Taylor series on [-pi, pi]).
+constexpr double cx_angle(int m, int R) {
+  const int q = ((m % R) + R) % R;
+  return 2.0 * 3.14159265358979323846 * (2 * q > R ? q - R : q) / R;
+}
+constexpr double cx_cos(int m, int R) {
+  const double x = cx_angle(m, R);
+  double t = 1.0, s = 1.0;
+  for (int i = 2; i < 40; i += 2) {
+    t *= -x * x / ((i - 1) * i);
+    s += t;
+  }
+  return s;
+}
+constexpr double cx_sin(int m, int R) {
+  const double x = cx_angle(m, R);
+  double t = x, s = x;
+  for (int i = 3; i < 40; i += 2) {
+    t *= -x * x / ((i - 1) * i);
+    s += t;
+  }
+  return s;
+}
+template <int M, int R>
+struct Root {
+  static constexpr float c = (float)cx_cos(M, R), s = (float)cx_sin(M, R);
+};
+
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F &&f) {
+  (f(std::integral_constant<int, I>()), ...);
+}
+// f(integral_constant<int, i>) for i = 0..N-1
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+  static_for_impl(std::make_integer_sequence<int, N>(), f);
+}
+
+// v * exp(DIR 2 pi i M / R)
+template <int M, int R, int DIR>
+__device__ __forceinline__ float2 rotate(float2 v) {
+  constexpr int m = M % R;
+  if constexpr (m == 0)
+    return v;
+  else if constexpr (2 * m == R)
+    return make_float2(-v.x, -v.y);
+  else if constexpr (4 * m == R)
+    return mul_i<DIR>(v);
+  else if constexpr (4 * m == 3 * R)
+    return mul_i<-DIR>(v);
+  else
+    return cmul(v, make_float2(Root<m, R>::c, DIR * Root<m, R>::s));
+}
+
+// First factor of the split R = A * B of a composite radix.
+constexpr int dft_split(int R) {
+  return R == 12 ? 4 : R == 20 ? 5 : R == 15 || R == 9 ? 3 : R == 18 ? 9 : 2;
+}
+
+// a <- DFT_R(a) in natural order, in registers, every constant a literal.
+template <int R, int DIR>
+__device__ __forceinline__ void dft(float2 *a) {
+  if constexpr (R <= 5 || R == 7 || R == 8) {
+    butterfly<R, DIR>(a);
+  } else if constexpr (R == 16) {
+    butterfly<16, DIR>(a);
+    float2 t[16];
+    static_for<16>([&](auto q) { t[q] = a[4 * (q & 3) + (q >> 2)]; });
+    static_for<16>([&](auto q) { a[q] = t[q]; });
+  } else if constexpr (R == 11 || R == 13 || R == 17) {
+    // cosine and sine pairs a_j +- a_(R-j)
+    constexpr int h = (R - 1) / 2;
+    float2 P[h + 1], M[h + 1];
+    const float2 a0 = a[0];
+    static_for<h>([&](auto i) {
+      constexpr int j = i + 1;
+      P[j] = cadd(a[j], a[R - j]);
+      M[j] = csub(a[j], a[R - j]);
+      a[0] = cadd(a[0], P[j]);
+    });
+    // (all real-coefficient sums, then all imaginary ones: P is dead before the
+    // second half, which keeps the registers of radix 17 at 80)
+    float2 re[h];
+    static_for<h>([&](auto i) {
+      constexpr int q = i + 1;
+      re[i] = a0;
+      static_for<h>([&](auto l) {
+        constexpr int j = l + 1, m = (j * q) % R;
+        re[i].x = fmaf(Root<m, R>::c, P[j].x, re[i].x);
+        re[i].y = fmaf(Root<m, R>::c, P[j].y, re[i].y);
+      });
+    });
+    static_for<h>([&](auto i) {
+      constexpr int q = i + 1;
+      float2 im = make_float2(0.f, 0.f);
+      static_for<h>([&](auto l) {
+        constexpr int j = l + 1, m = (j * q) % R;
+        im.x = fmaf(Root<m, R>::s, M[j].x, im.x);
+        im.y = fmaf(Root<m, R>::s, M[j].y, im.y);
+      });
+      const float2 mi = mul_i<DIR>(im);
+      a[q] = cadd(re[i], mi);
+      a[R - q] = csub(re[i], mi);
+    });
+  } else {
+    // n = B i1 + i2, k = k1 + A k2:
+    //   X[k] = sum_i2 W_B^(i2 k2) W_R^(i2 k1) sum_i1 W_A^(i1 k1) a[n]
+    constexpr int A = dft_split(R), B = R / A;
+    float2 c[R];
+    static_for<B>([&](auto i2) {
+      float2 t[A];
+      static_for<A>([&](auto i1) { t[i1] = a[B * i1 + i2]; });
+      dft<A, DIR>(t);
+      static_for<A>([&](auto k1) {
+        c[k1 * B + i2] = rotate<decltype(i2)::value * decltype(k1)::value, R, DIR>(t[k1]);
+      });
+    });
+    static_for<A>([&](auto k1) {
+      float2 t[B];
+      static_for<B>([&](auto i2) { t[i2] = c[k1 * B + i2]; });
+      dft<B, DIR>(t);
+      static_for<B>([&](auto k2) { a[k1 + A * k2] = t[k2]; });
+    });
+  }
+}
+
+// a[r] *= w^r, w = W_N^base (conjugated for the inverse): w, w^2 and every
+// fourth power from the table, the others products of two or three of them,
+// four at a time (few registers).
+template <int R, int DIR>
+__device__ __forceinline__ void rt_twiddle(float2 *a, TabPtr tw, unsigned base) {
+  auto ld = [&](unsigned r) {
+    float2 w = ldf2(tw + base * r);
+    if (DIR > 0) w.y = -w.y;
+    return w;
   };
+  float2 w[4];
+  w[1] = ld(1);
+  if constexpr (R > 2) w[2] = ld(2);
+  if constexpr (R > 3) w[3] = cmul(w[2], w[1]);
+  static_for<(R + 3) / 4>([&](auto blk) {
+    constexpr int r0 = 4 * blk;
+    float2 wb = make_float2(1.f, 0.f);
+    if constexpr (r0 > 0) {
+      wb = ld(r0);
+      a[r0] = cmul(a[r0], wb);
+    }
+    static_for<3>([&](auto i) {
+      constexpr int c = i + 1;
+      if constexpr (r0 + c < R) a[r0 + c] = cmul(a[r0 + c], r0 > 0 ? cmul(wb, w[c]) : w[c]);
+    });
+  });
+}
+
+// Butterflies of radix R a thread takes in a pass.
+constexpr int rt_maxb(int R) { return R <= kFftRtVals / 2 ? kFftRtVals / R : 1; }
+
+// One pass of radix R over 2^lgH interleaved transforms of length N (element
+// i of transform t at buf[(i << lgH) + t]); ends with a barrier.
+template <int R, int DIR>
+__device__ __noinline__ void rt_pass(LdsPtr buf, int N_, int Ns_, TabPtr tw, int lgH_, int tid,
+                                     int nt_) {
+  constexpr int MAXB = rt_maxb(R);
+  const int N = __builtin_amdgcn_readfirstlane(N_), Ns = __builtin_amdgcn_readfirstlane(Ns_);
+  const int lgH = __builtin_amdgcn_readfirstlane(lgH_), nt = __builtin_amdgcn_readfirstlane(nt_);
+  const int S = (N / R) << lgH;  // butterflies; distance between a butterfly's inputs
+  const int twstep = N / R / Ns;
+  const float invNs = 1.0f / (float)Ns;
   float2 v[MAXB][R];
+  int o[MAXB];
 #pragma unroll
   for (int q = 0; q < MAXB; ++q) {
     const int g = tid + q * nt;
-    if (g < nb) {
-      const int t = g & (H - 1), j = g >> lgH;
+    if (g < S) {
+      LdsPtr p = buf + g;
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[q][r] = buf[(lds_pad(j + r * nbPer) << lgH) + t];
-      if (Ns > 1) {
-        int jq, k;
-        split(j, jq, k);
-        twiddle<R, DIR>(v[q], tw, (unsigned)(k * twstep));
-      }
-      butterfly<R, DIR>(v[q]);
+      for (int r = 0; r < R; ++r) v[q][r] = ldf2(p + r * S);
+      const int j = g >> lgH;
+      // j / Ns and j mod Ns: float quotient, corrected
+      int jq = (int)((float)j * invNs), k = j - jq * Ns;
+      if (k < 0) jq -= 1, k += Ns;
+      if (k >= Ns) jq += 1, k -= Ns;
+      o[q] = ((jq * Ns * R + k) << lgH) + (g - (j << lgH));
+      if (Ns > 1) rt_twiddle<R, DIR>(v[q], tw, (unsigned)(k * twstep));
+      dft<R, DIR>(v[q]);
     }
   }
   __syncthreads();
+  const int W = Ns << lgH;
 #pragma unroll
   for (int q = 0; q < MAXB; ++q) {
-    const int g = tid + q * nt;
-    if (g < nb) {
-      const int t = g & (H - 1), j = g >> lgH;
-      int jq, k;
-      split(j, jq, k);
-      const int o = jq * Ns * R + k;
+    if (tid + q * nt < S) {
+      LdsPtr p = buf + o[q];
 #pragma unroll
-      for (int r = 0; r < R; ++r) buf[(lds_pad(o + r * Ns) << lgH) + t] = v[q][out_slot<R>(r)];
+      for (int r = 0; r < R; ++r) stf2(p + r * W, v[q][r]);
     }
   }
   __syncthreads();
 }
 
-// Radix-R pass for an odd prime 11 <= R <= 17 with the butterfly in
-// registers: inputs twiddled by W_N^(r k N/(Ns R)) from the table, then the
-// DFT from the cosine/sine pairs P_j = a_j + a_(R-j), M_j = a_j - a_(R-j):
-//   b_q, b_(R-q) = a_0 + sum_j cos(2 pi j q/R) P_j  -/+ i sum_j sin(2 pi j q/R) M_j
-// (signs of i swapped for the inverse), cos and sin read from the table
-// (W_R^m = W_N^(m N/R)).  One butterfly per thread and round when R > EPT.
-template <int R, int DIR, int EPT>
-__device__ __noinline__ void fft_pass_prime(float2 *buf, int N, int Ns, const float2 *tw,
-                                            int lgH, int tid, int nt) {
-  constexpr int MAXB = EPT / R > 0 ? EPT / R : 1;
-  constexpr int HR = (R - 1) / 2;
-  const int H = 1 << lgH;
-  const int nbPer = N / R;
-  const int nb = nbPer << lgH;
-  const int twstep = N / (Ns * R);
-  float cs[HR + 1], sn[HR + 1];  // cos, sin(2 pi m / R), m = 1..HR
-#pragma unroll
-  for (int m = 1; m <= HR; ++m) {
-    const float2 w = tw[m * nbPer];
-    cs[m] = w.x;
-    sn[m] = -w.y;
+// Columns of a prime's cosine/sine matrix: whole groups of 8, 12 or 16 pairs.
+constexpr int rt_prime_cols(int p) { return ((p - 1) / 2 + 47) / 48 * 48; }
+
+// Waves a pass of a prime p above kFftRegPrime needs with G output pairs per
+// wave, and the G it runs with.
+constexpr int rt_prime_waves(int nb, int p, int G) {
+  return ((nb + 63) / 64) * (((p - 1) / 2 + G - 1) / G);
+}
+constexpr int rt_prime_pairs(int nb, int p) {
+  return rt_prime_waves(nb, p, 8) <= 16 ? 8 : rt_prime_waves(nb, p, 12) <= 16 ? 12 : 16;
+}
+
+// Pass of a prime radix p > kFftRegPrime.  With P_j = a_j + a_(p-j) and
+// M_j = a_j - a_(p-j) (formed in place first, twiddles included),
+//   b_q, b_(p-q) = a_0 + sum_j cos(2 pi j q/p) P_j -/+ i sum_j sin(2 pi j q/p) M_j.
+// A wave takes 64 butterflies (one per lane) and G of the (p-1)/2 output
+// pairs, so the cosines and sines are the same for the whole wave: scalar
+// loads from the (p-1)/2 x hp matrix `pm` of (cos, sin), and an output pair
+// costs four multiply-adds per j instead of eight with two table reads.
+template <int G, int DIR>
+__device__ __noinline__ void rt_pass_prime(LdsPtr buf, int N_, int Ns_, int p_, TabPtr tw,
+                                           const float *pm_, int lgH_, int tid, int nt_) {
+  const int N = __builtin_amdgcn_readfirstlane(N_), Ns = __builtin_amdgcn_readfirstlane(Ns_);
+  const int p = __builtin_amdgcn_readfirstlane(p_), nt = __builtin_amdgcn_readfirstlane(nt_);
+  const int lgH = __builtin_amdgcn_readfirstlane(lgH_);
+  const uintptr_t pa = (uintptr_t)pm_;
+  const unsigned plo = __builtin_amdgcn_readfirstlane((unsigned)pa);
+  const unsigned phi = __builtin_amdgcn_readfirstlane((unsigned)(pa >> 32));
+  const ScalarPtr pm = (ScalarPtr)(((uintptr_t)phi << 32) | plo);
+  const int h = (p - 1) / 2, hp = rt_prime_cols(p);
+  const int nb = (N / p) << lgH, twstep = N / p / Ns;
+  for (int e = tid; e < nb * h; e += nt) {
+    const int jj = e / nb, g = e - jj * nb;
+    const LdsPtr x = buf + g + (jj + 1) * nb, y = buf + g + (p - 1 - jj) * nb;
+    float2 u = ldf2(x), v = ldf2(y);
+    if (Ns > 1) {
+      const int kt = ((g >> lgH) % Ns) * twstep;
+      float2 wu = ldf2(tw + kt * (jj + 1)), wv = ldf2(tw + kt * (p - 1 - jj));
+      if (DIR > 0) wu.y = -wu.y, wv.y = -wv.y;
+      u = cmul(u, wu);
+      v = cmul(v, wv);
+    }
+    stf2(x, cadd(u, v));
+    stf2(y, csub(u, v));
   }
-  float2 v[MAXB][R];
+  __syncthreads();
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int nblk = (nb + 63) / 64, grp = w / nblk;
+  const int g = (w - grp * nblk) * 64 + lane;
+  const bool live = grp * G < h && g < nb;
+  float2 A[G], B[G], a0 = make_float2(0.f, 0.f), y0 = a0;
 #pragma unroll
-  for (int q = 0; q < MAXB; ++q) {
-    const int g = tid + q * nt;
-    if (g < nb) {
-      const int t = g & (H - 1), j = g >> lgH;
-      const int k = j % Ns;
-      const unsigned base = (unsigned)(k * twstep);
+  for (int u = 0; u < G; ++u) A[u] = B[u] = make_float2(0.f, 0.f);
+  if (live) {
+    a0 = y0 = ldf2(buf + g);
+#pragma unroll 1
+    for (int j = 0; j < h; ++j) {
+      const float2 P = ldf2(buf + g + (j + 1) * nb), M = ldf2(buf + g + (p - 1 - j) * nb);
+      const ScalarPtr m = pm + 2 * (j * hp + grp * G);
+      y0 = cadd(y0, P);
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        float2 x = buf[(lds_pad(j + r * nbPer) << lgH) + t];
-        if (r > 0 && Ns > 1) {
-          float2 w = tw[base * r];
-          if (DIR > 0) w.y = -w.y;
-          x = cmul(x, w);
-        }
-        v[q][r] = x;
+      for (int u = 0; u < G; ++u) {
+        const float c = m[2 * u], s = m[2 * u + 1];
+        A[u].x = fmaf(c, P.x, A[u].x);
+        A[u].y = fmaf(c, P.y, A[u].y);
+        B[u].x = fmaf(s, M.x, B[u].x);
+        B[u].y = fmaf(s, M.y, B[u].y);
       }
-      float2 P[HR + 1], M[HR + 1];
-      float2 b0 = v[q][0];
-#pragma unroll
-      for (int jj = 1; jj <= HR; ++jj) {
-        P[jj] = make_float2(v[q][jj].x + v[q][R - jj].x, v[q][jj].y + v[q][R - jj].y);
-        M[jj] = make_float2(v[q][jj].x - v[q][R - jj].x, v[q][jj].y - v[q][R - jj].y);
-        b0.x += P[jj].x;
-        b0.y += P[jj].y;
-      }
-#pragma unroll
-      for (int qq = 1; qq <= HR; ++qq) {
-        float2 re = v[q][0], im = make_float2(0.f, 0.f);
-#pragma unroll
-        for (int jj = 1; jj <= HR; ++jj) {
-          const int m = (jj * qq) % R;  // compile-time after unrolling
-          const float c = m <= HR ? cs[m] : cs[R - m];
-          const float sv = m <= HR ? sn[m] : -sn[R - m];
-          re.x += c * P[jj].x;
-          re.y += c * P[jj].y;
-          im.x += sv * M[jj].x;
-          im.y += sv * M[jj].y;
-        }
-        const float2 mi = mul_i<DIR>(im);
-        v[q][qq] = make_float2(re.x + mi.x, re.y + mi.y);
-        v[q][R - qq] = make_float2(re.x - mi.x, re.y - mi.y);
-      }
-      v[q][0] = b0;
     }
   }
   __syncthreads();
+  if (live) {
+    const int j = g >> lgH, jq = j / Ns, k = j - jq * Ns;
+    LdsPtr o = buf + (((jq * Ns * p + k) << lgH) + (g - (j << lgH)));
+    const int W = Ns << lgH;
+    if (grp == 0) stf2(o, y0);
 #pragma unroll
-  for (int q = 0; q < MAXB; ++q) {
-    const int g = tid + q * nt;
-    if (g < nb) {
-      const int t = g & (H - 1), j = g >> lgH;
-      const int jq = j / Ns, k = j - jq * Ns;
-      const int o = jq * Ns * R + k;
-#pragma unroll
-      for (int r = 0; r < R; ++r) buf[(lds_pad(o + r * Ns) << lgH) + t] = v[q][r];
+    for (int u = 0; u < G; ++u) {
+      const int q = grp * G + u + 1;
+      if (q > h) break;
+      const float2 re = cadd(a0, A[u]), mi = mul_i<DIR>(B[u]);
+      stf2(o + q * W, cadd(re, mi));
+      stf2(o + (p - q) * W, csub(re, mi));
     }
   }
   __syncthreads();
 }
 
-// Pass with a prime radix 19 <= R <= kFftMaxPrime: each output y[o],
-// o = jq Ns R + q Ns + k, j = jq Ns + k, is the direct sum
-//   y[o] = sum_r x[j + r N/R] W_N^(r e mod N),  e = k N/(Ns R) + q N/R,
-// (the twiddle W_N^(r k N/(Ns R)) and the DFT_R factor W_R^(r q) in one table
-// entry), at most EPT outputs per thread held in registers across the barrier.
-template <int DIR, int EPT>
-__device__ __noinline__ void fft_pass_gen(float2 *buf, int N, int Ns, int R, const float2 *tw,
-                                          int lgH, int tid, int nt) {
-  const int H = 1 << lgH;
-  const int nbPer = N / R;
-  const int total = N << lgH;
-  const int twstep = N / (Ns * R);
-  float2 acc[EPT];
-#pragma unroll
-  for (int q = 0; q < EPT; ++q) {
-    const int g = tid + q * nt;
-    if (g < total) {
-      const int t = g & (H - 1), o = g >> lgH;
-      const int k = o % Ns, rest = o / Ns;
-      const int qq = rest % R, jq = rest / R;
-      const int j = jq * Ns + k;
-      const int e = k * twstep + qq * nbPer;  // < N
-      float2 s = make_float2(0.f, 0.f);
-      int m = 0;
-      for (int r = 0; r < R; ++r) {
-        const float2 x = buf[(lds_pad(j + r * nbPer) << lgH) + t];
-        float2 w = tw[m];
-        if (DIR > 0) w.y = -w.y;
-        s.x += x.x * w.x - x.y * w.y;
-        s.y += x.x * w.y + x.y * w.x;
-        m += e;
-        if (m >= N) m -= N;
-      }
-      acc[q] = s;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < EPT; ++q) {
-    const int g = tid + q * nt;
-    if (g < total) buf[(lds_pad(g >> lgH) << lgH) + (g & (H - 1))] = acc[q];
-  }
-  __syncthreads();
-}
-
-// fft_pass behind a call: the run-time-plan transform calls one per pass, so
-// the register demand of the largest radix does not add to the caller's.
-template <int R, int DIR, int EPT>
-__device__ __noinline__ void fft_pass_call(float2 *buf, int N, int Ns, const float2 *tw, int lgH,
-                                           int tid, int nt) {
-  fft_pass<R, DIR, EPT>(buf, N, Ns, tw, lgH, tid, nt);
-}
-
-// In-place transform of 2^lgH interleaved sequences of length d.N held in LDS:
-// element i of sequence t lives at buf[lds_pad(i) * 2^lgH + t].  Requires
-// 2^lgH * N <= 15 * nt (16 * nt without radix-3 passes); see fft_threads().
+// In-place transform of 2^lgH interleaved sequences of length d.N held in LDS
+// at buf[(i << lgH) + t], with a run-time plan and fft_rt_threads() threads.
 // The caller must __syncthreads() after filling buf; the function ends with a
-// barrier.
-// LV (fft_level of the sizes a kernel serves): 0 = radices 2, 3, 4, 8, 16;
-// 1 = also the butterflies of 5, 7, 11, 13, 17; 2 = also the direct-sum
-// primes 19..127.  Each level is compiled only into the kernels instantiated
-// for such sizes: the extra passes raise the register demand of every
-// instantiation.
-template <int DIR, int EPT = kFftEPT, int LV = 0>
-__device__ void lds_fft(float2 *buf, const FftDesc &d, int lgH, int tid, int nt) {
-  int Ns = 1;
+// barrier.  WIDE: also the prime passes of 16 pairs a wave, which a few
+// lengths above 13000 need (their registers would cost every other length a
+// fifth of the waves: row pass at n = 2448 378 us against 478).
+template <int DIR, bool WIDE = false>
+__device__ void lds_fft(float2 *buf_, const FftDesc &d, int lgH, int tid, int nt) {
+  const LdsPtr buf = (LdsPtr)buf_;
+  const TabPtr tw = (TabPtr)d.tw;
+  const int N = d.N;
+  int Ns = 1, np = 0;
   for (int s = 0; s < d.nr; ++s) {
     const int R = d.r[s];
-    if (R == 16) {
-      if constexpr (EPT >= 16) fft_pass_call<16, DIR, EPT>(buf, d.N, Ns, d.tw, lgH, tid, nt);
-    } else if (R == 8) {
-      fft_pass_call<8, DIR, EPT>(buf, d.N, Ns, d.tw, lgH, tid, nt);
-    }
-    else if (R == 4)
-      fft_pass_call<4, DIR, EPT>(buf, d.N, Ns, d.tw, lgH, tid, nt);
-    else if (R == 2)
-      fft_pass_call<2, DIR, EPT>(buf, d.N, Ns, d.tw, lgH, tid, nt);
-    else if (R == 3)
-      fft_pass_call<3, DIR, EPT>(buf, d.N, Ns, d.tw, lgH, tid, nt);
-    else if constexpr (LV >= 1) {
-      if (R == 5)
-        fft_pass_call<5, DIR, EPT>(buf, d.N, Ns, d.tw, lgH, tid, nt);
-      else if (R == 7)
-        fft_pass_call<7, DIR, EPT>(buf, d.N, Ns, d.tw, lgH, tid, nt);
-      else if (R == 11)
-        fft_pass_prime<11, DIR, EPT>(buf, d.N, Ns, d.tw, lgH, tid, nt);
-      else if (R == 13)
-        fft_pass_prime<13, DIR, EPT>(buf, d.N, Ns, d.tw, lgH, tid, nt);
-      else if (R == 17)
-        fft_pass_prime<17, DIR, EPT>(buf, d.N, Ns, d.tw, lgH, tid, nt);
-      else if constexpr (LV >= 2)
-        fft_pass_gen<DIR, EPT>(buf, d.N, Ns, R, d.tw, lgH, tid, nt);
+    switch (R) {
+#define TOMO_RT_PASS(r) \
+  case r: rt_pass<r, DIR>(buf, N, Ns, tw, lgH, tid, nt); break;
+      TOMO_RT_PASS(2) TOMO_RT_PASS(3) TOMO_RT_PASS(4) TOMO_RT_PASS(5) TOMO_RT_PASS(6)
+      TOMO_RT_PASS(7) TOMO_RT_PASS(8) TOMO_RT_PASS(9) TOMO_RT_PASS(10) TOMO_RT_PASS(11)
+      TOMO_RT_PASS(12) TOMO_RT_PASS(13) TOMO_RT_PASS(14) TOMO_RT_PASS(15) TOMO_RT_PASS(16)
+      TOMO_RT_PASS(17) TOMO_RT_PASS(18) TOMO_RT_PASS(20)
+#undef TOMO_RT_PASS
+      default:
+      {
+        const int G = rt_prime_pairs((N / R) << lgH, R);
+        if (WIDE && G == 16)
+          rt_pass_prime<16, DIR>(buf, N, Ns, R, tw, d.pm[np], lgH, tid, nt);
+        else if (G == 12)
+          rt_pass_prime<12, DIR>(buf, N, Ns, R, tw, d.pm[np], lgH, tid, nt);
+        else
+          rt_pass_prime<8, DIR>(buf, N, Ns, R, tw, d.pm[np], lgH, tid, nt);
+      }
+        ++np;
     }
     Ns *= R;
   }
+}
+
+// Threads of a workgroup transforming 2^lgH interleaved sequences with a
+// run-time plan: as few as hold the passes' butterflies (more resident
+// workgroups; N = 2000, row pass, us: 52 with 128 threads, 68 with 256), but
+// for lengths up to 1024, whose launches are short, one butterfly per thread;
+// -1 if more than 1024 would be needed.
+inline int fft_rt_threads(const FftDesc &d, int lgH) {
+  int64_t t = 64, one = 64;
+  for (int i = 0; i < d.nr; ++i) {
+    const int R = d.r[i];
+    const int64_t nb = (int64_t)(d.N / R) << lgH;
+    if (R > kFftRtVals || R == 19)
+      t = std::max<int64_t>(t, 64 * rt_prime_waves((int)nb, R, rt_prime_pairs((int)nb, R)));
+    else
+      t = std::max<int64_t>(t, (nb + rt_maxb(R) - 1) / rt_maxb(R));
+    if (R <= kFftRtVals && R != 19) one = std::max(one, nb);
+  }
+  if (d.N <= 1024 && one <= 512) t = std::max(t, one);
+  t = (t + 63) / 64 * 64;
+  return t > 1024 ? -1 : (int)t;
+}
+
+// True if the plan has a prime pass of 16 pairs a wave (lds_fft's WIDE).
+inline bool fft_rt_wide(const FftDesc &d, int lgH) {
+  bool wide = false;
+  for (int i = 0; i < d.nr; ++i) {
+    const int R = d.r[i];
+    wide |= (R > kFftRtVals || R == 19) && rt_prime_pairs((d.N / R) << lgH, R) == 16;
+  }
+  return wide;
 }
 
 // ---- transforms of a compile-time size ---------------------------------------
@@ -546,8 +724,11 @@ __device__ __forceinline__ void fft_pass_c(float2 *buf, const float2 *__restrict
   __syncthreads();
 }
 
-// lds_fft for a compile-time size N (StaticPlan); `tw` is the twiddle table
-// of size N.  Same layout, requirements and barriers as lds_fft.
+// In-place transform of 2^LGH interleaved sequences of a compile-time length N
+// (StaticPlan) held in LDS, element i of sequence t at
+// buf[lds_pad(i) * 2^LGH + t]; `tw` is the twiddle table of size N.  Needs
+// fft_threads() threads; the caller must __syncthreads() after filling buf,
+// and the function ends with a barrier.
 // Passes S .. SEnd-1 only (Ns: the sub-transform length entering pass S).
 template <int N, int DIR, int EPT, int LGH, int S = 0, int Ns = 1,
           int SEnd = StaticPlan<N>::passes>
@@ -660,6 +841,7 @@ __device__ __forceinline__ void fft_c_global(float2 *buf, const float2 *__restri
 template <typename F>
 inline void with_static_size(int N, F &&f) {
   switch (N) {
+    case 256: f(std::integral_constant<int, 256>()); break;
     case 512: f(std::integral_constant<int, 512>()); break;
     case 768: f(std::integral_constant<int, 768>()); break;
     case 1280: f(std::integral_constant<int, 1280>()); break;
@@ -675,8 +857,6 @@ inline void with_static_size(int N, F &&f) {
     case 2048: f(std::integral_constant<int, 2048>()); break;
     case 4096: f(std::integral_constant<int, 4096>()); break;
     case 8192: f(std::integral_constant<int, 8192>()); break;
-    case -1: f(std::integral_constant<int, -1>()); break;  // run-time sizes, fft_level 1
-    case -2: f(std::integral_constant<int, -2>()); break;  // run-time sizes, fft_level 2
     default: f(std::integral_constant<int, 0>()); break;
   }
 }
@@ -719,16 +899,14 @@ __device__ __forceinline__ void stage_lds(int count, int tid, int nt, Ld ld, St 
 }
 
 // Workgroup size for transforming `elems` complex values (all interleaved
-// sequences) with plan d: 16 values per thread for radices 2/4/8/16, fewer
-// with a radix-3, 5, 7, 11 or 13 pass (15, 15, 14, 11, 13: whole butterflies;
-// the other prime passes take any count); at least 256 and a multiple of 64.  Returns -1
-// if more than 1024 threads would be needed.
-inline int fft_threads(const FftDesc &d, int64_t elems, int ept = kFftEPT) {
+// sequences) of a compiled size, and the size by which a width is accepted:
+// 16 values per thread for radices 2/4/8/16, fewer with a radix-3, 5, 7, 11 or
+// 13 pass (15, 15, 14, 11, 13: whole butterflies); at least 256 and a multiple
+// of 64.  Returns -1 if more than 1024 threads would be needed.
+inline int fft_threads(const FftRule &d, int64_t elems, int ept = kFftEPT) {
   int64_t per = ept;  // values a thread covers in every pass: whole butterflies
   for (int i = 0; i < d.nr; ++i) {
     const int R = d.r[i];
-    // whole butterflies; a register-butterfly prime pass above ept runs one
-    // per thread (nt >= N/16 > N/R butterflies), the direct-sum pass any count
     if (R <= 8 || R == 16 || (R <= 17 && R <= ept)) per = std::min<int64_t>(per, (ept / R) * R);
   }
   int64_t t = (elems + per - 1) / per;
@@ -737,35 +915,13 @@ inline int fft_threads(const FftDesc &d, int64_t elems, int ept = kFftEPT) {
   return (int)(t < 256 ? 256 : t);
 }
 
-// Transform level of a length N (the LV of lds_fft): 0 if N = 2^a 3^b, 1 if
-// its other prime factors are at most 17, 2 otherwise.
-inline int fft_level(int64_t N) {
-  if (N < 1) return 0;
+// True if N has a prime factor other than 2 and 3.
+inline bool fft_general(int64_t N) {
+  if (N < 1) return false;
   while (N % 2 == 0) N /= 2;
   while (N % 3 == 0) N /= 3;
-  if (N == 1) return 0;
-  for (int64_t p : {5, 7, 11, 13, 17})
-    while (N % p == 0) N /= p;
-  return N == 1 ? 1 : 2;
+  return N != 1;
 }
-
-// True if N has a prime factor other than 2 and 3 (its plans need level 1 or
-// 2 transforms).
-inline bool fft_general(int64_t N) { return fft_level(N) > 0; }
-
-// f(std::integral_constant<int, L>()) for the transform level L in 0..2.
-template <typename F>
-inline void with_fft_level(int L, F &&f) {
-  if (L == 2)
-    f(std::integral_constant<int, 2>());
-  else if (L == 1)
-    f(std::integral_constant<int, 1>());
-  else
-    f(std::integral_constant<int, 0>());
-}
-
-// lds_fft level of the run-time-size kernels NS = -1 and NS = -2.
-constexpr int fft_lv(int NS) { return NS == -2 ? 2 : (NS == -1 ? 1 : 0); }
 
 // True if N >= 1 and every prime factor of N is at most kFftMaxPrime.
 inline bool fft_size_ok(int64_t N) {

@@ -42,7 +42,7 @@ __global__ void k_flt_weights(const float *__restrict__ wfilter, const float *__
 
 // mode 0: rows of width ne already padded (cfunc_filter::filter);
 // mode 1: rows of width n, edge-replicate padded on load and cropped on store
-template <int MODE, typename T, int LV = 0>
+template <int MODE, typename T, bool WIDE>
 __global__ __launch_bounds__(1024) void k_flt_rows(T *__restrict__ g, const float2 *__restrict__ w,
                                                    FftDesc fd, int ne, int n, int nproj) {
   extern __shared__ float2 sm[];
@@ -60,9 +60,9 @@ __global__ __launch_bounds__(1024) void k_flt_rows(T *__restrict__ g, const floa
         const int src = MODE == 1 ? min(max(j - pad, 0), n - 1) : j;
         return cpx<T>{r0[src], has1 ? r1[src] : T(0)};
       },
-      [&](int j, cpx<T> v) { sm[lds_pad(j)] = tof2(v); });
+      [&](int j, cpx<T> v) { sm[j] = tof2(v); });
   __syncthreads();
-  lds_fft<-1, kFftEPT, LV>(sm, fd, 0, tid, nt);
+  lds_fft<-1, WIDE>(sm, fd, 0, tid, nt);
   const float2 *wz = w + (size_t)z * (ne / 2 + 1);
   const int nh = ne / 2;
   for (int k = tid; k < ne; k += nt) {
@@ -74,19 +74,19 @@ __global__ __launch_bounds__(1024) void k_flt_rows(T *__restrict__ g, const floa
     } else {
       W = cconj(wz[ne - k]);
     }
-    sm[lds_pad(k)] = cmul(sm[lds_pad(k)], W);
+    sm[k] = cmul(sm[k], W);
   }
   __syncthreads();
-  lds_fft<1, kFftEPT, LV>(sm, fd, 0, tid, nt);
+  lds_fft<1, WIDE>(sm, fd, 0, tid, nt);
   if (MODE == 0) {
     for (int j = tid; j < ne; j += nt) {
-      const float2 y = sm[lds_pad(j)];
+      const float2 y = sm[j];
       str(r0 + j, y.x);
       if (has1) str(r1 + j, y.y);
     }
   } else {
     for (int j = tid; j < n; j += nt) {
-      const float2 y = sm[lds_pad(pad + j)];
+      const float2 y = sm[pad + j];
       str(r0 + j, y.x);
       if (has1) str(r1 + j, y.y);
     }
@@ -455,7 +455,7 @@ extern "C" int flt_create(tomo_flt_plan **plan, int64_t n, int64_t ne, int64_t n
                "flt_create: unknown dtype %d", dtype);
   {
     // workgroup of the ne-point row kernels, from the radix sequence alone
-    FftDesc d{};
+    FftRule d{};
     const int rc0 = FftPlan::radices((int)ne, d);
     if (rc0) return rc0;
     TOMO_REQUIRE(fft_threads(d, ne) > 0,
@@ -493,23 +493,20 @@ extern "C" int flt_create(tomo_flt_plan **plan, int64_t n, int64_t ne, int64_t n
       return rc;
     }
   }
-  P->threads = fft_threads(P->fft.d, ne);
-  P->lds = sizeof(float2) * lds_padded_len((int)ne);
+  P->threads = fft_rt_threads(P->fft.d, 0);
+  P->lds = sizeof(float2) * (size_t)ne;
   if (P->threads <= 0 || P->lds > max_lds_per_block()) {
     set_error("flt_create: ne=%lld too large for one workgroup", (long long)ne);
     flt_destroy(P);
     return TOMO_EINVAL;
   }
   const void *rows_kernels[] = {
-      (const void *)k_flt_rows<0, float>, (const void *)k_flt_rows<1, float>,
-      (const void *)k_flt_rows<0, _Float16>, (const void *)k_flt_rows<1, _Float16>,
-      (const void *)k_flt_rows<0, __bf16>, (const void *)k_flt_rows<1, __bf16>,
-      (const void *)k_flt_rows<0, float, 1>, (const void *)k_flt_rows<1, float, 1>,
-      (const void *)k_flt_rows<0, _Float16, 1>, (const void *)k_flt_rows<1, _Float16, 1>,
-      (const void *)k_flt_rows<0, __bf16, 1>, (const void *)k_flt_rows<1, __bf16, 1>,
-      (const void *)k_flt_rows<0, float, 2>, (const void *)k_flt_rows<1, float, 2>,
-      (const void *)k_flt_rows<0, _Float16, 2>, (const void *)k_flt_rows<1, _Float16, 2>,
-      (const void *)k_flt_rows<0, __bf16, 2>, (const void *)k_flt_rows<1, __bf16, 2>};
+      (const void *)k_flt_rows<0, float, false>, (const void *)k_flt_rows<1, float, false>,
+      (const void *)k_flt_rows<0, _Float16, false>, (const void *)k_flt_rows<1, _Float16, false>,
+      (const void *)k_flt_rows<0, __bf16, false>, (const void *)k_flt_rows<1, __bf16, false>,
+      (const void *)k_flt_rows<0, float, true>, (const void *)k_flt_rows<1, float, true>,
+      (const void *)k_flt_rows<0, _Float16, true>, (const void *)k_flt_rows<1, _Float16, true>,
+      (const void *)k_flt_rows<0, __bf16, true>, (const void *)k_flt_rows<1, __bf16, true>};
   hipError_t e = hipSuccess;
   for (const void *k : rows_kernels)
     if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->lds);
@@ -525,15 +522,11 @@ extern "C" int flt_create(tomo_flt_plan **plan, int64_t n, int64_t ne, int64_t n
 template <int MODE, typename T>
 static void launch_rows(tomo_flt_plan *P, void *g, const float2 *w, hipStream_t st) {
   const dim3 grid((unsigned)ceil_div(P->nproj, 2), (unsigned)P->nz);
-  const int lv = fft_level(P->ne);  // transforms with the level-1 or level-2 passes
-  if (lv == 2)
-    hipLaunchKernelGGL((k_flt_rows<MODE, T, 2>), grid, dim3(P->threads), P->lds, st, (T *)g, w,
-                       P->fft.d, (int)P->ne, (int)P->n, (int)P->nproj);
-  else if (lv == 1)
-    hipLaunchKernelGGL((k_flt_rows<MODE, T, 1>), grid, dim3(P->threads), P->lds, st, (T *)g, w,
+  if (fft_rt_wide(P->fft.d, 0))
+    hipLaunchKernelGGL((k_flt_rows<MODE, T, true>), grid, dim3(P->threads), P->lds, st, (T *)g, w,
                        P->fft.d, (int)P->ne, (int)P->n, (int)P->nproj);
   else
-    hipLaunchKernelGGL((k_flt_rows<MODE, T>), grid, dim3(P->threads), P->lds, st, (T *)g, w,
+    hipLaunchKernelGGL((k_flt_rows<MODE, T, false>), grid, dim3(P->threads), P->lds, st, (T *)g, w,
                        P->fft.d, (int)P->ne, (int)P->n, (int)P->nproj);
 }
 
@@ -578,8 +571,8 @@ extern "C" int flt_filter_center(tomo_flt_plan *P, void *data, const float *wfil
 
 extern "C" void flt_destroy(tomo_flt_plan *P) {
   if (!P) return;
-  P->fft.tw.release();
-  P->fft2n.tw.release();
+  P->fft.release();
+  P->fft2n.release();
   P->w.release();
   P->H2.release();
   P->HL.release();

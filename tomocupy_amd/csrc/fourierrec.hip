@@ -47,7 +47,7 @@ constexpr int kSeLen = kGridBatch + kGridBatch / 8;
 constexpr int kSgLen = kGridBatch + kGridBatch / 4;
 __device__ __forceinline__ int se_at(int e) { return e + (e >> 3); }
 __device__ __forceinline__ int sg_at(int e) { return e + 2 * (e >> 3); }
-constexpr int kColEPT = 32;     // FFT values per thread in the column pass
+constexpr int kColEPT = 32;     // column-pass values per thread in the width rule (fr_fft_shapes_ok)
 // log2 of the columns a column-pass workgroup transforms for 2n = N: as many
 // as fit 512 threads at kColEPT values each (and the LDS), at most 16
 constexpr int col_lg(int N) { return ilog2c(16384 / N) > 4 ? 4 : ilog2c(16384 / N); }
@@ -55,9 +55,8 @@ constexpr int col_lg(int N) { return ilog2c(16384 / N) > 4 ? 4 : ilog2c(16384 / 
 // Sign 1 - 2*((t+1) % 2): -1 for even t, +1 for odd t (kernels_fourierrec.cuh:121-132).
 __device__ __forceinline__ float shift_sign(int t) { return (t & 1) ? 1.f : -1.f; }
 
-// NS: n as a compile-time constant (0 = sizes known at run time only, -1 and
-// -2 the same for sizes of fft_level 1 and 2), as in
-// every FFT kernel of this file.
+// NS of the FFT kernels: the transform length as a compile-time constant, 0 =
+// known at run time only.
 // max over the workgroup of the threads' m; thread 0 gets the result
 // (LDS for the per-wave maxima; every thread must call it)
 __device__ __forceinline__ float block_max(float m) {
@@ -92,12 +91,13 @@ __device__ __forceinline__ float2 block_sum2(float2 v) {
 // Writes the shifted spectrum row out[k] = sm[k] * (-1)^k * scale and, for
 // float32 plans with a gmax buffer, the row's largest |re|, |im| to gmax[row]
 // (the gridding scales its split half-precision factors with the maximum).
+// (run-time sizes)
 template <typename T>
 __device__ __forceinline__ void store_spectrum(cpx<T> *out, const float2 *sm, int n, float scale,
                                                int tid, int nt, float *gmax, size_t row) {
   float m = 0.f;
   for (int k = tid; k < n; k += nt) {
-    const float2 v = cscale(sm[lds_pad(k)], shift_sign(k) * scale);
+    const float2 v = cscale(sm[k], shift_sign(k) * scale);
     m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)));
     stc(out + k, v);
   }
@@ -122,7 +122,7 @@ __device__ __forceinline__ void store_max(float m, float *gmax, size_t row) {
 }
 
 template <typename T, int NS>
-__global__ __launch_bounds__(512) void k_fr_prep(const T *__restrict__ data, cpx<T> *__restrict__ G,
+__global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_prep(const T *__restrict__ data, cpx<T> *__restrict__ G,
                                                  FftDesc fd, int n, int nproj, int nz, int nzc,
                                                  float scale, float *__restrict__ gmax) {
   extern __shared__ float2 sm[];
@@ -150,9 +150,9 @@ __global__ __launch_bounds__(512) void k_fr_prep(const T *__restrict__ data, cpx
   } else {
     stage_lds<8, cpx<T>>(
         n, tid, nt, [&](int j) { return cpx<T>{r1[j], has2 ? r2[j] : T(0)}; },
-        [&](int j, cpx<T> v) { sm[lds_pad(j)] = cscale(tof2(v), shift_sign(j)); });
+        [&](int j, cpx<T> v) { sm[j] = cscale(tof2(v), shift_sign(j)); });
     __syncthreads();
-    lds_fft<-1, kFftEPT, fft_lv(NS)>(sm, fd, 0, tid, nt);
+    lds_fft<-1>(sm, fd, 0, tid, nt);
     store_spectrum(out, sm, n, scale, tid, nt, gmax, (size_t)c * nproj + p);
   }
 }
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(512) void k_fr_prep(const T *__restrict__ data, cpx
 // (H1-H2)/2, exact for real rows), IFFT_2n, add the edge-replication terms
 // x[0] HL + x[n-1] HR per slice, then the shifted n-point DFT of k_fr_prep.
 template <typename T, int NS>
-__global__ __launch_bounds__(512) void k_fr_filtprep(
+__global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_filtprep(
     const T *__restrict__ data, cpx<T> *__restrict__ G, const float2 *__restrict__ H2,
     const float *__restrict__ HL, const float *__restrict__ HR, FftDesc fd2, FftDesc fd1, int n,
     int nproj, int nz, int nzc, float scale, float *__restrict__ gmax) {
@@ -219,13 +219,13 @@ __global__ __launch_bounds__(512) void k_fr_filtprep(
       fft_c_from_global<2 * NS, -1, kFftEPT, 0>(sm, fd2.tw, tid, nt,
                                                 [&](int j, int) { return zat(j); });
   } else {
-    auto st = [&](int j, float2 v) { sm[lds_pad(j)] = v; };
+    auto st = [&](int j, float2 v) { sm[j] = v; };
     if (diff)
       stage_lds<8, float2>(n2, tid, nt, [&](int j) { return zdiff(j); }, st);
     else
       stage_lds<8, float2>(n2, tid, nt, [&](int j) { return zat(j); }, st);
     __syncthreads();
-    lds_fft<-1, kFftEPT, fft_lv(NS)>(sm, fd2, 0, tid, nt);
+    lds_fft<-1>(sm, fd2, 0, tid, nt);
   }
   float2 z0 = make_float2(0.f, 0.f);  // Z[0] (thread 0), for the differenced form
   if (diff) z0 = block_sum2(zsum);
@@ -233,29 +233,29 @@ __global__ __launch_bounds__(512) void k_fr_filtprep(
   const float2 *Hb = diff ? H2b + (size_t)nz * n2 : H2b;
   for (int k = tid; k <= n; k += nt) {
     const int km = (n2 - k) % n2;
-    float2 zk = sm[lds_pad(k)], zm = sm[lds_pad(km)];
+    float2 zk = sm[lidx<NS>(k)], zm = sm[lidx<NS>(km)];
     if (diff && k == 0) zk = zm = z0;
     const float2 ak = Ha[k], bk = Hb[k], am = Ha[km], bm = Hb[km];
     const float2 sk = cscale(cadd(ak, bk), 0.5f), dk = cscale(csub(ak, bk), 0.5f);
     const float2 sm_ = cscale(cadd(am, bm), 0.5f), dm = cscale(csub(am, bm), 0.5f);
     const float2 yk = cadd(cmul(zk, sk), cmul(cconj(zm), dk));
     const float2 ym = cadd(cmul(zm, sm_), cmul(cconj(zk), dm));
-    sm[lds_pad(k)] = yk;
-    if (km != k) sm[lds_pad(km)] = ym;
+    sm[lidx<NS>(k)] = yk;
+    if (km != k) sm[lidx<NS>(km)] = ym;
   }
   __syncthreads();
   if constexpr (NS > 0)
     lds_fft_c<2 * NS, 1, kFftEPT, 0>(sm, fd2.tw, tid, nt);
   else
-    lds_fft<1, kFftEPT, fft_lv(NS)>(sm, fd2, 0, tid, nt);
+    lds_fft<1>(sm, fd2, 0, tid, nt);
   const float *hl1 = HL + (size_t)c * n, *hr1 = HR + (size_t)c * n;
   const float *hl2 = HL + (size_t)zb * n, *hr2 = HR + (size_t)zb * n;
   const float e0 = edge[0], e1 = edge[1], e2 = edge[2], e3 = edge[3];
   for (int j = tid; j < n; j += nt) {
-    float2 y = sm[lds_pad(j)];
+    float2 y = sm[lidx<NS>(j)];
     y.x += e0 * hl1[j] + e1 * hr1[j];
     y.y += e2 * hl2[j] + e3 * hr2[j];
-    sm[lds_pad(j)] = cscale(y, shift_sign(j));
+    sm[lidx<NS>(j)] = cscale(y, shift_sign(j));
   }
   __syncthreads();
   if constexpr (NS > 0) {
@@ -271,7 +271,7 @@ __global__ __launch_bounds__(512) void k_fr_filtprep(
     });
     store_max<T>(m, gmax, (size_t)c * nproj + p);
   } else {
-    lds_fft<-1, kFftEPT, fft_lv(NS)>(sm, fd1, 0, tid, nt);
+    lds_fft<-1>(sm, fd1, 0, tid, nt);
     store_spectrum(out, sm, n, scale, tid, nt, gmax, (size_t)c * nproj + p);
   }
 }
@@ -751,7 +751,7 @@ template <typename T, int NS>
 // the column pass reads each of its blocks contiguously; the workgroups of
 // neighbouring rows then share an XCD, whose L2 merges their partial-line
 // writes.  lgB = 0: R[c][a][v'].
-__global__ __launch_bounds__(512) void k_fr_rowfft(const cpx<T> *__restrict__ F,
+__global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_rowfft(const cpx<T> *__restrict__ F,
                                                    cpx<T> *__restrict__ R, FftDesc fd, int n,
                                                    int nzc, int lgB,
                                                    const int2 *__restrict__ span) {
@@ -793,36 +793,36 @@ __global__ __launch_bounds__(512) void k_fr_rowfft(const cpx<T> *__restrict__ F,
         [&](int b) { return (b >= sp.x && b < sp.y) ? src[b] : cpx<T>{T(0), T(0)}; },
         [&](int b, cpx<T> v) {
           const float2 x = tof2(v);
-          sm[lds_pad(b)] = (b & 1) ? make_float2(-x.x, -x.y) : x;
+          sm[lidx<NS>(b)] = (b & 1) ? make_float2(-x.x, -x.y) : x;
         });
     __syncthreads();
     if constexpr (NS > 0)
       lds_fft_c<NS, 1, kFftEPT, 0>(sm, fd.tw, tid, nt);
     else
-      lds_fft<1, kFftEPT, fft_lv(NS)>(sm, fd, 0, tid, nt);
+      lds_fft<1>(sm, fd, 0, tid, nt);
     if (lgB > 0) {
       const int B = 1 << lgB;
       cpx<T> *dst = R + (size_t)c * n2 * n + (size_t)a * B;
       for (int v = tid; v < n; v += nt) {
-        const float2 x = sm[lds_pad(v + h)];
+        const float2 x = sm[lidx<NS>(v + h)];
         stc(dst + (size_t)(v >> lgB) * n2 * B + (v & (B - 1)),
             ((v + h) & 1) ? make_float2(-x.x, -x.y) : x);
       }
     } else {
       cpx<T> *dst = R + ((size_t)c * n2 + a) * n;
       for (int v = tid; v < n; v += nt) {
-        const float2 x = sm[lds_pad(v + h)];
+        const float2 x = sm[lidx<NS>(v + h)];
         stc(dst + v, ((v + h) & 1) ? make_float2(-x.x, -x.y) : x);
       }
     }
   }
 }
 
-// The size-specialised column pass runs 16 values per thread (1024 threads):
-// its LDS (4 columns of 2n) admits one workgroup per CU, so the extra waves
-// are the only latency cover.
+// The compiled column pass runs 16 values per thread (1024 threads): its LDS
+// (4 columns of 2n) admits one workgroup per CU, so the extra waves are the
+// only latency cover.
 template <typename T, int NS>
-__global__ __launch_bounds__(NS > 0 ? 1024 : 512) void k_fr_colfft(const cpx<T> *__restrict__ R, T *__restrict__ obj,
+__global__ __launch_bounds__(1024) void k_fr_colfft(const cpx<T> *__restrict__ R, T *__restrict__ obj,
                             const float *__restrict__ phix, const float *__restrict__ phiy,
                             const int2 *__restrict__ circ, FftDesc fd, int n, int nz, int nzc,
                             int lgCB, int blocked) {
@@ -873,19 +873,19 @@ __global__ __launch_bounds__(NS > 0 ? 1024 : 512) void k_fr_colfft(const cpx<T> 
         [&](int idx, cpx<T> v) {
           const int a = idx >> lgCB, t = idx & (CB - 1);
           const float2 x = tof2(v);
-          sm[(lds_pad(a) << lgCB) + t] = (a & 1) ? make_float2(-x.x, -x.y) : x;
+          sm[(lidx<NS>(a) << lgCB) + t] = (a & 1) ? make_float2(-x.x, -x.y) : x;
         });
     __syncthreads();
     if constexpr (NS > 0)
       lds_fft_c<NS, 1, kFftEPT, col_lg(NS)>(sm, fd.tw, tid, nt);
     else
-      lds_fft<1, (NS < 0 ? kFftEPT : kColEPT), fft_lv(NS)>(sm, fd, lgCB, tid, nt);
+      lds_fft<1>(sm, fd, lgCB, tid, nt);
     for (int idx = tid; idx < CB * n; idx += nt) {
       const int ty = idx >> lgCB, t = idx & (CB - 1);
       const int tx = v0 + t;
       if (tx >= n) continue;
       const int u = ty + 1 + h;
-      float2 x = sm[(lds_pad(u) << lgCB) + t];
+      float2 x = sm[(lidx<NS>(u) << lgCB) + t];
       const int2 ci = circ[ty];
       const float ph = (tx >= ci.x && tx < ci.y) ? phix[tx] * phiy[ty] * ((u & 1) ? -1.f : 1.f) : 0.f;
       str(obj + ((size_t)c * n + ty) * n + tx, x.x * ph);
@@ -896,11 +896,9 @@ __global__ __launch_bounds__(NS > 0 ? 1024 : 512) void k_fr_colfft(const cpx<T> 
 
 // ---- adjoint (forward projection) kernels --------------------------------
 
-// NS as k_fr_colfft: a compiled 2n = 2^k or 3 * 2^k (up to 1024 threads,
-// col_lg(NS) columns per workgroup) or 0 / -1 / -2 for the run-time plans of
-// fft_level 0 / 1 / 2.
+// NS as k_fr_colfft (compiled: col_lg(NS) columns per workgroup).
 template <int NS>
-__global__ __launch_bounds__(NS > 0 ? 1024 : 512) void k_fr_colfft_adj(const float *__restrict__ obj, float2 *__restrict__ R,
+__global__ __launch_bounds__(1024) void k_fr_colfft_adj(const float *__restrict__ obj, float2 *__restrict__ R,
                                 const float *__restrict__ phix, const float *__restrict__ phiy,
                                 const int2 *__restrict__ circ, FftDesc fd, int n, int nz,
                                 int nzc, int lgCB) {
@@ -934,7 +932,7 @@ __global__ __launch_bounds__(NS > 0 ? 1024 : 512) void k_fr_colfft_adj(const flo
         });
     return;
   }
-  for (int idx = tid; idx < CB * lds_padded_len(n2); idx += nt) sm[idx] = make_float2(0.f, 0.f);
+  for (int idx = tid; idx < CB * n2; idx += nt) sm[idx] = make_float2(0.f, 0.f);
   __syncthreads();
   stage_lds<8, float2>(
       CB * n, tid, nt,
@@ -952,20 +950,20 @@ __global__ __launch_bounds__(NS > 0 ? 1024 : 512) void k_fr_colfft_adj(const flo
         const int2 ci = circ[ty];
         const float ph =
             (tx >= ci.x && tx < ci.y) ? phix[tx] * phiy[ty] * ((u & 1) ? -1.f : 1.f) : 0.f;
-        sm[(lds_pad(u) << lgCB) + t] = make_float2(v.x * ph, v.y * ph);
+        sm[(u << lgCB) + t] = make_float2(v.x * ph, v.y * ph);
       });
   __syncthreads();
-  lds_fft<-1, (NS < 0 ? kFftEPT : kColEPT), fft_lv(NS)>(sm, fd, lgCB, tid, nt);
+  lds_fft<-1>(sm, fd, lgCB, tid, nt);
   for (int idx = tid; idx < CB * n2; idx += nt) {
     const int a = idx >> lgCB, t = idx & (CB - 1);
     if (v0 + t >= n) continue;
-    const float2 x = sm[(lds_pad(a) << lgCB) + t];
+    const float2 x = sm[(a << lgCB) + t];
     dst[(size_t)a * n + v0 + t] = (a & 1) ? make_float2(-x.x, -x.y) : x;
   }
 }
 
 template <int NS>
-__global__ __launch_bounds__(512) void k_fr_rowfft_adj(const float2 *__restrict__ R, float2 *__restrict__ F, FftDesc fd,
+__global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_rowfft_adj(const float2 *__restrict__ R, float2 *__restrict__ F, FftDesc fd,
                                 int n, int nzc) {
   extern __shared__ float2 sm[];
   const int a = blockIdx.x, c = blockIdx.y;
@@ -987,12 +985,12 @@ __global__ __launch_bounds__(512) void k_fr_rowfft_adj(const float2 *__restrict_
   stage_lds<8, float2>(
       n2, tid, nt,
       [&](int v) { return (v >= h && v < h + n) ? src[v - h] : make_float2(0.f, 0.f); },
-      [&](int v, float2 x) { sm[lds_pad(v)] = (v & 1) ? make_float2(-x.x, -x.y) : x; });
+      [&](int v, float2 x) { sm[v] = (v & 1) ? make_float2(-x.x, -x.y) : x; });
   __syncthreads();
-  lds_fft<-1, kFftEPT, fft_lv(NS)>(sm, fd, 0, tid, nt);
+  lds_fft<-1>(sm, fd, 0, tid, nt);
   float2 *dst = F + ((size_t)c * n2 + a) * n2;
   for (int b = tid; b < n2; b += nt) {
-    const float2 x = sm[lds_pad(b)];
+    const float2 x = sm[b];
     dst[b] = (b & 1) ? make_float2(-x.x, -x.y) : x;
   }
 }
@@ -1118,7 +1116,7 @@ __global__ __launch_bounds__(256) void k_fr_interp_sum(const int4 *__restrict__ 
 // back to the two real slices of the pair.  NS as k_fr_prep: compiled sizes
 // read the spectrum straight into the first pass and store from the last.
 template <int NS>
-__global__ __launch_bounds__(512) void k_fr_prep_adj(const float2 *__restrict__ G,
+__global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_prep_adj(const float2 *__restrict__ G,
                                                      float *__restrict__ data, FftDesc fd, int n,
                                                      int nproj, int nz, int nzc, float scale) {
   extern __shared__ float2 sm[];
@@ -1140,11 +1138,11 @@ __global__ __launch_bounds__(512) void k_fr_prep_adj(const float2 *__restrict__ 
   } else {
     stage_lds<8, float2>(
         n, tid, nt, [&](int k) { return in[k]; },
-        [&](int k, float2 v) { sm[lds_pad(k)] = cscale(v, shift_sign(k) * scale); });
+        [&](int k, float2 v) { sm[k] = cscale(v, shift_sign(k) * scale); });
     __syncthreads();
-    lds_fft<1, kFftEPT, fft_lv(NS)>(sm, fd, 0, tid, nt);
+    lds_fft<1>(sm, fd, 0, tid, nt);
     for (int j = tid; j < n; j += nt) {
-      const float2 x = cscale(sm[lds_pad(j)], shift_sign(j));
+      const float2 x = cscale(sm[j], shift_sign(j));
       r1[j] = x.x;
       if (z2 < nz) r2[j] = x.y;
     }
@@ -1168,11 +1166,11 @@ struct tomo_fr_plan {
   int ntile = 0, nitems = 0, nred = 0, nslots = 0;
   DevBuf G, F, R;
   int colCB = 1, lgCB = 0, colThreads = 256, prepThreads = 256, rowThreads = 256;
+  int fpThreads = 256;                   // k_fr_filtprep (transforms of n and 2n)
   int nsRow = 0, nsCol = 0, nsPrep = 0;  // compiled FFT sizes in use (0 = run-time sizes)
-  int colThreadsStatic = 1024;           // column-pass workgroup of the compiled sizes
   int lgB = 0;                           // column-blocked R (see k_fr_rowfft)
   int gridChunk = kGridChunk;            // max list entries per gridding work item
-  int rowLds = 0, prepLds = 0;
+  int rowLds = 0, prepLds = 0, fpLds = 0;
   size_t colLds = 0;
   float scale1 = 0.f, K2 = 0.f;
 };
@@ -1389,7 +1387,7 @@ int build_tables(tomo_fr_plan *P, const std::vector<float> &theta) {
 // 512 threads at their values per thread.  Rejects e.g. n = 4000
 // (2n = 2^6 5^3: 15 values per thread in the radix-5 passes, 576 threads).
 int fr_fft_shapes_ok(int64_t n) {
-  FftDesc d1{}, d2{};
+  FftRule d1{}, d2{};
   int rc = FftPlan::radices((int)n, d1);
   if (!rc) rc = FftPlan::radices((int)(2 * n), d2);
   if (rc) return rc;
@@ -1483,58 +1481,61 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
   // F and R in the plan's storage precision (float32 when the adjoint may run)
   if ((rc = P->F.alloc(P->csz * (size_t)P->ngrp * 4 * plane))) return fail(rc);
   if ((rc = P->R.alloc(P->csz * (size_t)P->ngrp * 4 * n2 * n))) return fail(rc);
-  // column pass: CB columns of length 2n in LDS
+  // workgroup shapes: size-specialised kernels where 2n is a compiled size
+  // (with_static_size): the row pass, and the column pass with col_lg(2n)
+  // columns per workgroup (up to 1024 threads at 16 values each, 15 with
+  // radix-3/5 passes); the spectrum kernels where n is one too.  Otherwise the
+  // run-time plans.
   const size_t maxlds = max_lds_per_block();
-  const size_t col1 = (size_t)lds_padded_len((int)n2) * sizeof(float2);
-  // the general-size column kernel (NS = -1) stages 16 values per thread: its
-  // radix-5/7 and prime passes spill at 32
-  const int colEPT = fft_general(n) ? kFftEPT : kColEPT;
-  int CB = 1, lg = 0;
-  while (CB * 2 <= 16 && (size_t)(CB * 2) * col1 <= maxlds &&
-         fft_threads(P->fft2.d, (int64_t)(CB * 2) * n2, colEPT) > 0 &&
-         fft_threads(P->fft2.d, (int64_t)(CB * 2) * n2, colEPT) <= 512)
-    CB *= 2, lg += 1;
-  P->colCB = CB;
-  P->lgCB = lg;
-  P->colLds = (size_t)CB * col1;
-  TOMO_REQUIRE(P->colLds <= maxlds, "fr_create: 2n=%lld exceeds the LDS of one workgroup", (long long)n2);
-  P->colThreads = fft_threads(P->fft2.d, (int64_t)CB * n2, colEPT);
-  P->prepThreads = fft_threads(P->fft1.d, n);
-  P->rowThreads = fft_threads(P->fft2.d, n2);
-  if (P->colThreads < 0 || P->prepThreads < 0 || P->rowThreads < 0 || P->colThreads > 512 ||
-      P->prepThreads > 512 || P->rowThreads > 512) {
-    set_error("fr_create: n=%lld needs more than 512 threads per FFT workgroup", (long long)n);
-    return fail(TOMO_EINVAL);
-  }
-  // size-specialised kernels where 2n is a compiled size (with_static_size):
-  // the row pass, and the column pass with col_lg(2n) columns per workgroup
-  // (up to 1024 threads at 16 values each, 15 with radix-3/5 passes); the
-  // spectrum kernels where n is one too.  Otherwise the run-time-plan
-  // kernels of the size's transform level (0, -1, -2).
-  const int lev = fft_level(n);
-  const int rt = lev == 2 ? -2 : (lev == 1 ? -1 : 0);
   const bool st2 = !fft_generic && static_fft_size((int)n2);
-  P->nsRow = st2 ? (int)n2 : rt;
-  P->nsCol = rt;
+  auto lds_bytes = [](bool compiled, int64_t N) {
+    return sizeof(float2) * (size_t)(compiled ? lds_padded_len((int)N) : N);
+  };
+  P->nsRow = st2 ? (int)n2 : 0;
+  P->nsPrep = (st2 && static_fft_size((int)n)) ? (int)n : 0;
+  P->rowThreads = st2 ? fft_threads(P->fft2.rule, n2) : fft_rt_threads(P->fft2.d, 0);
+  P->rowLds = (int)lds_bytes(st2, n2);
+  if (P->nsPrep > 0) {
+    P->prepThreads = fft_threads(P->fft1.rule, n);
+    P->fpThreads = fft_threads(P->fft2.rule, n2);
+  } else {
+    P->prepThreads = fft_rt_threads(P->fft1.d, 0);
+    P->fpThreads = std::max(P->prepThreads, fft_rt_threads(P->fft2.d, 0));
+  }
+  P->prepLds = (int)lds_bytes(P->nsPrep > 0, n);
+  P->fpLds = (int)lds_bytes(P->nsPrep > 0, n2);
+  P->nsCol = 0;
   if (st2) {
     const int lgs = col_lg((int)n2);
-    const size_t lds_s = (size_t)(1 << lgs) * col1;
-    const int thr = fft_threads(P->fft2.d, (int64_t)n2 << lgs, kFftEPT);
+    const size_t lds_s = lds_bytes(true, n2) << lgs;
+    const int thr = fft_threads(P->fft2.rule, (int64_t)n2 << lgs, kFftEPT);
     if (lds_s <= maxlds && thr > 0 && thr <= 1024) {
       P->nsCol = (int)n2;
-      CB = 1 << lgs;
-      lg = lgs;
-      P->colCB = CB;
-      P->lgCB = lg;
+      P->lgCB = lgs;
       P->colLds = lds_s;
-      P->colThreadsStatic = thr;
+      P->colThreads = thr;
     }
+  }
+  if (P->nsCol == 0) {
+    // run-time plan: as many columns (a power of two, at most 16) as fit
+    while (P->lgCB < 4 && (lds_bytes(false, n2) << (P->lgCB + 1)) <= maxlds &&
+           fft_rt_threads(P->fft2.d, P->lgCB + 1) > 0 && !fft_rt_wide(P->fft2.d, P->lgCB + 1))
+      P->lgCB += 1;
+    P->colLds = lds_bytes(false, n2) << P->lgCB;
+    P->colThreads = fft_rt_threads(P->fft2.d, P->lgCB);
+  }
+  P->colCB = 1 << P->lgCB;
+  const int lg = P->lgCB;
+  if (P->colThreads <= 0 || P->prepThreads <= 0 || P->rowThreads <= 0 || P->fpThreads <= 0 ||
+      P->colLds > maxlds) {
+    set_error("fr_create: n=%lld needs more threads or LDS than an FFT workgroup has",
+              (long long)n);
+    return fail(TOMO_EINVAL);
   }
   // column-blocked R for 16-bit plans only: measured at n=2048 the column
   // pass gains 40-50 us per chunk of 8 slices, the row pass loses 22 us
   // (16-byte segments) in half precision and 43 us (32-byte) in float32
   P->lgB = (dtype != TOMO_F32 && n % (1 << lg) == 0) ? lg : 0;
-  P->nsPrep = (st2 && static_fft_size((int)n)) ? (int)n : rt;
   hipError_t ea = hipSuccess;
   auto lds_attr = [&](const void *k, size_t bytes) {
     if (ea == hipSuccess)
@@ -1553,9 +1554,7 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
   with_static_size(P->nsCol, [&](auto ns) {
     lds_attr((const void *)k_fr_colfft_adj<decltype(ns)::value>, P->colLds);
   });
-  const int rowLds = (int)(lds_padded_len((int)n2) * sizeof(float2));
-  P->rowLds = rowLds;
-  P->prepLds = (int)(lds_padded_len((int)n) * sizeof(float2));
+  const int rowLds = P->rowLds;
   with_static_size(P->nsRow, [&](auto ns) {
     constexpr int NS = decltype(ns)::value;
     lds_attr((const void *)k_fr_rowfft<float, NS>, rowLds);
@@ -1640,7 +1639,7 @@ static int fr_tail_after_grid(tomo_fr_plan *P, T *obj, hipStream_t st) {
     with_static_size(P->nsCol, [&](auto ns) {
       hipLaunchKernelGGL((k_fr_colfft<T, decltype(ns)::value>),
                          dim3((unsigned)ceil_div(n, P->colCB), ng * 4),
-                         dim3(decltype(ns)::value > 0 ? P->colThreadsStatic : P->colThreads),
+                         dim3(P->colThreads),
                          P->colLds, st, R, obj, P->phix.as<float>(), P->phiy.as<float>(),
                          P->circ.as<int2>(), P->fft2.d, n, nz, nzc, P->lgCB, P->lgB > 0 ? 1 : 0);
     });
@@ -1673,7 +1672,7 @@ static int fr_head(tomo_fr_plan *P, tomo_flt_plan *F, const T *data, hipStream_t
     ProfScope ps_("k_fr_filtprep", st);
     with_static_size(P->nsPrep, [&](auto ns) {
       hipLaunchKernelGGL((k_fr_filtprep<T, decltype(ns)::value>), dim3(nproj, ng * 4),
-                         dim3(P->rowThreads), P->rowLds, st, data, P->G.as<cpx<T>>(),
+                         dim3(P->fpThreads), P->fpLds, st, data, P->G.as<cpx<T>>(),
                          F->H2.as<float2>(), F->HL.as<float>(), F->HR.as<float>(), F->fft2n.d,
                          P->fft1.d, n, nproj, nz, nzc, P->scale1, P->gmax.as<float>());
     });
@@ -1977,7 +1976,7 @@ extern "C" int fr_forward(tomo_fr_plan *P, void *data_, const void *obj_, void *
     with_static_size(P->nsCol, [&](auto ns) {
       constexpr int NS = decltype(ns)::value;
       hipLaunchKernelGGL(k_fr_colfft_adj<NS>, dim3((unsigned)ceil_div(n, P->colCB), ng * 4),
-                         dim3(NS > 0 ? P->colThreadsStatic : P->colThreads), P->colLds, st, obj,
+                         dim3(P->colThreads), P->colLds, st, obj,
                          P->R.as<float2>(),
                          P->phix.as<float>(), P->phiy.as<float>(), P->circ.as<int2>(),
                          P->fft2.d, n, nz, nzc, P->lgCB);
@@ -2042,8 +2041,8 @@ extern "C" void fr_destroy(tomo_fr_plan *P) {
   P->G.release();
   P->F.release();
   P->R.release();
-  P->fft1.tw.release();
-  P->fft2.tw.release();
+  P->fft1.release();
+  P->fft2.release();
   delete P;
 }
 

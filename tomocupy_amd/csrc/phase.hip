@@ -53,6 +53,38 @@ constexpr double kPi = 3.14159265359;               // retrieve_phase.py:48
 constexpr double kPlanck = 6.58211928e-19;          // [keV s], :49
 constexpr double kLight = 299792458e+2;             // [cm/s], :47
 
+// Padded lengths are powers of two: f(integral_constant<int, N>) for the
+// compiled lengths 512 .. 8192, f(integral_constant<int, 0>) (run-time plan)
+// below.
+template <typename F>
+void with_ph_size(int N, F &&f) {
+  switch (N) {
+    case 512: f(std::integral_constant<int, 512>()); break;
+    case 1024: f(std::integral_constant<int, 1024>()); break;
+    case 2048: f(std::integral_constant<int, 2048>()); break;
+    case 4096: f(std::integral_constant<int, 4096>()); break;
+    case 8192: f(std::integral_constant<int, 8192>()); break;
+    default: f(std::integral_constant<int, 0>()); break;
+  }
+}
+
+// log2 of the columns of a column-pass workgroup: at most 8 columns and 8192
+// elements (64 KB of LDS)
+constexpr int ph_lg(int N) {
+  int lg = 0;
+  while (lg < 3 && (N << (lg + 1)) <= 8192) ++lg;
+  return lg;
+}
+
+// the transform of 2^LG (compiled) or 2^lg (run-time) sequences in LDS
+template <int NS, int DIR, int LG>
+__device__ __forceinline__ void ph_fft(float2 *sm, const FftDesc &fd, int lg, int tid, int nt) {
+  if constexpr (NS > 0)
+    lds_fft_c<NS, DIR, kFftEPT, LG>(sm, fd.tw, tid, nt);
+  else
+    lds_fft<DIR>(sm, fd, lg, tid, nt);
+}
+
 // the method's factor at one grid point, from the sum of the two 1-D terms
 __device__ __forceinline__ float ph_factor(int method, float s, float A, float B, float alpha,
                                            float db) {
@@ -85,27 +117,28 @@ __global__ __launch_bounds__(256) void k_ph_fmax(const float *__restrict__ ty,
 // Forward FFTs of the column-padded real rows 2 pr and 2 pr + 1 of
 // projection blockIdx.y: z = row0 + i row1, Z = fft(z);
 // X0 = (Z[k] + conj Z[-k]) / 2, X1 = (Z[k] - conj Z[-k]) / (2i).
+template <int NS>
 __global__ __launch_bounds__(512) void k_ph_rows_fwd(const float *__restrict__ data,
                                                       float2 *__restrict__ F, FftDesc fd, int dy,
                                                       int dz, int pz) {
   extern __shared__ float2 sm[];
   const int pr = blockIdx.x, b = blockIdx.y;
   const int tid = threadIdx.x, nt = blockDim.x;
-  const int Nx = fd.N;
+  const int Nx = NS > 0 ? NS : fd.N;
   const int iy0 = 2 * pr;
   const float *img = data + (size_t)b * dy * dz;
   const float *r0 = img + (size_t)iy0 * dz;
   const float *r1 = r0 + dz;
   for (int ix = tid; ix < Nx; ix += nt) {
     const int sx = min(max(ix - pz, 0), dz - 1);
-    sm[lds_pad(ix)] = make_float2(r0[sx], r1[sx]);
+    sm[lidx<NS>(ix)] = make_float2(r0[sx], r1[sx]);
   }
   __syncthreads();
-  lds_fft<-1>(sm, fd, 0, tid, nt);
+  ph_fft<NS, -1, 0>(sm, fd, 0, tid, nt);
   float2 *f0 = F + ((size_t)b * dy + iy0) * Nx;
   float2 *f1 = f0 + Nx;
   for (int k = tid; k < Nx; k += nt) {
-    const float2 zk = sm[lds_pad(k)], zm = cconj(sm[lds_pad(k == 0 ? 0 : Nx - k)]);
+    const float2 zk = sm[lidx<NS>(k)], zm = cconj(sm[lidx<NS>(k == 0 ? 0 : Nx - k)]);
     f0[k] = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y + zm.y));
     f1[k] = make_float2(0.5f * (zk.y - zm.y), -0.5f * (zk.x - zm.x));
   }
@@ -115,6 +148,7 @@ __global__ __launch_bounds__(512) void k_ph_rows_fwd(const float *__restrict__ d
 // padded column (padded row ky holds real row clamp(ky - py, 0, dy - 1)),
 // forward FFT, times H / max H / (Ny Nx), inverse FFT; rows py .. py+dy-1
 // written back in place.
+template <int NS>
 __global__ __launch_bounds__(512) void k_ph_cols(float2 *__restrict__ F, FftDesc fd,
                                                   int lgC, int Nx, int dy, int py,
                                                   const float *__restrict__ ty,
@@ -123,7 +157,8 @@ __global__ __launch_bounds__(512) void k_ph_cols(float2 *__restrict__ F, FftDesc
                                                   float hmax, float scale) {
   extern __shared__ float2 sm[];
   const int tid = threadIdx.x, nt = blockDim.x;
-  const int Ny = fd.N, C = 1 << lgC;
+  if (NS > 0) lgC = ph_lg(NS);
+  const int Ny = NS > 0 ? NS : fd.N, C = 1 << lgC;
   // workgroups are dealt to the 8 XCDs in turn: give each XCD a contiguous
   // range of column groups, so that the groups sharing cache lines (2^lgC
   // columns = 8 << lgC bytes of each row) share its L2
@@ -133,21 +168,21 @@ __global__ __launch_bounds__(512) void k_ph_cols(float2 *__restrict__ F, FftDesc
   float2 *fb = F + (size_t)b * dy * Nx + kx0;
   for (int e = tid; e < (Ny << lgC); e += nt) {
     const int ky = e >> lgC, c = e & (C - 1);
-    sm[(lds_pad(ky) << lgC) + c] = fb[(size_t)min(max(ky - py, 0), dy - 1) * Nx + c];
+    sm[(lidx<NS>(ky) << lgC) + c] = fb[(size_t)min(max(ky - py, 0), dy - 1) * Nx + c];
   }
   __syncthreads();
-  lds_fft<-1>(sm, fd, lgC, tid, nt);
+  ph_fft<NS, -1, ph_lg(NS)>(sm, fd, lgC, tid, nt);
   for (int e = tid; e < (Ny << lgC); e += nt) {
     const int ky = e >> lgC, c = e & (C - 1);
     const float h = ph_factor(method, ty[ky] + tx[kx0 + c], A, B, alpha, db) / hmax * scale;
-    float2 &v = sm[(lds_pad(ky) << lgC) + c];
+    float2 &v = sm[(lidx<NS>(ky) << lgC) + c];
     v = make_float2(v.x * h, v.y * h);
   }
   __syncthreads();
-  lds_fft<1>(sm, fd, lgC, tid, nt);
+  ph_fft<NS, 1, ph_lg(NS)>(sm, fd, lgC, tid, nt);
   for (int e = tid; e < (dy << lgC); e += nt) {
     const int y = e >> lgC, c = e & (C - 1);
-    fb[(size_t)y * Nx + c] = sm[(lds_pad(y + py) << lgC) + c];
+    fb[(size_t)y * Nx + c] = sm[(lidx<NS>(y + py) << lgC) + c];
   }
 }
 
@@ -155,13 +190,14 @@ __global__ __launch_bounds__(512) void k_ph_cols(float2 *__restrict__ F, FftDesc
 // Re ifft(G) = ifft(Herm G), Herm G[k] = (G[k] + conj G[-k]) / 2, so
 // ifft(Herm G0 + i Herm G1) = Re ifft(G0) + i Re ifft(G1); cropped columns
 // written back to the projection.
+template <int NS>
 __global__ __launch_bounds__(512) void k_ph_rows_inv(float *__restrict__ data,
                                                       const float2 *__restrict__ F, FftDesc fd,
                                                       int dy, int dz, int pz) {
   extern __shared__ float2 sm[];
   const int pr = blockIdx.x, b = blockIdx.y;
   const int tid = threadIdx.x, nt = blockDim.x;
-  const int Nx = fd.N;
+  const int Nx = NS > 0 ? NS : fd.N;
   const int oy0 = 2 * pr, oy1 = oy0 + 1;  // dy is even: both rows exist
   const float2 *g0 = F + ((size_t)b * dy + oy0) * Nx;
   const float2 *g1 = g0 + Nx;
@@ -170,13 +206,13 @@ __global__ __launch_bounds__(512) void k_ph_rows_inv(float *__restrict__ data,
     const float2 a = g0[k], am = g0[km], c = g1[k], cm = g1[km];
     const float2 h0 = make_float2(0.5f * (a.x + am.x), 0.5f * (a.y - am.y));
     const float2 h1 = make_float2(0.5f * (c.x + cm.x), 0.5f * (c.y - cm.y));
-    sm[lds_pad(k)] = make_float2(h0.x - h1.y, h0.y + h1.x);
+    sm[lidx<NS>(k)] = make_float2(h0.x - h1.y, h0.y + h1.x);
   }
   __syncthreads();
-  lds_fft<1>(sm, fd, 0, tid, nt);
+  ph_fft<NS, 1, 0>(sm, fd, 0, tid, nt);
   float *img = data + (size_t)b * dy * dz;
   for (int x = tid; x < dz; x += nt) {
-    const float2 v = sm[lds_pad(pz + x)];
+    const float2 v = sm[lidx<NS>(pz + x)];
     img[(size_t)oy0 * dz + x] = v.x;
     if (oy1 < dy) img[(size_t)oy1 * dz + x] = v.y;
   }
@@ -194,8 +230,8 @@ bool pow2(int v) { return v >= 2 && (v & (v - 1)) == 0; }
 
 extern "C" void ph_destroy(tomo_ph_plan *P) {
   if (!P) return;
-  P->fy.tw.release();
-  P->fx.tw.release();
+  P->fy.release();
+  P->fx.release();
   P->ty.release();
   P->tx.release();
   P->F.release();
@@ -300,14 +336,28 @@ extern "C" int ph_create(tomo_ph_plan **plan, int64_t dy, int64_t dz, int64_t ba
       return TOMO_EINVAL;
     }
   }
-  // launch shapes: rows one transform per workgroup; columns 2^lgC
-  // interleaved transforms, at most 8192 elements (64 KB of LDS)
-  P->lgC = 0;
-  while (P->lgC < 3 && ((int64_t)P->Ny << (P->lgC + 1)) <= 8192) ++P->lgC;
-  P->rowThreads = fft_threads(P->fx.d, P->Nx);
-  P->colThreads = fft_threads(P->fy.d, (int64_t)P->Ny << P->lgC);
-  P->rowLds = sizeof(float2) * lds_padded_len(P->Nx);
-  P->colLds = sizeof(float2) * ((size_t)lds_padded_len(P->Ny) << P->lgC);
+  // launch shapes: rows one transform per workgroup, columns 2^lgC interleaved
+  // transforms
+  P->lgC = ph_lg(P->Ny);
+  hipError_t e = hipSuccess;
+  auto lds_attr = [&](const void *k, size_t bytes) {
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  };
+  with_ph_size(P->Nx, [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    P->rowThreads = NS > 0 ? fft_threads(P->fx.rule, NS) : fft_rt_threads(P->fx.d, 0);
+    P->rowLds = sizeof(float2) * (NS > 0 ? lds_padded_len(NS) : P->Nx);
+    lds_attr((const void *)k_ph_rows_fwd<NS>, P->rowLds);
+    lds_attr((const void *)k_ph_rows_inv<NS>, P->rowLds);
+  });
+  with_ph_size(P->Ny, [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    P->colThreads = NS > 0 ? fft_threads(P->fy.rule, (int64_t)NS << P->lgC)
+                           : fft_rt_threads(P->fy.d, P->lgC);
+    P->colLds = sizeof(float2) * ((size_t)(NS > 0 ? lds_padded_len(NS) : P->Ny) << P->lgC);
+    lds_attr((const void *)k_ph_cols<NS>, P->colLds);
+  });
   if (P->rowThreads <= 0 || P->rowThreads > 512 || P->colThreads <= 0 ||
       P->colThreads > 512 || P->rowLds > max_lds_per_block() ||
       P->colLds > max_lds_per_block()) {
@@ -315,14 +365,6 @@ extern "C" int ph_create(tomo_ph_plan **plan, int64_t dy, int64_t dz, int64_t ba
     ph_destroy(P);
     return TOMO_EINVAL;
   }
-  hipError_t e = hipFuncSetAttribute((const void *)k_ph_rows_fwd,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->rowLds);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void *)k_ph_rows_inv,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->rowLds);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void *)k_ph_cols, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)P->colLds);
   if (e != hipSuccess) {
     set_error("ph_create: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
     ph_destroy(P);
@@ -355,22 +397,30 @@ extern "C" int ph_apply(tomo_ph_plan *P, float *data, int64_t nproj, void *strea
     float *img = data + (size_t)b0 * dy * dz;
     {
       ProfScope ps_("k_ph_rows_fwd", st);
-      hipLaunchKernelGGL(k_ph_rows_fwd, dim3((unsigned)(dy / 2), nb), dim3(P->rowThreads),
-                         P->rowLds, st, img, P->F.as<float2>(), P->fx.d, dy, dz, P->pz);
+      with_ph_size(P->Nx, [&](auto ns) {
+        hipLaunchKernelGGL(k_ph_rows_fwd<decltype(ns)::value>, dim3((unsigned)(dy / 2), nb),
+                           dim3(P->rowThreads), P->rowLds, st, img, P->F.as<float2>(), P->fx.d,
+                           dy, dz, P->pz);
+      });
     }
     TOMO_LAUNCH_CHECK();
     {
       ProfScope ps_("k_ph_cols", st);
-      hipLaunchKernelGGL(k_ph_cols, dim3((unsigned)(P->Nx >> P->lgC), nb), dim3(P->colThreads),
-                         P->colLds, st, P->F.as<float2>(), P->fy.d, P->lgC, P->Nx, dy, P->py,
-                         P->ty.as<float>(), P->tx.as<float>(), P->method, P->A, P->B, P->alpha,
-                         P->db, P->hmax, scale);
+      with_ph_size(P->Ny, [&](auto ns) {
+        hipLaunchKernelGGL(k_ph_cols<decltype(ns)::value>, dim3((unsigned)(P->Nx >> P->lgC), nb),
+                           dim3(P->colThreads), P->colLds, st, P->F.as<float2>(), P->fy.d,
+                           P->lgC, P->Nx, dy, P->py, P->ty.as<float>(), P->tx.as<float>(),
+                           P->method, P->A, P->B, P->alpha, P->db, P->hmax, scale);
+      });
     }
     TOMO_LAUNCH_CHECK();
     {
       ProfScope ps_("k_ph_rows_inv", st);
-      hipLaunchKernelGGL(k_ph_rows_inv, dim3((unsigned)(dy / 2), nb), dim3(P->rowThreads),
-                         P->rowLds, st, img, P->F.as<float2>(), P->fx.d, dy, dz, P->pz);
+      with_ph_size(P->Nx, [&](auto ns) {
+        hipLaunchKernelGGL(k_ph_rows_inv<decltype(ns)::value>, dim3((unsigned)(dy / 2), nb),
+                           dim3(P->rowThreads), P->rowLds, st, img, P->F.as<float2>(), P->fx.d,
+                           dy, dz, P->pz);
+      });
     }
     TOMO_LAUNCH_CHECK();
   }
