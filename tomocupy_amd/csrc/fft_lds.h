@@ -353,7 +353,7 @@ __device__ __forceinline__ float2 rotate(float2 v) {
 
 // First factor of the split R = A * B of a composite radix.
 constexpr int dft_split(int R) {
-  return R == 12 ? 4 : R == 20 ? 5 : R == 15 || R == 9 ? 3 : R == 18 ? 9 : 2;
+  return R == 12 || R == 32 ? 4 : R == 20 ? 5 : R == 15 || R == 9 ? 3 : R == 18 ? 9 : 2;
 }
 
 // a <- DFT_R(a) in natural order, in registers, every constant a literal.
@@ -781,8 +781,9 @@ __device__ __forceinline__ void fft_pass_c_first(float2 *buf, int tid, int nt, L
   }
 }
 
-// The last pass (sub-transform length Ns) from LDS to st.
-template <int R, int Ns, int N, int DIR, int EPT, int LGH, typename St>
+// The last pass (sub-transform length Ns) from LDS to st.  Outputs outside
+// [LO, HI) are dropped, and not computed where all of a register's are outside.
+template <int R, int Ns, int N, int DIR, int EPT, int LGH, int LO = 0, int HI = N, typename St>
 __device__ __forceinline__ void fft_pass_c_last(const float2 *buf, const float2 *__restrict__ tw,
                                                 int tid, int nt, St st) {
   constexpr int MAXB = EPT / R;
@@ -804,9 +805,14 @@ __device__ __forceinline__ void fft_pass_c_last(const float2 *buf, const float2 
       const int k = j % Ns;
       twiddle<R, DIR>(v, tw, (unsigned)(k * twstep));
       butterfly<R, DIR>(v);
-      const int o = (j - k) * R + k;
+      // (Ns = N / R: k = j, output r is element k + r Ns)
+      __builtin_assume(k >= 0 && k < Ns);
 #pragma unroll
-      for (int r = 0; r < R; ++r) st(o + r * Ns, t, v[out_slot<R>(r)]);
+      for (int r = 0; r < R; ++r) {
+        if ((r + 1) * Ns <= LO || r * Ns >= HI) continue;
+        const int o = k + r * Ns;
+        if (o >= LO && o < HI) st(o, t, v[out_slot<R>(r)]);
+      }
     }
   }
 }
@@ -821,7 +827,7 @@ __device__ __forceinline__ void fft_c_from_global(float2 *buf, const float2 *__r
   lds_fft_c<N, DIR, EPT, LGH, 1, R0>(buf, tw, tid, nt);
 }
 
-template <int N, int DIR, int EPT, int LGH, typename Ld, typename St>
+template <int N, int DIR, int EPT, int LGH, int LO = 0, int HI = N, typename Ld, typename St>
 __device__ __forceinline__ void fft_c_global(float2 *buf, const float2 *__restrict__ tw, int tid,
                                              int nt, Ld ld, St st) {
   using SP = StaticPlan<N>;
@@ -831,7 +837,152 @@ __device__ __forceinline__ void fft_c_global(float2 *buf, const float2 *__restri
   fft_pass_c_first<R0, N, DIR, EPT, LGH>(buf, tid, nt, ld);
   __syncthreads();
   lds_fft_c<N, DIR, EPT, LGH, 1, R0, SP::passes - 1>(buf, tw, tid, nt);
-  fft_pass_c_last<RL, N / RL, N, DIR, EPT, LGH>(buf, tw, tid, nt, st);
+  fft_pass_c_last<RL, N / RL, N, DIR, EPT, LGH, LO, HI>(buf, tw, tid, nt, st);
+}
+
+// ---- compile-time transforms exchanged one component at a time ----------
+// fft_c_split is fft_c_global with kFftSplitEPT values per thread kept in
+// registers through the whole transform: between passes the real parts go
+// through LDS, then the imaginary parts, so the buffer holds 4 bytes per
+// element and a workgroup takes twice the sequences.  For the column passes,
+// whose sequences are columns, that doubles the bytes a workgroup uses of each
+// cache line (a line is read once per workgroup that needs a part of it).
+// Outputs outside [LO, HI) are dropped, and not computed where a whole
+// register of the last pass is outside.
+constexpr int kFftSplitEPT = 32;
+
+// log2 of the sequences a split workgroup takes: as many as 1024 threads hold,
+// at most 16 (15 of a thread's values in the radix-3 and 5 passes).
+constexpr int split_lg(int N) {
+  return ilog2c(1024 * kFftSplitEPT / N) > 4 ? 4 : ilog2c(1024 * kFftSplitEPT / N);
+}
+
+// Its radices: those of StaticPlan, but a left-over factor 2 joins the first
+// pass (radix 32, without twiddles).
+template <int N>
+struct SplitPlan {
+  using SP = StaticPlan<N>;
+  static constexpr bool r32 = SP::rest == 2;
+  static constexpr int passes = SP::passes - (r32 ? 1 : 0);
+  static constexpr int radix(int s) {
+    return !r32 ? SP::radix(s) : s == 0 ? 32 : s < SP::n16 ? 16 : SP::radix(s + 1);
+  }
+};
+
+// a <- DFT_R(a), outputs in slots out_slot<R>(q).
+template <int R, int DIR>
+__device__ __forceinline__ void split_butterfly(float2 *a) {
+  if constexpr (R == 32)
+    dft<32, DIR>(a);
+  else
+    butterfly<R, DIR>(a);
+}
+
+template <int R, int Ns, int N, int DIR, int LGH>
+__device__ __forceinline__ void split_butterflies(float2 *v, const float2 *__restrict__ tw,
+                                                  int tid, int nt) {
+  constexpr int MAXB = kFftSplitEPT / R, nb = (N / R) << LGH;
+#pragma unroll
+  for (int q = 0; q < MAXB; ++q) {
+    const int g = tid + q * nt;
+    if (g < nb) {
+      if constexpr (Ns > 1)
+        twiddle<R, DIR>(v + q * R, tw, (unsigned)(((g >> LGH) % Ns) * (N / (Ns * R))));
+      split_butterfly<R, DIR>(v + q * R);
+    }
+  }
+}
+
+// Outputs of a radix-R pass (length Ns before it) to the inputs of the next,
+// radix R2: v is replaced.
+template <int R, int Ns, int R2, int N, int LGH>
+__device__ __forceinline__ void split_exchange(float2 *v, float *buf, int tid, int nt) {
+  constexpr int MAXB = kFftSplitEPT / R, nb = (N / R) << LGH, H = 1 << LGH;
+  constexpr int MAXB2 = kFftSplitEPT / R2, nb2 = (N / R2) << LGH;
+  static_assert((N / R) % 16 == 0 && (N / R2) % 16 == 0 && (Ns == 1 || Ns % 16 == 0), "layout");
+  // (output r of the first pass is element j R + r: a pad slot after 16)
+  constexpr int wstride = Ns == 1 ? H : (Ns + Ns / 16) << LGH;
+  constexpr int wpad = Ns == 1 ? H : 0;
+  constexpr int rstride = (N / R2 + N / R2 / 16) << LGH;
+  float x[kFftSplitEPT];
+  auto write = [&](auto part) {
+#pragma unroll
+    for (int q = 0; q < MAXB; ++q) {
+      const int g = tid + q * nt;
+      if (g < nb) {
+        const int t = g & (H - 1), j = g >> LGH, k = j % Ns;
+        float *o = buf + (lds_pad((j - k) * R + k) << LGH) + t;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          o[r * wstride + (r >> 4) * wpad] = part(v[q * R + out_slot<R>(r)]);
+      }
+    }
+  };
+  auto read = [&](auto put) {
+#pragma unroll
+    for (int q = 0; q < MAXB2; ++q) {
+      const int g = tid + q * nt;
+      if (g < nb2) {
+        const int t = g & (H - 1), j = g >> LGH;
+        const float *i = buf + (lds_pad(j) << LGH) + t;
+#pragma unroll
+        for (int r = 0; r < R2; ++r) put(q * R2 + r, i[r * rstride]);
+      }
+    }
+  };
+  write([](float2 a) { return a.x; });
+  __syncthreads();
+  read([&](int i, float a) { x[i] = a; });
+  __syncthreads();
+  write([](float2 a) { return a.y; });
+  __syncthreads();
+  read([&](int i, float a) { v[i] = make_float2(x[i], a); });
+}
+
+template <int N, int DIR, int LGH, int LO, int HI, int S, int Ns, typename St>
+__device__ __forceinline__ void split_rest(float2 *v, float *buf, const float2 *__restrict__ tw,
+                                           int tid, int nt, St st) {
+  using SP = SplitPlan<N>;
+  constexpr int R = SP::radix(S);
+  split_butterflies<R, Ns, N, DIR, LGH>(v, tw, tid, nt);
+  if constexpr (S + 1 < SP::passes) {
+    if constexpr (S > 0) __syncthreads();  // the last exchange's reads
+    split_exchange<R, Ns, SP::radix(S + 1), N, LGH>(v, buf, tid, nt);
+    split_rest<N, DIR, LGH, LO, HI, S + 1, Ns * R>(v, buf, tw, tid, nt, st);
+  } else {
+    constexpr int MAXB = kFftSplitEPT / R, nb = (N / R) << LGH, H = 1 << LGH;
+#pragma unroll
+    for (int q = 0; q < MAXB; ++q) {
+      const int g = tid + q * nt;
+      if (g < nb) {
+        const int t = g & (H - 1), j = g >> LGH;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          if ((r + 1) * Ns <= LO || r * Ns >= HI) continue;
+          const int o = j + r * Ns;
+          if (o >= LO && o < HI) st(o, t, v[q * R + out_slot<R>(r)]);
+        }
+      }
+    }
+  }
+}
+
+// buf: lds_padded_len(N) << LGH floats.
+template <int N, int DIR, int LGH, int LO, int HI, typename Ld, typename St>
+__device__ __forceinline__ void fft_c_split(float *buf, const float2 *__restrict__ tw, int tid,
+                                            int nt, Ld ld, St st) {
+  constexpr int R = SplitPlan<N>::radix(0);
+  constexpr int MAXB = kFftSplitEPT / R, nb = (N / R) << LGH, H = 1 << LGH;
+  float2 v[kFftSplitEPT];
+#pragma unroll
+  for (int q = 0; q < MAXB; ++q) {
+    const int g = tid + q * nt;
+    if (g < nb) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[q * R + r] = ld((g >> LGH) + r * (N / R), g & (H - 1));
+    }
+  }
+  split_rest<N, DIR, LGH, LO, HI, 0, 1>(v, buf, tw, tid, nt, st);
 }
 
 // Calls f(std::integral_constant<int, N>) for the sizes with a compiled

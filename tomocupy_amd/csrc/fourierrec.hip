@@ -51,6 +51,15 @@ constexpr int kColEPT = 32;     // column-pass values per thread in the width ru
 // log2 of the columns a column-pass workgroup transforms for 2n = N: as many
 // as fit 512 threads at kColEPT values each (and the LDS), at most 16
 constexpr int col_lg(int N) { return ilog2c(16384 / N) > 4 ? 4 : ilog2c(16384 / N); }
+// 2n = N whose column passes run fft_c_split (split_lg(N) columns): the sizes
+// where the split gives a workgroup twice the columns and at least 24 waves'
+// worth of values (row + column pass, us per chunk of 8 slices, float32, split
+// against fft_c_global: 2n = 2048 39+37 against 39+41, 3072 109+103 against
+// 99+123, 8192 782+533 against 729+1181; 2304, whose 8 columns are 18432
+// values, 61+81 against 56+59, so it stays with fft_c_global)
+constexpr bool col_split(int N) {
+  return N > 4096 || (N >= 2048 && (N << split_lg(N)) >= 24576);
+}
 
 // Sign 1 - 2*((t+1) % 2): -1 for even t, +1 for odd t (kernels_fourierrec.cuh:121-132).
 __device__ __forceinline__ float shift_sign(int t) { return (t & 1) ? 1.f : -1.f; }
@@ -766,9 +775,9 @@ __global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_rowfft(const cpx<T> 
   const int2 sp = span[a];
   const int h = n / 2;
   // compiled sizes, float32: the first pass loads the row and the last one
-  // stores R (measured at n = 2048: 161 -> 146 us per chunk of 8 slices; the
-  // 16-bit column-blocked R went from 164 to 209 us that way, so 16-bit plans
-  // stage through LDS)
+  // stores R (measured at n = 2048: 161 -> 146 us per chunk of 8 slices, the
+  // rate of a copy; 16-bit plans went from 170 to 209 us that way, their 2- and
+  // 4-byte accesses being too narrow for it, and stage through LDS)
   if constexpr (NS > 0 && std::is_same<T, float>::value) {
     fft_c_global<NS, 1, kFftEPT, 0>(
         sm, fd.tw, tid, nt,
@@ -818,9 +827,8 @@ __global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_rowfft(const cpx<T> 
   }
 }
 
-// The compiled column pass runs 16 values per thread (1024 threads): its LDS
-// (4 columns of 2n) admits one workgroup per CU, so the extra waves are the
-// only latency cover.
+// The compiled column pass fills a CU's LDS with one workgroup of 1024 threads
+// (8 columns of 4096 points, one component at a time).
 template <typename T, int NS>
 __global__ __launch_bounds__(1024) void k_fr_colfft(const cpx<T> *__restrict__ R, T *__restrict__ obj,
                             const float *__restrict__ phix, const float *__restrict__ phiy,
@@ -838,30 +846,37 @@ __global__ __launch_bounds__(1024) void k_fr_colfft(const cpx<T> *__restrict__ R
   const cpx<T> *blk = src + (size_t)v0 * n2;  // block cb of the column-blocked layout
   const int z2 = c + nzc;
   const int h = n / 2;
-  // compiled sizes, float32: the first pass loads R and the last one stores
-  // the slices (n = 2048: 205 -> 187 us per chunk of 8 slices; 16-bit plans,
-  // 129 -> 145 us, stage through LDS)
-  if constexpr (NS > 0 && std::is_same<T, float>::value) {
-    constexpr int LG = col_lg(NS);  // == lgCB (the plan picks NS only then)
-    fft_c_global<NS, 1, kFftEPT, LG>(
-        sm, fd.tw, tid, nt,
-        [&](int a, int t) {
-          float2 x;
-          if (blocked)
-            x = tof2(blk[(a << LG) + t]);
-          else
-            x = (v0 + t < n) ? tof2(src[(size_t)a * n + v0 + t]) : make_float2(0.f, 0.f);
-          return (a & 1) ? make_float2(-x.x, -x.y) : x;
-        },
-        [&](int u, int t, float2 x) {
-          const int ty = u - 1 - h, tx = v0 + t;
-          if (ty < 0 || ty >= n || tx >= n) return;
-          const int2 ci = circ[ty];
-          const float ph =
-              (tx >= ci.x && tx < ci.y) ? phix[tx] * phiy[ty] * ((u & 1) ? -1.f : 1.f) : 0.f;
-          str(obj + ((size_t)c * n + ty) * n + tx, x.x * ph);
-          if (z2 < nz) str(obj + ((size_t)z2 * n + ty) * n + tx, x.y * ph);
-        });
+  // compiled sizes: the first pass loads R and the last one stores the
+  // slices, rows outside [h + 1, h + n] being left out of the last pass.
+  // What bounds it is latency: one workgroup fills a CU's LDS, so its load,
+  // exchange and store phases do not overlap; the split exchange halves the
+  // LDS per column, which doubles the bytes in flight per phase and the width
+  // of the segments (n = 2048, us per chunk of 8 slices: 194 -> 147 at 2.5
+  // TB/s, n = 4096 1181 -> 533; float16 n = 2048 138 -> 117)
+  if constexpr (NS > 0) {
+    constexpr int LG = col_split(NS) ? split_lg(NS) : col_lg(NS);  // == lgCB
+    constexpr int H = NS / 4;
+    auto ld = [&](int a, int t) {
+      float2 x;
+      if (blocked)
+        x = tof2(blk[(a << LG) + t]);
+      else
+        x = tof2(src[(size_t)a * n + v0 + t]);
+      return (a & 1) ? make_float2(-x.x, -x.y) : x;
+    };
+    auto st = [&](int u, int t, float2 x) {
+      const int ty = u - 1 - H, tx = v0 + t;
+      const int2 ci = circ[ty];
+      const float ph =
+          (tx >= ci.x && tx < ci.y) ? phix[tx] * phiy[ty] * ((u & 1) ? -1.f : 1.f) : 0.f;
+      str(obj + ((size_t)c * n + ty) * n + tx, x.x * ph);
+      if (z2 < nz) str(obj + ((size_t)z2 * n + ty) * n + tx, x.y * ph);
+    };
+    if constexpr (col_split(NS))
+      fft_c_split<NS, 1, LG, H + 1, H + NS / 2 + 1>(reinterpret_cast<float *>(sm), fd.tw, tid, nt,
+                                                    ld, st);
+    else
+      fft_c_global<NS, 1, kFftEPT, LG, H + 1, H + NS / 2 + 1>(sm, fd.tw, tid, nt, ld, st);
   } else {
     stage_lds<16, cpx<T>>(
         CB * n2, tid, nt,
@@ -901,7 +916,7 @@ template <int NS>
 __global__ __launch_bounds__(1024) void k_fr_colfft_adj(const float *__restrict__ obj, float2 *__restrict__ R,
                                 const float *__restrict__ phix, const float *__restrict__ phiy,
                                 const int2 *__restrict__ circ, FftDesc fd, int n, int nz,
-                                int nzc, int lgCB) {
+                                int nzc, int lgCB, int blocked) {
   extern __shared__ float2 sm[];  // [a][t]: CB interleaved columns
   const int L = xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
   const int cb = L % gridDim.x, c = L / gridDim.x;
@@ -911,25 +926,28 @@ __global__ __launch_bounds__(1024) void k_fr_colfft_adj(const float *__restrict_
   const int n2 = 2 * n, v0 = cb * CB, h = n / 2;
   const int z2 = c + nzc;
   float2 *dst = R + (size_t)c * n2 * n;
+  float2 *blk = dst + (size_t)v0 * n2;  // block cb of the column-blocked layout
   if constexpr (NS > 0) {
     // compiled sizes: first pass from obj (rows outside [1+h, n+h] are
     // zero), last pass straight to R
-    constexpr int LG = col_lg(NS);
-    fft_c_global<NS, -1, kFftEPT, LG>(
-        sm, fd.tw, tid, nt,
-        [&](int u, int t) {
-          const int ty = u - 1 - h, tx = v0 + t;
-          if (ty < 0 || ty >= n || tx >= n) return make_float2(0.f, 0.f);
-          const int2 ci = circ[ty];
-          if (tx < ci.x || tx >= ci.y) return make_float2(0.f, 0.f);
-          const float ph = phix[tx] * phiy[ty] * ((u & 1) ? -1.f : 1.f);
-          return make_float2(obj[((size_t)c * n + ty) * n + tx] * ph,
-                             (z2 < nz) ? obj[((size_t)z2 * n + ty) * n + tx] * ph : 0.f);
-        },
-        [&](int a, int t, float2 x) {
-          if (v0 + t >= n) return;
-          dst[(size_t)a * n + v0 + t] = (a & 1) ? make_float2(-x.x, -x.y) : x;
-        });
+    constexpr int LG = col_split(NS) ? split_lg(NS) : col_lg(NS);
+    auto ld = [&](int u, int t) {
+      const int ty = u - 1 - h, tx = v0 + t;
+      if (ty < 0 || ty >= n || tx >= n) return make_float2(0.f, 0.f);
+      const int2 ci = circ[ty];
+      if (tx < ci.x || tx >= ci.y) return make_float2(0.f, 0.f);
+      const float ph = phix[tx] * phiy[ty] * ((u & 1) ? -1.f : 1.f);
+      return make_float2(obj[((size_t)c * n + ty) * n + tx] * ph,
+                         (z2 < nz) ? obj[((size_t)z2 * n + ty) * n + tx] * ph : 0.f);
+    };
+    auto st = [&](int a, int t, float2 x) {
+      (blocked ? blk[(a << LG) + t] : dst[(size_t)a * n + v0 + t]) =
+          (a & 1) ? make_float2(-x.x, -x.y) : x;
+    };
+    if constexpr (col_split(NS))
+      fft_c_split<NS, -1, LG, 0, NS>(reinterpret_cast<float *>(sm), fd.tw, tid, nt, ld, st);
+    else
+      fft_c_global<NS, -1, kFftEPT, LG>(sm, fd.tw, tid, nt, ld, st);
     return;
   }
   for (int idx = tid; idx < CB * n2; idx += nt) sm[idx] = make_float2(0.f, 0.f);
@@ -964,19 +982,26 @@ __global__ __launch_bounds__(1024) void k_fr_colfft_adj(const float *__restrict_
 
 template <int NS>
 __global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_rowfft_adj(const float2 *__restrict__ R, float2 *__restrict__ F, FftDesc fd,
-                                int n, int nzc) {
+                                int n, int nzc, int lgB) {
   extern __shared__ float2 sm[];
-  const int a = blockIdx.x, c = blockIdx.y;
+  const int L = lgB > 0 ? xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y)
+                        : blockIdx.x + gridDim.x * blockIdx.y;
+  const int a = L % gridDim.x, c = L / gridDim.x;
   if (c >= nzc) return;
   const int tid = threadIdx.x, nt = blockDim.x;
   const int n2 = 2 * n, h = n / 2;
   const float2 *src = R + ((size_t)c * n2 + a) * n;
+  const float2 *blk = R + (size_t)c * n2 * n + ((size_t)a << lgB);
   if constexpr (NS > 0) {
     float2 *dst = F + ((size_t)c * n2 + a) * n2;
     fft_c_global<NS, -1, kFftEPT, 0>(
         sm, fd.tw, tid, nt,
         [&](int v, int) {
-          const float2 x = (v >= h && v < h + n) ? src[v - h] : make_float2(0.f, 0.f);
+          const int o = v - h;
+          const float2 x =
+              (o < 0 || o >= n) ? make_float2(0.f, 0.f)
+              : lgB > 0 ? blk[((size_t)(o >> lgB) * n2 << lgB) + (o & ((1 << lgB) - 1))]
+                        : src[o];
           return (v & 1) ? make_float2(-x.x, -x.y) : x;
         },
         [&](int b, int, float2 x) { dst[b] = (b & 1) ? make_float2(-x.x, -x.y) : x; });
@@ -1506,9 +1531,12 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
   P->fpLds = (int)lds_bytes(P->nsPrep > 0, n2);
   P->nsCol = 0;
   if (st2) {
-    const int lgs = col_lg((int)n2);
-    const size_t lds_s = lds_bytes(true, n2) << lgs;
-    const int thr = fft_threads(P->fft2.rule, (int64_t)n2 << lgs, kFftEPT);
+    // (n is a multiple of the columns: 2^8 divides 2n)
+    const bool split = col_split((int)n2);
+    const int lgs = split ? split_lg((int)n2) : col_lg((int)n2);
+    const size_t lds_s = (lds_bytes(true, n2) << lgs) / (split ? 2 : 1);
+    const int thr =
+        fft_threads(P->fft2.rule, (int64_t)n2 << lgs, split ? kFftSplitEPT : kFftEPT);
     if (lds_s <= maxlds && thr > 0 && thr <= 1024) {
       P->nsCol = (int)n2;
       P->lgCB = lgs;
@@ -1532,10 +1560,24 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
               (long long)n);
     return fail(TOMO_EINVAL);
   }
-  // column-blocked R for 16-bit plans only: measured at n=2048 the column
-  // pass gains 40-50 us per chunk of 8 slices, the row pass loses 22 us
-  // (16-byte segments) in half precision and 43 us (32-byte) in float32
-  P->lgB = (dtype != TOMO_F32 && n % (1 << lg) == 0) ? lg : 0;
+  // R column-blocked (log2 of the block) or row-major, us per chunk of 8
+  // slices, row + column pass. The column pass gains contiguous reads, the
+  // row pass loses its long stores, so blocks pay where a workgroup's columns
+  // cover less than a 128-byte line of a row and the split column pass reads
+  // them: float32, 8 columns: 2n = 4096 164+147 against 149+174 row-major,
+  // 3840 199+165 against 183+195; 4 columns (32-byte segments): 5120 408+298
+  // against 314+367 and 6144 573+405 against 421+516, so row-major, except at
+  // 8192, where the 2^15-byte row stride puts a column into few memory
+  // channels: 782+533 against 729+1181. 16-bit, 4 or 8 columns: 2n = 2560
+  // 70+60 against 67+71, 4096 170+117 against 160+134, 5120 335+274 against
+  // 305+356, 8192 977+437 against 816+620; 16 columns (2048): 38+31 against
+  // 36+30, so row-major. Without a compiled column pass 16-bit R is blocked
+  // as before.
+  const bool pow2 = (n & (n - 1)) == 0;
+  if (P->nsCol > 0)
+    P->lgB = col_split((int)n2) && lg < 4 && (dtype != TOMO_F32 || lg == 3 || pow2) ? lg : 0;
+  else
+    P->lgB = (dtype != TOMO_F32 && n % (1 << lg) == 0) ? lg : 0;
   hipError_t ea = hipSuccess;
   auto lds_attr = [&](const void *k, size_t bytes) {
     if (ea == hipSuccess)
@@ -1979,7 +2021,7 @@ extern "C" int fr_forward(tomo_fr_plan *P, void *data_, const void *obj_, void *
                          dim3(P->colThreads), P->colLds, st, obj,
                          P->R.as<float2>(),
                          P->phix.as<float>(), P->phiy.as<float>(), P->circ.as<int2>(),
-                         P->fft2.d, n, nz, nzc, P->lgCB);
+                         P->fft2.d, n, nz, nzc, P->lgCB, P->lgB > 0 ? 1 : 0);
     });
   }
   TOMO_LAUNCH_CHECK();
@@ -1988,7 +2030,7 @@ extern "C" int fr_forward(tomo_fr_plan *P, void *data_, const void *obj_, void *
     with_static_size(P->nsRow, [&](auto ns) {
       hipLaunchKernelGGL(k_fr_rowfft_adj<decltype(ns)::value>, dim3(n2, ng * 4),
                          dim3(P->rowThreads), P->rowLds,
-                         st, P->R.as<float2>(), P->F.as<float2>(), P->fft2.d, n, nzc);
+                         st, P->R.as<float2>(), P->F.as<float2>(), P->fft2.d, n, nzc, P->lgB);
     });
   }
   TOMO_LAUNCH_CHECK();
