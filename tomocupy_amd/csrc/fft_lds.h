@@ -967,6 +967,49 @@ __device__ __forceinline__ void split_rest(float2 *v, float *buf, const float2 *
   }
 }
 
+// The passes S .. of a transform whose values stay in registers (v: the inputs
+// of pass S, then the outputs of the last pass in its order).
+template <int N, int DIR, int LGH, int S, int Ns>
+__device__ __forceinline__ void split_regs(float2 *v, float *buf, const float2 *__restrict__ tw,
+                                           int tid, int nt) {
+  using SP = SplitPlan<N>;
+  constexpr int R = SP::radix(S);
+  // (a pass computes its own addresses: kept from one for the next, they and
+  // the 64 registers of v would not fit 128)
+  asm volatile("" : "+v"(tid));
+  split_butterflies<R, Ns, N, DIR, LGH>(v, tw, tid, nt);
+  if constexpr (S + 1 < SP::passes) {
+    __syncthreads();  // the last exchange's reads, of this transform or the one before
+    split_exchange<R, Ns, SP::radix(S + 1), N, LGH>(v, buf, tid, nt);
+    split_regs<N, DIR, LGH, S + 1, Ns * R>(v, buf, tw, tid, nt);
+  }
+}
+
+// Threads of fft_split_regs: every one holds kFftSplitEPT values.
+constexpr int split_threads(int N, int LGH) { return (N << LGH) / kFftSplitEPT; }
+
+// Transform of 2^LGH interleaved sequences of a power of two length N in
+// registers, thread tid of split_threads(N, LGH) holding elements
+// (tid >> LGH) + s N / 32 of sequence tid mod 2^LGH in a[s], before and after.
+// buf: lds_padded_len(N) << LGH floats (a barrier precedes its first use).
+template <int N, int DIR, int LGH>
+__device__ __forceinline__ void fft_split_regs(float2 *a, float *buf,
+                                               const float2 *__restrict__ tw, int tid) {
+  using SP = SplitPlan<N>;
+  static_assert((N & (N - 1)) == 0, "every butterfly of every pass has a thread");
+  constexpr int E = kFftSplitEPT, R0 = SP::radix(0), RL = SP::radix(SP::passes - 1);
+  float2 v[E];
+#pragma unroll
+  for (int q = 0; q < E / R0; ++q)
+#pragma unroll
+    for (int r = 0; r < R0; ++r) v[q * R0 + r] = a[q + r * (E / R0)];
+  split_regs<N, DIR, LGH, 0, 1>(v, buf, tw, tid, split_threads(N, LGH));
+#pragma unroll
+  for (int q = 0; q < E / RL; ++q)
+#pragma unroll
+    for (int r = 0; r < RL; ++r) a[q + r * (E / RL)] = v[q * RL + out_slot<RL>(r)];
+}
+
 // buf: lds_padded_len(N) << LGH floats.
 template <int N, int DIR, int LGH, int LO, int HI, typename Ld, typename St>
 __device__ __forceinline__ void fft_c_split(float *buf, const float2 *__restrict__ tw, int tid,

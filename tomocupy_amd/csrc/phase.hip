@@ -13,15 +13,22 @@
 // u, v the reference's reciprocal coordinates (k - (N-1)/2) / ((N-1) ps),
 // half a sample off zero for even N.
 //
+// H is real but not even (half a sample off zero), and the projection is real,
+// so Re ifft2(F H) = ifft2(F He) with the even part He(k) = (H(k) + H(-k)) / 2:
+// F He is Hermitian, and half of its columns hold it all.
+//
 // Three kernels per batch of projections, through a complex work buffer of
-// the dy real rows' spectra (the py padded rows above and below a projection
-// are copies of its first and last rows, so their row spectra are those
-// rows' spectra): rows (two real rows packed into one complex FFT, split into
-// their two spectra), columns (the padded column rebuilt from the edge
-// spectra, forward FFT, filter, inverse FFT scaled by 1/(Ny Nx), the dy rows
-// the crop keeps written back), and inverse rows (the Hermitian parts of two
-// row spectra packed into one inverse FFT, whose real and imaginary parts
-// are the two real rows).  The
+// the left half of the dy real rows' spectra (the py padded rows above and
+// below a projection are copies of its first and last rows, so their row
+// spectra are those rows' spectra): rows (two real rows packed into one complex
+// FFT, split into their two half spectra), columns (the padded column rebuilt
+// from the edge spectra, forward FFT, filter He / max H / (Ny Nx), inverse FFT,
+// the dy rows the crop keeps written back), and inverse rows (two half spectra
+// extended and packed into one inverse FFT, whose real and imaginary parts are
+// the two real rows).  The columns 0 and Nx / 2 of a real row's spectrum are
+// real, so column 0 of the buffer holds both, as its real and imaginary parts.
+// The buffer is blocked by 2^lgB columns, F[projection][block][row][column]: two
+// rows of a block are adjacent.  The
 // FFTs are the LDS Stockham transforms of fft_lds.h; the filter is evaluated
 // in float32 (the reference's precision) from 1-D tables built in FP64.
 #include <algorithm>
@@ -38,13 +45,17 @@ struct tomo_ph_plan {
   int64_t dy = 0, dz = 0, batch = 0;
   int method = 0;
   int py = 0, pz = 0, Ny = 0, Nx = 0;
-  int lgC = 0;  // log2 of the columns per workgroup of the column pass
+  int lgC = 0;     // log2 of the columns per workgroup of the column pass
+  int lgB = 0;     // log2 of the columns per block of F
+  size_t Fb = 0;   // elements of F per projection
+  float cHi = 0.f, cLo = 0.f;  // 1 / (2 max H Ny Nx) as an unrounded sum
   float A = 0.f, B = 0.f, alpha = 0.f, db = 0.f, hmax = 1.f;
   int rowThreads = 0, colThreads = 0;
   size_t rowLds = 0, colLds = 0;
   FftPlan fy, fx;
   DevBuf ty, tx;  // fftshifted 1-D terms of the filter (rows, columns)
-  DevBuf F;       // (batch, dy, Nx) float2: spectra of the real rows
+  DevBuf h0;      // float2 per padded row: the filter of column 0 (k_ph_col0)
+  DevBuf F;       // (batch, Nx/2 >> lgB, dy, 2^lgB) float2: half spectra of the real rows
 };
 
 namespace {
@@ -68,31 +79,23 @@ void with_ph_size(int N, F &&f) {
   }
 }
 
-// log2 of the columns of a column-pass workgroup: at most 8 columns and 8192
-// elements (64 KB of LDS)
-constexpr int ph_lg(int N) {
-  int lg = 0;
-  while (lg < 3 && (N << (lg + 1)) <= 8192) ++lg;
-  return lg;
-}
+// log2 of the columns of a column-pass workgroup: compiled lengths, as many as
+// 512 threads hold in registers, so that two workgroups share a CU and one's
+// loads run under the other's butterflies; run-time lengths, 8
+constexpr int ph_lg(int N) { return N > 0 ? split_lg(N) - (N > 1024) : 3; }
+// log2 of the columns of a block of the work buffer: 8 or a workgroup's, so
+// that the row passes store and load 128-byte segments (8 columns of 2 rows)
+constexpr int ph_lgb(int N) { return ph_lg(N) > 3 ? ph_lg(N) : 3; }
 
-// the transform of 2^LG (compiled) or 2^lg (run-time) sequences in LDS
-template <int NS, int DIR, int LG>
-__device__ __forceinline__ void ph_fft(float2 *sm, const FftDesc &fd, int lg, int tid, int nt) {
-  if constexpr (NS > 0)
-    lds_fft_c<NS, DIR, kFftEPT, LG>(sm, fd.tw, tid, nt);
-  else
-    lds_fft<DIR>(sm, fd, lg, tid, nt);
-}
-
-// the method's factor at one grid point, from the sum of the two 1-D terms
-__device__ __forceinline__ float ph_factor(int method, float s, float A, float B, float alpha,
-                                           float db) {
-  if (method == 0) return 1.f / (A * s + alpha);             // paganin
-  if (method == 1) return 1.f / (1.f - B * (s - 2.f));       // Gpaganin
-  float sn, cs;                                              // farago
+// the reciprocal of the method's factor at one grid point, from the sum of the
+// two 1-D terms
+__device__ __forceinline__ float ph_denom(int method, float s, float A, float B, float alpha,
+                                          float db) {
+  if (method == 0) return A * s + alpha;             // paganin
+  if (method == 1) return 1.f - B * (s - 2.f);       // Gpaganin
+  float sn, cs;                                      // farago
   sincosf(A * s, &sn, &cs);
-  return 1.f / (cs + db * sn);
+  return cs + db * sn;
 }
 
 // row maxima of the factor over the grid (the normalisation max H)
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(256) void k_ph_fmax(const float *__restrict__ ty,
   const int ky = blockIdx.x;
   float m = -INFINITY;
   for (int kx = threadIdx.x; kx < Nx; kx += 256)
-    m = fmaxf(m, ph_factor(method, ty[ky] + tx[kx], A, B, alpha, db));
+    m = fmaxf(m, 1.f / ph_denom(method, ty[ky] + tx[kx], A, B, alpha, db));
   red[threadIdx.x] = m;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
@@ -114,13 +117,46 @@ __global__ __launch_bounds__(256) void k_ph_fmax(const float *__restrict__ ty,
   if (threadIdx.x == 0) rowmax[ky] = red[0];
 }
 
+// 1 / d for a normal d: the hardware's reciprocal (1 ulp) and one Newton step,
+// whose single rounding leaves it correctly rounded but next to a tie.  A
+// division takes three times the instructions.
+__device__ __forceinline__ float ph_rcp(float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  return fmaf(r, fmaf(-d, r, 1.f), r);
+}
+
+// The even part of the factor, times 2 (c_hi + c_lo).
+__device__ __forceinline__ float ph_even(int method, float s0, float s1, float A, float B,
+                                         float alpha, float db, float c_hi, float c_lo) {
+  const float h = ph_rcp(ph_denom(method, s0, A, B, alpha, db)) +
+                  ph_rcp(ph_denom(method, s1, A, B, alpha, db));
+  return fmaf(h, c_hi, h * c_lo);
+}
+
+// Column 0 of the work buffer is P = A + i B with A column 0 and B column
+// Nx / 2 of a real image's spectrum: times their even, real factors hA and hB
+// that is P[k] (hA + hB) / 2 + conj(P[-k]) (hA - hB) / 2.
+__global__ __launch_bounds__(256) void k_ph_col0(const float *__restrict__ ty,
+                                                 const float *__restrict__ tx, int Ny, int Nx,
+                                                 int method, float A, float B, float alpha,
+                                                 float db, float c_hi, float c_lo,
+                                                 float2 *__restrict__ h0) {
+  const int ky = blockIdx.x * 256 + threadIdx.x;
+  if (ky >= Ny) return;
+  const float t0 = ty[ky], t1 = ty[ky == 0 ? 0 : Ny - ky];
+  const float a = ph_even(method, t0 + tx[0], t1 + tx[0], A, B, alpha, db, c_hi, c_lo);
+  const float x = tx[Nx / 2];
+  const float b = ph_even(method, t0 + x, t1 + x, A, B, alpha, db, c_hi, c_lo);
+  h0[ky] = make_float2(0.5f * (a + b), 0.5f * (a - b));
+}
+
 // Forward FFTs of the column-padded real rows 2 pr and 2 pr + 1 of
 // projection blockIdx.y: z = row0 + i row1, Z = fft(z);
-// X0 = (Z[k] + conj Z[-k]) / 2, X1 = (Z[k] - conj Z[-k]) / (2i).
+// X0 = (Z[k] + conj Z[-k]) / 2, X1 = (Z[k] - conj Z[-k]) / (2i), k < Nx / 2.
 template <int NS>
 __global__ __launch_bounds__(512) void k_ph_rows_fwd(const float *__restrict__ data,
                                                       float2 *__restrict__ F, FftDesc fd, int dy,
-                                                      int dz, int pz) {
+                                                      int dz, int pz, int lgB, size_t Fb) {
   extern __shared__ float2 sm[];
   const int pr = blockIdx.x, b = blockIdx.y;
   const int tid = threadIdx.x, nt = blockDim.x;
@@ -129,92 +165,187 @@ __global__ __launch_bounds__(512) void k_ph_rows_fwd(const float *__restrict__ d
   const float *img = data + (size_t)b * dy * dz;
   const float *r0 = img + (size_t)iy0 * dz;
   const float *r1 = r0 + dz;
-  for (int ix = tid; ix < Nx; ix += nt) {
+  auto ld = [&](int ix, int) {
     const int sx = min(max(ix - pz, 0), dz - 1);
-    sm[lidx<NS>(ix)] = make_float2(r0[sx], r1[sx]);
+    return make_float2(r0[sx], r1[sx]);
+  };
+  if constexpr (NS > 0) {
+    fft_c_from_global<NS, -1, kFftEPT, 0>(sm, fd.tw, tid, nt, ld);
+  } else {
+    for (int ix = tid; ix < Nx; ix += nt) sm[ix] = ld(ix, 0);
+    __syncthreads();
+    lds_fft<-1>(sm, fd, 0, tid, nt);
   }
-  __syncthreads();
-  ph_fft<NS, -1, 0>(sm, fd, 0, tid, nt);
-  float2 *f0 = F + ((size_t)b * dy + iy0) * Nx;
-  float2 *f1 = f0 + Nx;
-  for (int k = tid; k < Nx; k += nt) {
-    const float2 zk = sm[lidx<NS>(k)], zm = cconj(sm[lidx<NS>(k == 0 ? 0 : Nx - k)]);
-    f0[k] = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y + zm.y));
-    f1[k] = make_float2(0.5f * (zk.y - zm.y), -0.5f * (zk.x - zm.x));
+  // (a block's columns of the first row, then of the second, then the next
+  // block's: 16 << lgB contiguous bytes)
+  float2 *f = F + (size_t)b * Fb + ((size_t)iy0 << lgB);
+  for (int e = tid; e < max(Nx, 2 << lgB); e += nt) {
+    const int c = e & ((1 << lgB) - 1), blk = e >> (lgB + 1), row = (e >> lgB) & 1;
+    const int k = (blk << lgB) + c;
+    if (2 * k >= Nx) continue;  // (Nx / 2 may be less than a block)
+    float2 x;
+    if (k == 0) {
+      const float2 z0 = sm[0], zn = sm[lidx<NS>(Nx / 2)];
+      x = row ? make_float2(z0.y, zn.y) : make_float2(z0.x, zn.x);
+    } else {
+      const float2 zk = sm[lidx<NS>(k)], zm = cconj(sm[lidx<NS>(Nx - k)]);
+      x = row ? make_float2(0.5f * (zk.y - zm.y), -0.5f * (zk.x - zm.x))
+              : make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y + zm.y));
+    }
+    f[(((size_t)blk * dy + row) << lgB) + c] = x;
   }
 }
 
-// Column pass over 2^lgC adjacent columns of projection blockIdx.y: the
-// padded column (padded row ky holds real row clamp(ky - py, 0, dy - 1)),
-// forward FFT, times H / max H / (Ny Nx), inverse FFT; rows py .. py+dy-1
-// written back in place.
+// Column pass over 2^lgC columns of a projection: the padded column (padded row ky holds real row clamp(ky - py, 0, dy - 1)),
+// forward FFT, times He / max H / (Ny Nx), inverse FFT; rows py .. py+dy-1
+// written back in place.  Compiled lengths keep a column's values in registers
+// from the load to the store; what bounds them is vector arithmetic (two
+// transforms and the factor).  Measured for 4 projections of 2048 x 2048
+// (padded 4096 x 4096): 164 us with two workgroups of 4 columns per CU, 195
+// with one of 8 columns (and divisions for the factor); 443 for all 4096
+// columns through LDS passes.  The row passes, half a spectrum each, 52 and 46
+// us, were 90 and 90.
 template <int NS>
-__global__ __launch_bounds__(512) void k_ph_cols(float2 *__restrict__ F, FftDesc fd,
-                                                  int lgC, int Nx, int dy, int py,
-                                                  const float *__restrict__ ty,
-                                                  const float *__restrict__ tx, int method,
-                                                  float A, float B, float alpha, float db,
-                                                  float hmax, float scale) {
+__global__ __launch_bounds__(1024) void k_ph_cols(float2 *__restrict__ F, FftDesc fd, int lgC,
+                                                   int Nx, int dy, int py,
+                                                   const float *__restrict__ ty,
+                                                   const float *__restrict__ tx,
+                                                   const float2 *__restrict__ h0, int method,
+                                                   float A, float B, float alpha, float db,
+                                                   float c_hi, float c_lo, size_t Fb) {
   extern __shared__ float2 sm[];
   const int tid = threadIdx.x, nt = blockDim.x;
+  const int lgB = ph_lgb(NS);
   if (NS > 0) lgC = ph_lg(NS);
   const int Ny = NS > 0 ? NS : fd.N, C = 1 << lgC;
-  // workgroups are dealt to the 8 XCDs in turn: give each XCD a contiguous
-  // range of column groups, so that the groups sharing cache lines (2^lgC
-  // columns = 8 << lgC bytes of each row) share its L2
-  const int G = gridDim.x;
-  const int g = (G % 8 == 0) ? (blockIdx.x % 8) * (G / 8) + blockIdx.x / 8 : blockIdx.x;
-  const int kx0 = g << lgC, b = blockIdx.y;
-  float2 *fb = F + (size_t)b * dy * Nx + kx0;
-  for (int e = tid; e < (Ny << lgC); e += nt) {
-    const int ky = e >> lgC, c = e & (C - 1);
-    sm[(lidx<NS>(ky) << lgC) + c] = fb[(size_t)min(max(ky - py, 0), dy - 1) * Nx + c];
-  }
-  __syncthreads();
-  ph_fft<NS, -1, ph_lg(NS)>(sm, fd, lgC, tid, nt);
-  for (int e = tid; e < (Ny << lgC); e += nt) {
-    const int ky = e >> lgC, c = e & (C - 1);
-    const float h = ph_factor(method, ty[ky] + tx[kx0 + c], A, B, alpha, db) / hmax * scale;
-    float2 &v = sm[(lidx<NS>(ky) << lgC) + c];
-    v = make_float2(v.x * h, v.y * h);
-  }
-  __syncthreads();
-  ph_fft<NS, 1, ph_lg(NS)>(sm, fd, lgC, tid, nt);
-  for (int e = tid; e < (dy << lgC); e += nt) {
-    const int y = e >> lgC, c = e & (C - 1);
-    fb[(size_t)y * Nx + c] = sm[(lidx<NS>(y + py) << lgC) + c];
+  // workgroups of one block of the work buffer go to the same XCD
+  const int L = xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+  const int kx0 = (L % gridDim.x) << lgC, b = L / gridDim.x;
+  float2 *fb = F + (size_t)b * Fb + (((size_t)(kx0 >> lgB) * dy) << lgB) + (kx0 & ((1 << lgB) - 1));
+  auto row = [&](int ky) { return min(max(ky - py, 0), dy - 1); };
+  if constexpr (NS > 0) {
+    // Values stay in registers from the load to the store.
+    constexpr int LG = ph_lg(NS), E = kFftSplitEPT, T = split_threads(NS, LG), U = NS / E;
+    float *buf = reinterpret_cast<float *>(sm);
+    const int t = tid & (C - 1), kx = kx0 + t;
+    int j = tid >> LG;
+    const bool live = 2 * kx < Nx;  // (Nx / 2 may be less than a block)
+    // (32-bit offsets: a thread's 32 addresses would not fit its registers)
+    auto at = [&](int y, int c) {
+      return reinterpret_cast<float2 *>(reinterpret_cast<char *>(fb) +
+                                        ((unsigned)((y << lgB) + c) * 8u));
+    };
+    float2 a[E];
+#pragma unroll
+    for (int s = 0; s < E; ++s) a[s] = *at(row(j + s * U), live ? t : 0);
+    asm volatile("" : "+v"(j));  // recompute what hangs on j: held, it would spill
+    fft_split_regs<NS, -1, LG>(a, buf, fd.tw, tid);
+    // the factors in a rolled loop (one copy of the method's code), through
+    // the thread's own LDS words
+    __syncthreads();
+    const float x0 = tx[live ? kx : 0], x1 = tx[live && kx > 0 ? Nx - kx : 0];
+#pragma unroll 2
+    for (int s = 0; s < E; ++s) {
+      const int ky = j + s * U;
+      const float h = ph_even(method, ty[ky] + x0, ty[ky == 0 ? 0 : NS - ky] + x1, A, B, alpha,
+                              db, c_hi, c_lo);
+      buf[s * T + tid] = kx == 0 ? 1.f : h;
+    }
+#pragma unroll
+    for (int s = 0; s < E; ++s) {
+      const float h = buf[s * T + tid];
+      a[s] = make_float2(a[s].x * h, a[s].y * h);
+    }
+    if (kx0 == 0) {  // column 0 is two
+      __syncthreads();
+      if (t == 0) {
+#pragma unroll
+        for (int s = 0; s < E; ++s) sm[j + s * U] = a[s];
+      }
+      __syncthreads();
+      if (t == 0) {
+#pragma unroll
+        for (int s = 0; s < E; ++s) {
+          const int ky = j + s * U;
+          const float2 m = sm[ky == 0 ? 0 : NS - ky], h = h0[ky];
+          a[s] = make_float2(a[s].x * h.x + m.x * h.y, a[s].y * h.x - m.y * h.y);
+        }
+      }
+    }
+    fft_split_regs<NS, 1, LG>(a, buf, fd.tw, tid);
+    asm volatile("" : "+v"(j));
+#pragma unroll
+    for (int s = 0; s < E; ++s) {
+      const int y = j + s * U - py;
+      if (live && y >= 0 && y < dy) *at(y, t) = a[s];
+    }
+  } else {
+    for (int e = tid; e < (Ny << lgC); e += nt) {
+      const int ky = e >> lgC, c = e & (C - 1);
+      sm[e] = 2 * (kx0 + c) < Nx ? fb[((size_t)row(ky) << lgB) + c] : make_float2(0.f, 0.f);
+    }
+    __syncthreads();
+    lds_fft<-1>(sm, fd, lgC, tid, nt);
+    for (int e = tid; e < (Ny << lgC); e += nt) {
+      const int ky = e >> lgC, c = e & (C - 1), kx = kx0 + c, km = ky == 0 ? 0 : Ny - ky;
+      if (2 * kx >= Nx) continue;
+      const float2 v = sm[e];
+      if (kx > 0) {
+        const float h = ph_even(method, ty[ky] + tx[kx], ty[km] + tx[Nx - kx], A, B, alpha, db,
+                                c_hi, c_lo);
+        sm[e] = make_float2(v.x * h, v.y * h);
+      } else if (2 * ky <= Ny) {  // this thread does rows ky and -ky
+        const float2 m = sm[km << lgC], h = h0[ky], hm = h0[km];
+        sm[e] = make_float2(v.x * h.x + m.x * h.y, v.y * h.x - m.y * h.y);
+        if (km != ky)
+          sm[km << lgC] = make_float2(m.x * hm.x + v.x * hm.y, m.y * hm.x - v.y * hm.y);
+      }
+    }
+    __syncthreads();
+    lds_fft<1>(sm, fd, lgC, tid, nt);
+    for (int e = tid; e < (dy << lgC); e += nt) {
+      const int y = e >> lgC, c = e & (C - 1);
+      if (2 * (kx0 + c) < Nx) fb[((size_t)y << lgB) + c] = sm[((y + py) << lgC) + c];
+    }
   }
 }
 
-// Inverse row FFTs for output rows 2 pr and 2 pr + 1:
-// Re ifft(G) = ifft(Herm G), Herm G[k] = (G[k] + conj G[-k]) / 2, so
-// ifft(Herm G0 + i Herm G1) = Re ifft(G0) + i Re ifft(G1); cropped columns
-// written back to the projection.
+// Inverse row FFTs for output rows 2 pr and 2 pr + 1 from their half spectra
+// G0, G1: z[k] = G0[k] + i G1[k], z[-k] = conj G0[k] + i conj G1[k]; cropped
+// columns written back to the projection.
 template <int NS>
 __global__ __launch_bounds__(512) void k_ph_rows_inv(float *__restrict__ data,
                                                       const float2 *__restrict__ F, FftDesc fd,
-                                                      int dy, int dz, int pz) {
+                                                      int dy, int dz, int pz, int lgB, size_t Fb) {
   extern __shared__ float2 sm[];
   const int pr = blockIdx.x, b = blockIdx.y;
   const int tid = threadIdx.x, nt = blockDim.x;
   const int Nx = NS > 0 ? NS : fd.N;
   const int oy0 = 2 * pr, oy1 = oy0 + 1;  // dy is even: both rows exist
-  const float2 *g0 = F + ((size_t)b * dy + oy0) * Nx;
-  const float2 *g1 = g0 + Nx;
-  for (int k = tid; k < Nx; k += nt) {
-    const int km = k == 0 ? 0 : Nx - k;
-    const float2 a = g0[k], am = g0[km], c = g1[k], cm = g1[km];
-    const float2 h0 = make_float2(0.5f * (a.x + am.x), 0.5f * (a.y - am.y));
-    const float2 h1 = make_float2(0.5f * (c.x + cm.x), 0.5f * (c.y - cm.y));
-    sm[lidx<NS>(k)] = make_float2(h0.x - h1.y, h0.y + h1.x);
+  const float2 *g = F + (size_t)b * Fb + ((size_t)oy0 << lgB);
+  for (int k = tid; 2 * k < Nx; k += nt) {
+    const float2 *gk = g + (((size_t)(k >> lgB) * dy) << lgB) + (k & ((1 << lgB) - 1));
+    const float2 x0 = gk[0], x1 = gk[1 << lgB];
+    sm[lidx<NS>(k)] = k == 0 ? make_float2(x0.x, x1.x) : make_float2(x0.x - x1.y, x0.y + x1.x);
+    sm[lidx<NS>(k == 0 ? Nx / 2 : Nx - k)] =
+        k == 0 ? make_float2(x0.y, x1.y) : make_float2(x0.x + x1.y, x1.x - x0.y);
   }
   __syncthreads();
-  ph_fft<NS, 1, 0>(sm, fd, 0, tid, nt);
   float *img = data + (size_t)b * dy * dz;
-  for (int x = tid; x < dz; x += nt) {
-    const float2 v = sm[lidx<NS>(pz + x)];
+  auto st = [&](int o, int, float2 v) {
+    const int x = o - pz;
+    if (x < 0 || x >= dz) return;
     img[(size_t)oy0 * dz + x] = v.x;
-    if (oy1 < dy) img[(size_t)oy1 * dz + x] = v.y;
+    img[(size_t)oy1 * dz + x] = v.y;
+  };
+  if constexpr (NS > 0) {
+    using SP = StaticPlan<NS>;
+    constexpr int RL = SP::radix(SP::passes - 1);
+    lds_fft_c<NS, 1, kFftEPT, 0, 0, 1, SP::passes - 1>(sm, fd.tw, tid, nt);
+    fft_pass_c_last<RL, NS / RL, NS, 1, kFftEPT, 0>(sm, fd.tw, tid, nt, st);
+  } else {
+    lds_fft<1>(sm, fd, 0, tid, nt);
+    for (int o = tid; o < Nx; o += nt) st(o, 0, sm[o]);
   }
 }
 
@@ -234,6 +365,7 @@ extern "C" void ph_destroy(tomo_ph_plan *P) {
   P->fx.release();
   P->ty.release();
   P->tx.release();
+  P->h0.release();
   P->F.release();
   delete P;
 }
@@ -302,7 +434,14 @@ extern "C" int ph_create(tomo_ph_plan **plan, int64_t dy, int64_t dz, int64_t ba
   if (!rc) rc = P->fx.init(P->Nx);
   if (!rc) rc = P->ty.alloc(sizeof(float) * P->Ny);
   if (!rc) rc = P->tx.alloc(sizeof(float) * P->Nx);
-  if (!rc) rc = P->F.alloc(sizeof(float2) * (size_t)batch * dy * P->Nx);
+  // columns per block of the work buffer; one block at least
+  with_ph_size(P->Ny, [&](auto ns) {
+    P->lgC = ph_lg(decltype(ns)::value);
+    P->lgB = ph_lgb(decltype(ns)::value);
+  });
+  P->Fb = (size_t)std::max(P->Nx / 2, 1 << P->lgB) * dy;
+  if (!rc) rc = P->h0.alloc(sizeof(float2) * P->Ny);
+  if (!rc) rc = P->F.alloc(sizeof(float2) * (size_t)batch * P->Fb);
   if (rc) {
     ph_destroy(P);
     return rc;
@@ -336,10 +475,21 @@ extern "C" int ph_create(tomo_ph_plan **plan, int64_t dy, int64_t dz, int64_t ba
       return TOMO_EINVAL;
     }
   }
+  const double cs = 0.5 / ((double)P->hmax * P->Ny * P->Nx);
+  P->cHi = (float)cs;
+  P->cLo = (float)(cs - (double)P->cHi);
+  hipLaunchKernelGGL(k_ph_col0, dim3((unsigned)((P->Ny + 255) / 256)), dim3(256), 0, 0,
+                     P->ty.as<float>(), P->tx.as<float>(), P->Ny, P->Nx, method, P->A, P->B,
+                     P->alpha, P->db, P->cHi, P->cLo, P->h0.as<float2>());
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipStreamSynchronize(0);
+  if (e != hipSuccess) {
+    set_error("ph_create: %s", hipGetErrorString(e));
+    ph_destroy(P);
+    return TOMO_EHIP;
+  }
   // launch shapes: rows one transform per workgroup, columns 2^lgC interleaved
   // transforms
-  P->lgC = ph_lg(P->Ny);
-  hipError_t e = hipSuccess;
   auto lds_attr = [&](const void *k, size_t bytes) {
     if (e == hipSuccess)
       e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
@@ -353,13 +503,13 @@ extern "C" int ph_create(tomo_ph_plan **plan, int64_t dy, int64_t dz, int64_t ba
   });
   with_ph_size(P->Ny, [&](auto ns) {
     constexpr int NS = decltype(ns)::value;
-    P->colThreads = NS > 0 ? fft_threads(P->fy.rule, (int64_t)NS << P->lgC)
-                           : fft_rt_threads(P->fy.d, P->lgC);
-    P->colLds = sizeof(float2) * ((size_t)(NS > 0 ? lds_padded_len(NS) : P->Ny) << P->lgC);
+    P->colThreads = NS > 0 ? split_threads(NS, P->lgC) : fft_rt_threads(P->fy.d, P->lgC);
+    P->colLds = NS > 0 ? sizeof(float) * ((size_t)lds_padded_len(NS) << P->lgC)
+                       : sizeof(float2) * ((size_t)P->Ny << P->lgC);
     lds_attr((const void *)k_ph_cols<NS>, P->colLds);
   });
   if (P->rowThreads <= 0 || P->rowThreads > 512 || P->colThreads <= 0 ||
-      P->colThreads > 512 || P->rowLds > max_lds_per_block() ||
+      P->colThreads > 1024 || P->rowLds > max_lds_per_block() ||
       P->colLds > max_lds_per_block()) {
     set_error("ph_create: padded size %d x %d too large for one workgroup", P->Ny, P->Nx);
     ph_destroy(P);
@@ -391,7 +541,6 @@ extern "C" int ph_apply(tomo_ph_plan *P, float *data, int64_t nproj, void *strea
   TOMO_REQUIRE(nproj >= 0, "ph_apply: nproj < 0");
   hipStream_t st = (hipStream_t)stream;
   const int dy = (int)P->dy, dz = (int)P->dz;
-  const float scale = 1.f / ((float)P->Ny * (float)P->Nx);
   for (int64_t b0 = 0; b0 < nproj; b0 += P->batch) {
     const unsigned nb = (unsigned)std::min<int64_t>(P->batch, nproj - b0);
     float *img = data + (size_t)b0 * dy * dz;
@@ -400,17 +549,18 @@ extern "C" int ph_apply(tomo_ph_plan *P, float *data, int64_t nproj, void *strea
       with_ph_size(P->Nx, [&](auto ns) {
         hipLaunchKernelGGL(k_ph_rows_fwd<decltype(ns)::value>, dim3((unsigned)(dy / 2), nb),
                            dim3(P->rowThreads), P->rowLds, st, img, P->F.as<float2>(), P->fx.d,
-                           dy, dz, P->pz);
+                           dy, dz, P->pz, P->lgB, P->Fb);
       });
     }
     TOMO_LAUNCH_CHECK();
     {
       ProfScope ps_("k_ph_cols", st);
       with_ph_size(P->Ny, [&](auto ns) {
-        hipLaunchKernelGGL(k_ph_cols<decltype(ns)::value>, dim3((unsigned)(P->Nx >> P->lgC), nb),
+        hipLaunchKernelGGL(k_ph_cols<decltype(ns)::value>, dim3((unsigned)std::max(P->Nx / 2 >> P->lgC, 1), nb),
                            dim3(P->colThreads), P->colLds, st, P->F.as<float2>(), P->fy.d,
                            P->lgC, P->Nx, dy, P->py, P->ty.as<float>(), P->tx.as<float>(),
-                           P->method, P->A, P->B, P->alpha, P->db, P->hmax, scale);
+                           P->h0.as<float2>(), P->method, P->A, P->B, P->alpha, P->db, P->cHi,
+                           P->cLo, P->Fb);
       });
     }
     TOMO_LAUNCH_CHECK();
@@ -419,7 +569,7 @@ extern "C" int ph_apply(tomo_ph_plan *P, float *data, int64_t nproj, void *strea
       with_ph_size(P->Nx, [&](auto ns) {
         hipLaunchKernelGGL(k_ph_rows_inv<decltype(ns)::value>, dim3((unsigned)(dy / 2), nb),
                            dim3(P->rowThreads), P->rowLds, st, img, P->F.as<float2>(), P->fx.d,
-                           dy, dz, P->pz);
+                           dy, dz, P->pz, P->lgB, P->Fb);
       });
     }
     TOMO_LAUNCH_CHECK();
