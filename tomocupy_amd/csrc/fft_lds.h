@@ -684,7 +684,8 @@ struct StaticPlan {
   }
 };
 
-template <int R, int Ns, int N, int DIR, int EPT, int LGH>
+// (ODD: of the transform at odd frequencies, see chain_first)
+template <int R, int Ns, int N, int DIR, int EPT, int LGH, bool ODD = false>
 __device__ __forceinline__ void fft_pass_c(float2 *buf, const float2 *__restrict__ tw, int tid,
                                            int nt) {
   constexpr int MAXB = EPT / R;
@@ -705,7 +706,8 @@ __device__ __forceinline__ void fft_pass_c(float2 *buf, const float2 *__restrict
       const int base = (lds_pad(j) << LGH) + t;
 #pragma unroll
       for (int r = 0; r < R; ++r) v[q][r] = buf[base + r * rstride];
-      if constexpr (Ns > 1) twiddle<R, DIR>(v[q], tw, (unsigned)((j % Ns) * twstep));
+      if constexpr (Ns > 1)
+        twiddle<R, DIR>(v[q], tw, (unsigned)((ODD ? 2 * (j % Ns) + 1 : j % Ns) * twstep));
       butterfly<R, DIR>(v[q]);
     }
   }
@@ -731,13 +733,13 @@ __device__ __forceinline__ void fft_pass_c(float2 *buf, const float2 *__restrict
 // and the function ends with a barrier.
 // Passes S .. SEnd-1 only (Ns: the sub-transform length entering pass S).
 template <int N, int DIR, int EPT, int LGH, int S = 0, int Ns = 1,
-          int SEnd = StaticPlan<N>::passes>
+          int SEnd = StaticPlan<N>::passes, bool ODD = false>
 __device__ __forceinline__ void lds_fft_c(float2 *buf, const float2 *__restrict__ tw, int tid,
                                           int nt) {
   if constexpr (S < SEnd) {
     constexpr int R = StaticPlan<N>::radix(S);
-    fft_pass_c<R, Ns, N, DIR, EPT, LGH>(buf, tw, tid, nt);
-    lds_fft_c<N, DIR, EPT, LGH, S + 1, Ns * R, SEnd>(buf, tw, tid, nt);
+    fft_pass_c<R, Ns, N, DIR, EPT, LGH, ODD>(buf, tw, tid, nt);
+    lds_fft_c<N, DIR, EPT, LGH, S + 1, Ns * R, SEnd, ODD>(buf, tw, tid, nt);
   }
 }
 
@@ -838,6 +840,100 @@ __device__ __forceinline__ void fft_c_global(float2 *buf, const float2 *__restri
   __syncthreads();
   lds_fft_c<N, DIR, EPT, LGH, 1, R0, SP::passes - 1>(buf, tw, tid, nt);
   fft_pass_c_last<RL, N / RL, N, DIR, EPT, LGH, LO, HI>(buf, tw, tid, nt, st);
+}
+
+// ---- pieces of chained compile-time transforms ------------------------------
+// A chain of transforms through one LDS buffer: chain_first takes a thread's
+// inputs from ld (which may read the buffer: a barrier separates the reads
+// from the writes), lds_fft_c runs the passes between, chain_last leaves the
+// outputs in registers.
+//
+// ODD: the N values of X[m] = sum_j x[j] W_2N^(j (2m + 1)), the transform of
+// length 2N of a zero-padded sequence at the odd frequencies.  Splitting j as
+// the passes do gives the same butterflies with the twiddles W_(2 Ns R)^((2k + 1) r)
+// for W_(Ns R)^(k r) (table index (2k + 1) N / (Ns R) of the table of size 2N),
+// in the first pass the constants W_2R^r.
+
+// Pass 0 of N points.  ld(i, s) gives element i; of a power of two length s is
+// the thread's element count, i = (tid >> LGH) + s N / EPT.
+template <int R, int N, int DIR, int EPT, int LGH, bool ODD, typename Ld>
+__device__ __forceinline__ void chain_first(float2 *buf, int tid, int nt, Ld ld) {
+  constexpr int MAXB = EPT / R, H = 1 << LGH, nbPer = N / R, nb = nbPer << LGH;
+  static_assert(MAXB >= 1 && nbPer % 16 == 0, "layout");
+  float2 v[MAXB][R];
+#pragma unroll
+  for (int q = 0; q < MAXB; ++q) {
+    const int g = tid + q * nt;
+    if (g < nb) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[q][r] = ld((g >> LGH) + r * nbPer, q + r * MAXB);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < MAXB; ++q) {
+    const int g = tid + q * nt;
+    if (g < nb) {
+      if constexpr (ODD)
+        static_for<R>([&](auto r) { v[q][r] = rotate<decltype(r)::value, 2 * R, DIR>(v[q][r]); });
+      butterfly<R, DIR>(v[q]);
+      const int base = (lds_pad((g >> LGH) * R) << LGH) + (g & (H - 1));
+#pragma unroll
+      for (int r = 0; r < R; ++r) buf[base + r * H] = v[q][out_slot<R>(r)];
+    }
+  }
+  __syncthreads();
+}
+
+// a[r] *= w^(2r + 1), w = exp(DIR pi i k / N): the twiddles W_N^(k r) of a last
+// pass and the common factor W_2N^k.  tw2: the table of size 2N.
+template <int R, int DIR>
+__device__ __forceinline__ void twiddle_mod(float2 *a, const float2 *__restrict__ tw2, int k) {
+  auto ld = [&](int m) {
+    float2 w = tw2[(unsigned)(k * m)];
+    if (DIR > 0) w.y = -w.y;
+    return w;
+  };
+  float2 p[R];
+  p[0] = ld(1);
+#pragma unroll
+  for (int h = 1; h < R; h *= 2) {
+    const float2 b = ld(2 * h);
+#pragma unroll
+    for (int r = h; r < 2 * h && r < R; ++r) p[r] = cmul(p[r - h], b);
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) a[r] = cmul(a[r], p[r]);
+}
+
+// The last pass; output (k, r) = element k + r N / R of butterfly q goes to
+// out[q * R + r].  MOD: times exp(DIR pi i element / N) (tw: the table of size 2N).
+template <int R, int N, int DIR, int EPT, int LGH, bool MOD>
+__device__ __forceinline__ void chain_last(const float2 *buf, const float2 *__restrict__ tw,
+                                           int tid, int nt, float2 *out) {
+  constexpr int MAXB = EPT / R, H = 1 << LGH, Ns = N / R, nb = Ns << LGH;
+  static_assert(MAXB >= 1 && Ns % 16 == 0, "layout");
+  constexpr int rstride = (Ns + Ns / 16) << LGH;
+#pragma unroll
+  for (int q = 0; q < MAXB; ++q) {
+    const int g = tid + q * nt;
+    if (g < nb) {
+      const int k = g >> LGH;
+      const int base = (lds_pad(k) << LGH) + (g & (H - 1));
+      float2 v[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = buf[base + r * rstride];
+      if constexpr (MOD)
+        twiddle_mod<R, DIR>(v, tw, k);
+      else
+        twiddle<R, DIR>(v, tw, (unsigned)k);
+      butterfly<R, DIR>(v);
+      static_for<R>([&](auto r) {
+        constexpr int M = decltype(r)::value;
+        out[q * R + M] = rotate<MOD ? M : 0, 2 * R, DIR>(v[out_slot<R>(M)]);
+      });
+    }
+  }
 }
 
 // ---- compile-time transforms exchanged one component at a time ----------

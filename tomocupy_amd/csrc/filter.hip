@@ -205,7 +205,8 @@ __global__ __launch_bounds__(1024) void k_flt_edges64(const double *__restrict__
 }
 
 // H2[k] = FFT_2n(h2)[k] / (2n), h2 = h on lags (-n, n) wrapped to length 2n
-// (h2[n] = 0); FP64 segment sums as above, rounded once.  Also, at
+// (h2[n] = 0); FP64 segment sums as above, rounded once; a slice's n even
+// frequencies, then its n odd ones.  Also, at
 // H2 + nz 2n, the spectra for a differenced input: with d[j] = z[j] - z[j-1]
 // (circular, length 2n), D[k] = Z[k] (1 - W^k), W = exp(-2 pi i/2n), so
 // Z[k] H2[k] = D[k] H2[k] / (1 - W^k) for k > 0; slot 0 keeps H2[0] (the DC
@@ -248,7 +249,8 @@ __global__ __launch_bounds__(1024) void k_flt_H2_64(const double *__restrict__ h
   }
   sr /= n2;
   si /= n2;
-  H2[(size_t)z * n2 + k] = make_float2((float)sr, (float)si);
+  const size_t at = (size_t)z * n2 + (k >> 1) + (size_t)(k & 1) * n;
+  H2[at] = make_float2((float)sr, (float)si);
   double gr = sr, gi = si;
   if (k > 0) {
     // 1 - W^k = 2 sin^2(pi k/2n) + i sin(pi k/n)
@@ -257,7 +259,7 @@ __global__ __launch_bounds__(1024) void k_flt_H2_64(const double *__restrict__ h
     gr = (sr * dr + si * di) / den;
     gi = (si * dr - sr * di) / den;
   }
-  H2[((size_t)gridDim.y + z) * n2 + k] = make_float2((float)gr, (float)gi);
+  H2[(size_t)gridDim.y * n2 + at] = make_float2((float)gr, (float)gi);
 }
 
 }  // namespace

@@ -80,15 +80,18 @@ __device__ __forceinline__ float block_max(float m) {
   return m;
 }
 
-// Sum over the workgroup of the threads' v; thread 0 gets the result (every
+// Sum over the workgroup of the threads' v, per sequence of 2^LG interleaved
+// ones (then of one wave); thread t < 2^LG gets the result of sequence t (every
 // thread must call it).
+template <int LG = 0>
 __device__ __forceinline__ float2 block_sum2(float2 v) {
   __shared__ float2 wsum[16];
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
+  for (int o = 32; o >= 1 << LG; o >>= 1) {
     v.x += __shfl_xor(v.x, o, 64);
     v.y += __shfl_xor(v.y, o, 64);
   }
+  if constexpr (LG > 0) return v;
   const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
   if ((threadIdx.x & 63) == 0) wsum[w] = v;
   __syncthreads();
@@ -169,119 +172,245 @@ __global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_prep(const T *__rest
 // Fused FBP filter + pair packing + shifted detector FFT (the fused form of
 // fbp_filter_center and the first stage of the backprojection).  Per angle p
 // and complex slice c: z = x1 + i*x2 zero-padded to 2n, FFT_2n, multiply by
-// the two slices' wrapped filter spectra (Y = Z (H1+H2)/2 + conj(Z(-k))
-// (H1-H2)/2, exact for real rows), IFFT_2n, add the edge-replication terms
-// x[0] HL + x[n-1] HR per slice, then the shifted n-point DFT of k_fr_prep.
-template <typename T, int NS>
-__global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_filtprep(
+// the two slices' wrapped filter spectra (Y[k] = (u H1 + v H2) / 2 with
+// u = Z[k] + conj Z[-k], v = Z[k] - conj Z[-k], exact for real rows), IFFT_2n,
+// add the edge-replication terms x[0] HL + x[n-1] HR per slice, then the
+// shifted n-point DFT of k_fr_prep.
+//
+// All of it in n-point transforms, as z is zero from n on and only outputs
+// j < n are used.  The even frequencies of Z are DFT_n(z), the odd ones DFT_n of
+// z[j] W_2n^j (Y[-k] pairs m with n - m and n - 1 - m).  The even half of the
+// inverse transform is a sequence of n points whose shifted DFT is Y's even half
+// again, moved by n/2: it needs no transform.  The odd half is
+// exp(pi i j / n) times an inverse DFT_n.  With s(j) = -(-1)^j,
+//   G[k] = s(k) scale (DFT_n(s(j) (odd half + edge terms))[k] - n Y[2 ((k + n/2) mod n)]):
+// four transforms of n points instead of two of 2n and one of n.
+//
+// Compiled sizes: the LDS buffer is one row of n points (2n before), a thread
+// holds 16 values, and short rows share a wave (fp_lg).  What bounds it is vector
+// arithmetic.  Powers of two go from the inverse transform to the next without
+// LDS, their last and first passes having the same elements per thread.
+// Measured, us (the two transforms of 2n and one of n in brackets): n = 2048, 1500
+// angles, 8 slices 127 (169), float16 120 (165), n = 4096 440 (728), n = 1280, 600
+// angles, 8 slices 44 (56), n = 2560 88 (133), run-time n = 2448 282 (349).
+//
+// WIDE: 256 threads for a row, a few values each, the odd and even frequencies
+// as two interleaved transforms: a third of the chain of passes that a wave of
+// the register form runs alone, which is the time of a launch that leaves most
+// SIMDs with one wave or none.  fp_wide draws the line, us for the whole
+// reconstruction, WIDE minus register form: n = 256 and 512 -3.7 and -10.4 at
+// 200 rows, -3.0 and -3.7 at 1800, +3.4 and +3.9 at 3600; n = 768 and 1024 -4.5
+// and -3.7 at 200, -4.3 and -2.8 at 1200, +1.6 and +3.5 at 1800; n = 1280 -0.6
+// at 200 and 1536 -2.3, +11.8 and +11.7 at 1200, so not beyond 1024.
+constexpr int kFpWideMax = 1024, kFpWideThreads = 256;
+inline bool fp_wide(int n, int64_t rows) {
+  return n <= kFpWideMax && rows <= (n <= 512 ? 2304 : 1536);
+}
+constexpr int fp_lg(int N) { return N == 256 ? 2 : N == 512 ? 1 : 0; }
+// threads: exact for powers of two, else 15 values each (radix 3 and 5 passes)
+constexpr int fp_threads(int N) {
+  return (N & (N - 1)) == 0 ? (N << fp_lg(N)) / kFftEPT : ((N + 14) / 15 + 63) / 64 * 64;
+}
+
+template <typename T, int NS, bool WIDE>
+__global__ __launch_bounds__(NS > 0 && !WIDE ? 512 : 1024) void k_fr_filtprep(
     const T *__restrict__ data, cpx<T> *__restrict__ G, const float2 *__restrict__ H2,
-    const float *__restrict__ HL, const float *__restrict__ HR, FftDesc fd2, FftDesc fd1, int n,
-    int nproj, int nz, int nzc, float scale, float *__restrict__ gmax) {
+    const float *__restrict__ HL, const float *__restrict__ HR, const float2 *__restrict__ tw2,
+    FftDesc fd, int n_, int nproj, int nz, int nzc, float scale, float *__restrict__ gmax) {
   extern __shared__ float2 sm[];
-  __shared__ float edge[4];
-  const int p = blockIdx.x, c = blockIdx.y;
-  const int tid = threadIdx.x, nt = blockDim.x;
+  constexpr int LG = NS > 0 && !WIDE ? fp_lg(NS) : 0, H = 1 << LG;
+  const int n = NS > 0 ? NS : n_, nt = NS > 0 && !WIDE ? fp_threads(NS) : blockDim.x;
+  const int tid = threadIdx.x, t = tid & (H - 1), c = blockIdx.y;
   if (c >= nzc) return;
+  __builtin_assume(tid >= 0 && tid < 1024);
+  const bool live = LG == 0 || (int)blockIdx.x * H + t < nproj;
+  const int p = live ? blockIdx.x * H + t : nproj - 1;
   cpx<T> *out = G + ((size_t)c * nproj + p) * n;
-  const int n2 = 2 * n;
   const int z2 = c + nzc;
   const bool has2 = z2 < nz;
   const int zb = has2 ? z2 : c;
   const T *r1 = data + ((size_t)c * nproj + p) * n;
   const T *r2 = data + ((size_t)zb * nproj + p) * n;
-  if (tid == 0) {
-    edge[0] = ldr(r1);
-    edge[1] = ldr(r1 + n - 1);
-    edge[2] = has2 ? ldr(r2) : 0.f;
-    edge[3] = has2 ? ldr(r2 + n - 1) : 0.f;
-  }
   // High-pass filters (|H2[0]| under 1 % of |H2[n/2]| for both slices, the
   // ramp family) transform the differenced row d[j] = z[j] - z[j-1] with the
   // spectra H2 / (1 - W^k) (k_flt_H2_64) and the DC term from the row sum:
   // the float32 rounding of the transform is then relative to the small
   // differences of a smooth row rather than to its large low frequencies,
-  // which the filter discards (at n = 2048, 24 angles, shepp: 1.1e-5 -> about
-  // 1e-6 rel-L2 against the FP64 filter).
+  // which the filter discards (at n = 2048, 24 angles, shepp: 1.1e-5 -> 4.3e-6
+  // rel-L2 against the FP64 filter).  d[n] = -z[n-1] joins d[0] as
+  // W^n = +-1 at even and odd frequencies.
   // (float32 plans only: 16-bit storage rounds far above this error)
-  const float2 *H2c = H2 + (size_t)c * n2, *H2b = H2 + (size_t)zb * n2;
+  const float2 *Ha = H2 + (size_t)c * 2 * n, *Hb = H2 + (size_t)zb * 2 * n;
+  const int hmid = (n / 4) + (n / 2 & 1) * n;  // (even frequencies, then odd)
   const bool diff = std::is_same<T, float>::value &&
-                    cabs2(H2c[0]) <= 1e-4f * cabs2(H2c[n / 2]) &&
-                    cabs2(H2b[0]) <= 1e-4f * cabs2(H2b[n / 2]);
-  auto zat = [&](int j) {  // z[j], zero outside [0, n)
-    return (unsigned)j < (unsigned)n ? tof2(cpx<T>{r1[j], has2 ? r2[j] : T(0)})
-                                     : make_float2(0.f, 0.f);
-  };
+                    cabs2(Ha[0]) <= 1e-4f * cabs2(Ha[hmid]) &&
+                    cabs2(Hb[0]) <= 1e-4f * cabs2(Hb[hmid]);
+  if (diff) {
+    Ha += (size_t)nz * 2 * n;
+    Hb += (size_t)nz * 2 * n;
+  }
+  const float back = diff ? -1.f : 0.f;
+  auto zat = [&](int j) { return tof2(cpx<T>{r1[j], has2 ? r2[j] : T(0)}); };
   float2 zsum = make_float2(0.f, 0.f);  // this thread's part of the row sum
-  auto zdiff = [&](int j) {
-    const float2 zj = zat(j);
-    zsum = cadd(zsum, zj);
-    return csub(zj, zat(j - 1));
+  // z[j] or d[j], the wrapped term of d[0] with the sign of the frequencies
+  auto zin = [&](int j, auto odd) {
+    const float2 z = zat(j);
+    if constexpr (!decltype(odd)::value) zsum = cadd(zsum, z);
+    if constexpr (!std::is_same<T, float>::value) return z;
+    const float2 zp = zat(j == 0 ? n - 1 : j - 1);
+    const float b = decltype(odd)::value && j == 0 ? -back : back;
+    return make_float2(fmaf(b, zp.x, z.x), fmaf(b, zp.y, z.y));
   };
-  // (one loader per branch: a branch inside the loader would keep the loads
-  // of a thread from being issued together)
-  if constexpr (NS > 0) {
-    // (the barriers inside make edge[] visible before its use below)
-    if (diff)
-      fft_c_from_global<2 * NS, -1, kFftEPT, 0>(sm, fd2.tw, tid, nt,
-                                                [&](int j, int) { return zdiff(j); });
-    else
-      fft_c_from_global<2 * NS, -1, kFftEPT, 0>(sm, fd2.tw, tid, nt,
-                                                [&](int j, int) { return zat(j); });
-  } else {
-    auto st = [&](int j, float2 v) { sm[j] = v; };
-    if (diff)
-      stage_lds<8, float2>(n2, tid, nt, [&](int j) { return zdiff(j); }, st);
-    else
-      stage_lds<8, float2>(n2, tid, nt, [&](int j) { return zat(j); }, st);
-    __syncthreads();
-    lds_fft<-1>(sm, fd2, 0, tid, nt);
-  }
-  float2 z0 = make_float2(0.f, 0.f);  // Z[0] (thread 0), for the differenced form
-  if (diff) z0 = block_sum2(zsum);
-  const float2 *Ha = diff ? H2c + (size_t)nz * n2 : H2c;
-  const float2 *Hb = diff ? H2b + (size_t)nz * n2 : H2b;
-  for (int k = tid; k <= n; k += nt) {
-    const int km = (n2 - k) % n2;
-    float2 zk = sm[lidx<NS>(k)], zm = sm[lidx<NS>(km)];
-    if (diff && k == 0) zk = zm = z0;
-    const float2 ak = Ha[k], bk = Hb[k], am = Ha[km], bm = Hb[km];
-    const float2 sk = cscale(cadd(ak, bk), 0.5f), dk = cscale(csub(ak, bk), 0.5f);
-    const float2 sm_ = cscale(cadd(am, bm), 0.5f), dm = cscale(csub(am, bm), 0.5f);
-    const float2 yk = cadd(cmul(zk, sk), cmul(cconj(zm), dk));
-    const float2 ym = cadd(cmul(zm, sm_), cmul(cconj(zk), dm));
-    sm[lidx<NS>(k)] = yk;
-    if (km != k) sm[lidx<NS>(km)] = ym;
-  }
-  __syncthreads();
-  if constexpr (NS > 0)
-    lds_fft_c<2 * NS, 1, kFftEPT, 0>(sm, fd2.tw, tid, nt);
-  else
-    lds_fft<1>(sm, fd2, 0, tid, nt);
+  auto mix = [](float2 zk, float2 zm, float2 a, float2 b) {  // 2 Y[k]
+    const float2 u = make_float2(zk.x + zm.x, zk.y - zm.y);
+    const float2 v = make_float2(zk.x - zm.x, zk.y + zm.y);
+    return cadd(cmul(u, a), cmul(v, b));
+  };
   const float *hl1 = HL + (size_t)c * n, *hr1 = HR + (size_t)c * n;
   const float *hl2 = HL + (size_t)zb * n, *hr2 = HR + (size_t)zb * n;
-  const float e0 = edge[0], e1 = edge[1], e2 = edge[2], e3 = edge[3];
-  for (int j = tid; j < n; j += nt) {
-    float2 y = sm[lidx<NS>(j)];
-    y.x += e0 * hl1[j] + e1 * hr1[j];
-    y.y += e2 * hl2[j] + e3 * hr2[j];
-    sm[lidx<NS>(j)] = cscale(y, shift_sign(j));
-  }
-  __syncthreads();
-  if constexpr (NS > 0) {
-    // the n-point pass from LDS, its last stage straight to the spectrum
-    constexpr int RL = StaticPlan<NS>::radix(StaticPlan<NS>::passes - 1);
-    lds_fft_c<NS, -1, kFftEPT, 0, 0, 1, StaticPlan<NS>::passes - 1>(sm, fd1.tw, tid, nt);
-    float m = 0.f;
-    fft_pass_c_last<RL, NS / RL, NS, -1, kFftEPT, 0>(sm, fd1.tw, tid, nt,
-                                                     [&](int k, int, float2 x) {
-      const float2 v = cscale(x, shift_sign(k) * scale);
-      m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)));
-      stc(out + k, v);
+  const float2 e0 = cscale(zat(0), 2.f), e1 = cscale(zat(n - 1), 2.f);
+  auto edges = [&](int j, float sg, float2 y) {  // s (y + edge terms), all doubled
+    return make_float2(sg * (y.x + (e0.x * hl1[j] + e1.x * hr1[j])),
+                       sg * (y.y + (e0.y * hl2[j] + e1.y * hr2[j])));
+  };
+  const float fn = (float)n, hscale = 0.5f * scale;
+  float m = 0.f;
+  auto store = [&](int k, float sg, float2 tk, float2 y) {
+    const float2 v = cscale(make_float2(fmaf(-fn, y.x, tk.x), fmaf(-fn, y.y, tk.y)), sg * hscale);
+    m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)));
+    if (live) stc(out + k, v);
+  };
+  typedef std::integral_constant<bool, true> Odd;
+  typedef std::integral_constant<bool, false> Even;
+  if constexpr (NS > 0 && WIDE) {
+    // odd and even frequencies as two interleaved transforms, then the odd
+    // half's two behind them
+    float2 *y = sm + 2 * lds_padded_len(NS);
+    for (int j = tid; j < NS; j += nt) {
+      sm[2 * lds_pad(j)] = cmul(zin(j, Odd()), tw2[j]);
+      sm[2 * lds_pad(j) + 1] = zin(j, Even());
+    }
+    __syncthreads();
+    lds_fft_c<NS, -1, kFftEPT, 1>(sm, fd.tw, tid, nt);
+    if (diff) {
+      const float2 z0 = block_sum2(zsum);
+      if (tid == 0) sm[1] = z0;
+    }
+    for (int k = tid; k < NS; k += nt)
+      y[lds_pad(k)] = mix(sm[2 * lds_pad(k)], sm[2 * lds_pad(NS - 1 - k)], Ha[NS + k], Hb[NS + k]);
+    __syncthreads();
+    lds_fft_c<NS, 1, kFftEPT, 0>(y, fd.tw, tid, nt);
+    for (int j = tid; j < NS; j += nt)
+      y[lds_pad(j)] = edges(j, shift_sign(j), cmul(y[lds_pad(j)], cconj(tw2[j])));
+    __syncthreads();
+    lds_fft_c<NS, -1, kFftEPT, 0>(y, fd.tw, tid, nt);
+    for (int k = tid; k < NS; k += nt) {
+      const int i = 2 * k < NS ? k + NS / 2 : k - NS / 2, im = i == 0 ? 0 : NS - i;
+      store(k, shift_sign(k), y[lds_pad(k)],
+            mix(sm[2 * lds_pad(i) + 1], sm[2 * lds_pad(im) + 1], Ha[i], Hb[i]));
+    }
+  } else if constexpr (NS > 0) {
+    using SP = StaticPlan<NS>;
+    constexpr int E = kFftEPT, R0 = SP::radix(0), RL = SP::radix(SP::passes - 1);
+    constexpr int MB = E / RL, NL = NS / RL, PL = SP::passes - 1;
+    constexpr bool pow2 = (NS & (NS - 1)) == 0;
+    auto at = [&](int i) -> float2 & { return sm[(lds_pad(i) << LG) + t]; };
+    // odd frequencies
+    chain_first<R0, NS, -1, E, LG, true>(sm, tid, nt, [&](int i, int) { return zin(i, Odd()); });
+    lds_fft_c<NS, -1, E, LG, 1, R0, SP::passes, true>(sm, tw2, tid, nt);
+    chain_first<R0, NS, 1, E, LG, false>(sm, tid, nt, [&](int i, int) {
+      return mix(at(i), at(NS - 1 - i), Ha[NS + i], Hb[NS + i]);
     });
-    store_max<T>(m, gmax, (size_t)c * nproj + p);
+    lds_fft_c<NS, 1, E, LG, 1, R0, PL>(sm, fd.tw, tid, nt);
+    float2 v[E];
+    chain_last<RL, NS, 1, E, LG, true>(sm, tw2, tid, nt, v);
+#pragma unroll
+    for (int q = 0; q < MB; ++q) {
+      const int j = (tid + q * nt) >> LG;
+      if (j >= NL) continue;
+#pragma unroll
+      for (int r = 0; r < RL; ++r) v[q * RL + r] = edges(j + r * NL, shift_sign(j), v[q * RL + r]);
+    }
+    if constexpr (pow2) {
+      chain_first<R0, NS, -1, E, LG, false>(
+          sm, tid, nt, [&](int, int s) { return v[(s % MB) * RL + s / MB]; });
+    } else {
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < MB; ++q) {
+        const int j = (tid + q * nt) >> LG;
+        if (j >= NL) continue;
+#pragma unroll
+        for (int r = 0; r < RL; ++r) at(j + r * NL) = v[q * RL + r];
+      }
+      __syncthreads();
+      chain_first<R0, NS, -1, E, LG, false>(sm, tid, nt, [&](int i, int) { return at(i); });
+    }
+    lds_fft_c<NS, -1, E, LG, 1, R0, PL>(sm, fd.tw, tid, nt);
+    chain_last<RL, NS, -1, E, LG, false>(sm, fd.tw, tid, nt, v);
+    // even frequencies
+    chain_first<R0, NS, -1, E, LG, false>(sm, tid, nt, [&](int i, int) { return zin(i, Even()); });
+    lds_fft_c<NS, -1, E, LG, 1, R0>(sm, fd.tw, tid, nt);
+    if (diff) {
+      const float2 z0 = block_sum2<LG>(zsum);
+      if (tid < H) sm[tid] = z0;
+      __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < MB; ++q) {
+      const int k = (tid + q * nt) >> LG;
+      if (k >= NL) continue;
+#pragma unroll
+      for (int r = 0; r < RL; ++r) {
+        const int kk = k + r * NL, i = kk < NS / 2 ? kk + NS / 2 : kk - NS / 2;
+        store(kk, shift_sign(k), v[q * RL + r],
+              mix(at(i), at(i == 0 ? 0 : NS - i), Ha[i], Hb[i]));
+      }
+    }
   } else {
-    lds_fft<-1>(sm, fd1, 0, tid, nt);
-    store_spectrum(out, sm, n, scale, tid, nt, gmax, (size_t)c * nproj + p);
+    // run-time sizes: the odd half in sm[0, n), the even half behind it
+    float2 *se = sm + n;
+    stage_lds<8, float2>(
+        n, tid, nt, [&](int j) { return zin(j, Odd()); },
+        [&](int j, float2 x) { sm[j] = cmul(x, tw2[j]); });
+    __syncthreads();
+    lds_fft<-1>(sm, fd, 0, tid, nt);
+    for (int k = tid; 2 * k < n; k += nt) {  // (H2[-k] = conj H2[k])
+      const int km = n - 1 - k;
+      const float2 zk = sm[k], zm = sm[km], a = Ha[n + k], b = Hb[n + k];
+      sm[k] = mix(zk, zm, a, b);
+      sm[km] = mix(zm, zk, cconj(a), cconj(b));
+    }
+    __syncthreads();
+    lds_fft<1>(sm, fd, 0, tid, nt);
+    for (int j = tid; j < n; j += nt) sm[j] = edges(j, shift_sign(j), cmul(sm[j], cconj(tw2[j])));
+    __syncthreads();
+    lds_fft<-1>(sm, fd, 0, tid, nt);
+    stage_lds<8, float2>(
+        n, tid, nt, [&](int j) { return zin(j, Even()); }, [&](int j, float2 x) { se[j] = x; });
+    __syncthreads();
+    lds_fft<-1>(se, fd, 0, tid, nt);
+    if (diff) {
+      const float2 z0 = block_sum2(zsum);
+      if (tid == 0) se[0] = z0;
+      __syncthreads();
+    }
+    for (int k = tid; k < n; k += nt) {
+      const int i = 2 * k < n ? k + n / 2 : k - n / 2;
+      store(k, shift_sign(k), sm[k], mix(se[i], se[i == 0 ? 0 : n - i], Ha[i], Hb[i]));
+    }
+  }
+  if constexpr (std::is_same<T, float>::value) {
+    if (gmax) {
+      if constexpr (LG > 0) {
+#pragma unroll
+        for (int o = 32; o >= H; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+        if (tid < H && live) gmax[(size_t)c * nproj + p] = m;
+      } else {
+        m = block_max(m);
+        if (tid == 0) gmax[(size_t)c * nproj + p] = m;
+      }
+    }
   }
 }
 
@@ -1191,7 +1320,7 @@ struct tomo_fr_plan {
   int ntile = 0, nitems = 0, nred = 0, nslots = 0;
   DevBuf G, F, R;
   int colCB = 1, lgCB = 0, colThreads = 256, prepThreads = 256, rowThreads = 256;
-  int fpThreads = 256;                   // k_fr_filtprep (transforms of n and 2n)
+  int fpThreads = 256;                   // k_fr_filtprep
   int nsRow = 0, nsCol = 0, nsPrep = 0;  // compiled FFT sizes in use (0 = run-time sizes)
   int lgB = 0;                           // column-blocked R (see k_fr_rowfft)
   int gridChunk = kGridChunk;            // max list entries per gridding work item
@@ -1522,13 +1651,14 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
   P->rowLds = (int)lds_bytes(st2, n2);
   if (P->nsPrep > 0) {
     P->prepThreads = fft_threads(P->fft1.rule, n);
-    P->fpThreads = fft_threads(P->fft2.rule, n2);
+    P->fpThreads = fp_threads((int)n);
   } else {
     P->prepThreads = fft_rt_threads(P->fft1.d, 0);
-    P->fpThreads = std::max(P->prepThreads, fft_rt_threads(P->fft2.d, 0));
+    P->fpThreads = P->prepThreads;
   }
   P->prepLds = (int)lds_bytes(P->nsPrep > 0, n);
-  P->fpLds = (int)lds_bytes(P->nsPrep > 0, n2);
+  P->fpLds =
+      (int)(P->nsPrep > 0 ? lds_bytes(true, n) << fp_lg((int)n) : lds_bytes(false, n2));
   P->nsCol = 0;
   if (st2) {
     // (n is a multiple of the columns: 2^8 divides 2n)
@@ -1712,11 +1842,23 @@ static int fr_head(tomo_fr_plan *P, tomo_flt_plan *F, const T *data, hipStream_t
   const int ng = (int)P->ngrp;
   {
     ProfScope ps_("k_fr_filtprep", st);
+    auto launch = [&](auto kernel, int rows, int threads, int lds) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(nproj, rows), ng * 4), dim3(threads), lds,
+                         st, data, P->G.as<cpx<T>>(), F->H2.as<float2>(), F->HL.as<float>(),
+                         F->HR.as<float>(), F->fft2n.d.tw, P->fft1.d, n, nproj, nz, nzc,
+                         P->scale1, P->gmax.as<float>());
+    };
+    const bool wide = fp_wide(n, (int64_t)nproj * nzc);
     with_static_size(P->nsPrep, [&](auto ns) {
-      hipLaunchKernelGGL((k_fr_filtprep<T, decltype(ns)::value>), dim3(nproj, ng * 4),
-                         dim3(P->fpThreads), P->fpLds, st, data, P->G.as<cpx<T>>(),
-                         F->H2.as<float2>(), F->HL.as<float>(), F->HR.as<float>(), F->fft2n.d,
-                         P->fft1.d, n, nproj, nz, nzc, P->scale1, P->gmax.as<float>());
+      constexpr int NS = decltype(ns)::value;
+      if constexpr (NS > 0 && NS <= kFpWideMax) {
+        if (wide) {
+          launch(k_fr_filtprep<T, NS, true>, 1, kFpWideThreads,
+                 3 * (int)sizeof(float2) * lds_padded_len(NS));
+          return;
+        }
+      }
+      launch(k_fr_filtprep<T, NS, false>, NS > 0 ? 1 << fp_lg(NS) : 1, P->fpThreads, P->fpLds);
     });
   }
   TOMO_LAUNCH_CHECK();
