@@ -34,7 +34,6 @@ using namespace tomo;
 namespace {
 
 constexpr int kGridWaves = 4;   // waves (= work items) per gridding workgroup
-constexpr int kGridChunk = 512; // default max list entries per work item (multiple of 16)
 constexpr int kGridBatch = 64;  // list entries a gridding wave stages at a time
 // device memory for the interpolation's tile partials (fr_forward): as many
 // groups of 4 complex slices per launch as fit
@@ -542,43 +541,54 @@ struct Mma16<__bf16> {
   }
 };
 
-template <typename T>
-__global__ __launch_bounds__(64 * kGridWaves) void k_fr_grid16(
-    const int4 *__restrict__ items, int nitems, const int4 *__restrict__ ent,
-    const cpx<T> *__restrict__ G, cpx<T> *__restrict__ F, float *__restrict__ part, int n,
-    int ntile, int nslots, int nsamp, int nzc, float K2) {
+// A gridding wave's staged list entries and spectra, double-buffered.
+struct GridStage {
+  int4 se[2][kSeLen];
+  float2 sg[2][4][kSgLen];
+};
+
+// f(integral_constant<int, NL>) for a group whose slices from its first on are
+// `live`: NL = 1 .. 4 of them.  The products of slices that do not exist (a chunk
+// of 1, 2, 3, 5 .. slices) cost as much as the others.
+template <typename F>
+__device__ __forceinline__ void with_live(int live, F &&f) {
+  switch (live) {
+    case 1: f(std::integral_constant<int, 1>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    case 3: f(std::integral_constant<int, 3>()); break;
+    default: f(std::integral_constant<int, 4>()); break;
+  }
+}
+
+// One work item of the 16-bit gridding for one group of NL complex slices.
+template <typename T, int NL>
+__device__ __forceinline__ void grid16_item(const int4 item, const int4 *__restrict__ ent,
+                                            const cpx<T> *__restrict__ Gg, cpx<T> *__restrict__ Fg,
+                                            float *__restrict__ Pg, int n, int ntile, int nsamp,
+                                            float K2, GridStage &sh, int lane) {
   typedef Mma16<T> M;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int it = blockIdx.x * kGridWaves + wave;
-  const int grp = blockIdx.y;
-  if (it >= nitems) return;
-  const int4 item = items[it];
   const int tile = item.x, ebeg = item.y, cnt = item.z, slot = item.w;
   const int g4 = lane >> 4, i = lane & 15;
-  const int nlive = min(4, nzc - 4 * grp);
-  const cpx<T> *Gg = G + (size_t)(4 * grp) * nsamp;
   const GaussLane gl(i, K2, 0.f, 0.f);
-  floatx4 acc[8];
+  floatx4 acc[2 * NL];
 #pragma unroll
-  for (int m = 0; m < 8; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
-  __shared__ int4 se[kGridWaves][2][kSeLen];
-  __shared__ float2 sg[kGridWaves][2][4][kSgLen];
+  for (int m = 0; m < 2 * NL; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int eend = ebeg + cnt;
   int4 re = make_int4(-1, kPadStarts, 0, 0);
-  cpx<T> rg[4];
+  cpx<T> rg[NL];
   auto fetch = [&](int base) {
     const int idx = base + lane;
     re = idx < eend ? ent[idx] : make_int4(-1, kPadStarts, 0, 0);
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      rg[c] = (re.x >= 0 && c < nlive) ? Gg[(size_t)c * nsamp + re.x] : cpx<T>{T(0), T(0)};
+    for (int c = 0; c < NL; ++c)
+      rg[c] = re.x >= 0 ? Gg[(size_t)c * nsamp + re.x] : cpx<T>{T(0), T(0)};
   };
   if (cnt > 0) fetch(ebeg);
   int buf = 0;
   for (int bb = ebeg; bb < eend; bb += kGridBatch, buf ^= 1) {
-    se[wave][buf][se_at(lane)] = re;
+    sh.se[buf][se_at(lane)] = re;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) sg[wave][buf][c][sg_at(lane)] = tof2(rg[c]);
+    for (int c = 0; c < NL; ++c) sh.sg[buf][c][sg_at(lane)] = tof2(rg[c]);
     __builtin_amdgcn_wave_barrier();
     if (bb + kGridBatch < eend) fetch(bb + kGridBatch);
     const int ngr = min(kGridBatch, eend - bb) >> 5;
@@ -587,14 +597,14 @@ __global__ __launch_bounds__(64 * kGridWaves) void k_fr_grid16(
       // 32q + 8 g4 + u (u < 8) to both operands
       float e0v[8], e1v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) gl.pair(se[wave][buf][se_at(32 * q + 8 * g4 + u)], e0v[u], e1v[u]);
+      for (int u = 0; u < 8; ++u) gl.pair(sh.se[buf][se_at(32 * q + 8 * g4 + u)], e0v[u], e1v[u]);
       const typename M::v8 b = M::pack8(e0v);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+      for (int c = 0; c < NL; ++c) {
         float ar[8], ai[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          const float2 v = sg[wave][buf][c][sg_at(32 * q + 8 * g4 + u)];
+          const float2 v = sh.sg[buf][c][sg_at(32 * q + 8 * g4 + u)];
           ar[u] = e1v[u] * v.x;
           ai[u] = e1v[u] * v.y;
         }
@@ -612,19 +622,18 @@ __global__ __launch_bounds__(64 * kGridWaves) void k_fr_grid16(
     const size_t plane = (size_t)n2 * n2;
     const bool whole = (n2 & 15) == 0;
     const int o0 = (16 * TA + ib) * n2 + bcol;
-    if (whole && grp * 4 + 4 <= nzc) {
+    if (whole) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        cpx<T> *Fc = F + (size_t)(grp * 4 + c) * plane;
+      for (int c = 0; c < NL; ++c) {
+        cpx<T> *Fc = Fg + (size_t)c * plane;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           stc(Fc + (o0 + r * n2), make_float2(acc[2 * c][r], acc[2 * c + 1][r]));
       }
     } else {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (grp * 4 + c >= nzc) continue;
-        cpx<T> *Fc = F + (size_t)(grp * 4 + c) * plane;
+      for (int c = 0; c < NL; ++c) {
+        cpx<T> *Fc = Fg + (size_t)c * plane;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int a = 16 * TA + ib + r;
@@ -634,12 +643,33 @@ __global__ __launch_bounds__(64 * kGridWaves) void k_fr_grid16(
       }
     }
   } else {
-    float *P = part + ((size_t)grp * nslots + slot) * 2048;
+    float *P = Pg + (size_t)slot * 2048;
 #pragma unroll
-    for (int m = 0; m < 8; ++m)
+    for (int m = 0; m < 2 * NL; ++m)
 #pragma unroll
       for (int r = 0; r < 4; ++r) P[m * 256 + (ib + r) * 16 + j] = acc[m][r];
   }
+}
+
+// (five waves a SIMD, which the LDS allows, need the register bound: at 111
+// instead of 92 registers 172 us for n = 2048, 158 before)
+template <typename T>
+__global__ __launch_bounds__(64 * kGridWaves, 5) void k_fr_grid16(
+    const int4 *__restrict__ items, int nitems, const int4 *__restrict__ ent,
+    const cpx<T> *__restrict__ G, cpx<T> *__restrict__ F, float *__restrict__ part, int n,
+    int ntile, int nslots, int nsamp, int nzc, float K2) {
+  __shared__ GridStage sh[kGridWaves];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int it = blockIdx.x * kGridWaves + wave;
+  const int grp = blockIdx.y;
+  if (it >= nitems) return;
+  const size_t plane = (size_t)(2 * n) * (2 * n);
+  with_live(nzc - 4 * grp, [&](auto nl) {
+    grid16_item<T, decltype(nl)::value>(items[it], ent, G + (size_t)(4 * grp) * nsamp,
+                                        F + (size_t)(4 * grp) * plane,
+                                        part + (size_t)grp * nslots * 2048, n, ntile, nsamp, K2,
+                                        sh[wave], lane);
+  });
 }
 
 // Scale exponent of the float32 gridding: kA = 13 - floor(log2(max |G|))
@@ -714,38 +744,37 @@ __device__ __forceinline__ void split8(const float *x, half8_t &hi, half8_t &lo)
   lo = __builtin_bit_cast(half8_t, make_uint4(l[0], l[1], l[2], l[3]));
 }
 
-// One work item of the float32 gridding for one group of (up to) 4 complex
-// slices: Gg/Fg/Pg are the group's spectra, grid planes and partial tiles,
-// nlive of its 4 slices exist, kA is the group's scale exponent.
+// One work item of the float32 gridding for one group of NL = 1 .. 4 complex
+// slices: Gg/Fg/Pg are the group's spectra, grid planes and partial tiles, kA is
+// the group's scale exponent, se and sg the wave's staging buffers.
+template <int NL>
 __device__ __forceinline__ void grid_x3_item(const int4 item, const int4 *__restrict__ ent,
                                              const float2 *__restrict__ Gg,
                                              float2 *__restrict__ Fg, float *__restrict__ Pg,
-                                             int kA, int n, int ntile, int nsamp, int nlive,
-                                             float K2, int wave, int lane) {
+                                             int kA, int n, int ntile, int nsamp, float K2,
+                                             GridStage &sh, int lane) {
   const int tile = item.x, ebeg = item.y, cnt = item.z, slot = item.w;
   const int g4 = lane >> 4, i = lane & 15;
   const GaussLane gl(i, K2, 10.f, (float)kA);
-  floatx4 acc[8];
+  floatx4 acc[2 * NL];
 #pragma unroll
-  for (int m = 0; m < 8; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
-  __shared__ int4 se[kGridWaves][2][kSeLen];
-  __shared__ float2 sg[kGridWaves][2][4][kSgLen];
+  for (int m = 0; m < 2 * NL; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int eend = ebeg + cnt;
   int4 re = make_int4(-1, kPadStarts, 0, 0);
-  float2 rg[4];
+  float2 rg[NL];
   auto fetch = [&](int base) {
     const int idx = base + lane;
     re = idx < eend ? ent[idx] : make_int4(-1, kPadStarts, 0, 0);
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      rg[c] = (re.x >= 0 && c < nlive) ? Gg[(size_t)c * nsamp + re.x] : make_float2(0.f, 0.f);
+    for (int c = 0; c < NL; ++c)
+      rg[c] = re.x >= 0 ? Gg[(size_t)c * nsamp + re.x] : make_float2(0.f, 0.f);
   };
   if (cnt > 0) fetch(ebeg);
   int buf = 0;
   for (int bb = ebeg; bb < eend; bb += kGridBatch, buf ^= 1) {
-    se[wave][buf][se_at(lane)] = re;
+    sh.se[buf][se_at(lane)] = re;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) sg[wave][buf][c][sg_at(lane)] = rg[c];
+    for (int c = 0; c < NL; ++c) sh.sg[buf][c][sg_at(lane)] = rg[c];
     __builtin_amdgcn_wave_barrier();
     if (bb + kGridBatch < eend) fetch(bb + kGridBatch);
     const int ngr = min(kGridBatch, eend - bb) >> 5;
@@ -754,15 +783,15 @@ __device__ __forceinline__ void grid_x3_item(const int4 item, const int4 *__rest
       // operands, so the K order inside the instruction does not matter
       float e0v[8], e1v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) gl.pair(se[wave][buf][se_at(32 * q + 8 * g4 + u)], e0v[u], e1v[u]);
+      for (int u = 0; u < 8; ++u) gl.pair(sh.se[buf][se_at(32 * q + 8 * g4 + u)], e0v[u], e1v[u]);
       half8_t bh, bl;
       split8(e0v, bh, bl);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+      for (int c = 0; c < NL; ++c) {
         float vr[8], vi[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          const float2 v = sg[wave][buf][c][sg_at(32 * q + 8 * g4 + u)];
+          const float2 v = sh.sg[buf][c][sg_at(32 * q + 8 * g4 + u)];
           vr[u] = v.x;
           vi[u] = v.y;
         }
@@ -790,9 +819,9 @@ __device__ __forceinline__ void grid_x3_item(const int4 item, const int4 *__rest
     // each plane's base
     const bool whole = (n2 & 15) == 0;
     const int o0 = (16 * TA + ib) * n2 + bcol;
-    if (whole && nlive == 4) {
+    if (whole) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+      for (int c = 0; c < NL; ++c) {
         float2 *Fc = Fg + (size_t)c * plane;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -800,8 +829,7 @@ __device__ __forceinline__ void grid_x3_item(const int4 item, const int4 *__rest
       }
     } else {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if (c >= nlive) continue;
+      for (int c = 0; c < NL; ++c) {
         float2 *Fc = Fg + (size_t)c * plane;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -814,7 +842,7 @@ __device__ __forceinline__ void grid_x3_item(const int4 item, const int4 *__rest
   } else {
     float *Pw = Pg + (size_t)slot * 2048;
 #pragma unroll
-    for (int m = 0; m < 8; ++m)
+    for (int m = 0; m < 2 * NL; ++m)
 #pragma unroll
       for (int r = 0; r < 4; ++r) Pw[m * 256 + (ib + r) * 16 + j] = acc[m][r] * unscale;
   }
@@ -824,14 +852,18 @@ __global__ __launch_bounds__(64 * kGridWaves) void k_fr_grid_x3(
     const int4 *__restrict__ items, int nitems, const int4 *__restrict__ ent,
     const float2 *__restrict__ G, float2 *__restrict__ F, float *__restrict__ part,
     const int *__restrict__ ksc, int n, int ntile, int nslots, int nsamp, int nzc, float K2) {
+  __shared__ GridStage sh[kGridWaves];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int it = blockIdx.x * kGridWaves + wave;
   const int grp = blockIdx.y;
   if (it >= nitems) return;
   const size_t plane = (size_t)(2 * n) * (2 * n);
-  grid_x3_item(items[it], ent, G + (size_t)(4 * grp) * nsamp, F + (size_t)(4 * grp) * plane,
-               part + (size_t)grp * nslots * 2048, ksc[0], n, ntile, nsamp,
-               min(4, nzc - 4 * grp), K2, wave, lane);
+  with_live(nzc - 4 * grp, [&](auto nl) {
+    grid_x3_item<decltype(nl)::value>(items[it], ent, G + (size_t)(4 * grp) * nsamp,
+                                      F + (size_t)(4 * grp) * plane,
+                                      part + (size_t)grp * nslots * 2048, ksc[0], n, ntile, nsamp,
+                                      K2, sh[wave], lane);
+  });
 }
 
 // One group of 4 complex slices of one plan in a batched gridding launch.
@@ -851,12 +883,15 @@ struct GridJob {
 __global__ __launch_bounds__(64 * kGridWaves) void k_fr_grid_x3_batch(
     const GridJob *__restrict__ jobs, const int4 *__restrict__ wi, const int *__restrict__ wj,
     int nwork) {
+  __shared__ GridStage sh[kGridWaves];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int w = blockIdx.x * kGridWaves + wave;
   if (w >= nwork) return;
-  const GridJob jb = jobs[wj[w]];
-  grid_x3_item(wi[w], jb.ent, jb.G, jb.F, jb.part, jb.ksc[0], jb.n, jb.ntile, jb.nsamp, jb.nlive,
-               jb.K2, wave, lane);
+  const GridJob jb = jobs[__builtin_amdgcn_readfirstlane(wj[w])];
+  with_live(jb.nlive, [&](auto nl) {
+    grid_x3_item<decltype(nl)::value>(wi[w], jb.ent, jb.G, jb.F, jb.part, jb.ksc[0], jb.n,
+                                      jb.ntile, jb.nsamp, jb.K2, sh[wave], lane);
+  });
 }
 
 // Sums the partial tiles of heavily loaded tiles in chunk order.
@@ -1323,7 +1358,7 @@ struct tomo_fr_plan {
   int fpThreads = 256;                   // k_fr_filtprep
   int nsRow = 0, nsCol = 0, nsPrep = 0;  // compiled FFT sizes in use (0 = run-time sizes)
   int lgB = 0;                           // column-blocked R (see k_fr_rowfft)
-  int gridChunk = kGridChunk;            // max list entries per gridding work item
+  int gridChunk = 0;                     // max list entries per gridding work item
   int rowLds = 0, prepLds = 0, fpLds = 0;
   size_t colLds = 0;
   float scale1 = 0.f, K2 = 0.f;
@@ -1459,7 +1494,18 @@ int build_tables(tomo_fr_plan *P, const std::vector<float> &theta) {
     if (rc0) return rc0;
     TOMO_HIP(hipMemcpy(P->span.p, span.data(), sizeof(int2) * n2, hipMemcpyHostToDevice));
   }
-  // work items: whole tiles, or chunks of gridChunk entries for heavy tiles
+  // work items: whole tiles, or chunks of gridChunk entries for heavy tiles.  A
+  // wave walks an item alone, so a launch of little work lasts as long as its
+  // longest item: the default follows the entries per wave the chip holds.
+  // Measured, us for a backprojection with chunks of 128, 256, 512, 768: 25
+  // entries a wave (n = 256, 180 angles) 2 slices 31 32 36 40, 8 slices 39 42 51
+  // 60; 101 (n = 512, 360) 64 60 66 77; 337 (n = 1024, 600) 159 141 138 136;
+  // 404 (n = 512, 720, 16 slices) 148 118 120 117; 1690 (n = 2048, 1500) 699 600
+  // 575 566 (partial tiles are stored and summed).
+  if (P->gridChunk == 0) {
+    const int64_t per = off[ntiles] * P->ngrp / 4096;
+    P->gridChunk = per < 64 ? 128 : per < 256 ? 256 : per < 1024 ? 512 : 768;
+  }
   const int64_t kChunk = P->gridChunk;
   std::vector<int4> items, red;
   int nslots = 0;
