@@ -59,6 +59,13 @@ constexpr int col_lg(int N) { return ilog2c(16384 / N) > 4 ? 4 : ilog2c(16384 / 
 constexpr bool col_split(int N) {
   return N > 4096 || (N >= 2048 && (N << split_lg(N)) >= 24576);
 }
+// The adjoint's column pass stores whole rows of R and is split only where that
+// pays: column + row pass, us for 8 slices, split against fft_c_global, 2n = 3072
+// 138+107 against 127+99, 3840 212+195 against 188+186, 4096 229+167 against
+// 215+167, 4608 382+308 against 317+293, 8192 1203+716 against 1057+708, but 5120
+// 418+320 against 447+312 and 6144 585+433 against 626+422, where fft_c_global has
+// two columns (column-blocked R, split: 3072 129+120, 3840 207+226, 8192 820+1011).
+constexpr bool col_split_adj(int N) { return N > 4608 && (N & (N - 1)) != 0; }
 
 // Sign 1 - 2*((t+1) % 2): -1 for even t, +1 for odd t (kernels_fourierrec.cuh:121-132).
 __device__ __forceinline__ float shift_sign(int t) { return (t & 1) ? 1.f : -1.f; }
@@ -1080,7 +1087,7 @@ template <int NS>
 __global__ __launch_bounds__(1024) void k_fr_colfft_adj(const float *__restrict__ obj, float2 *__restrict__ R,
                                 const float *__restrict__ phix, const float *__restrict__ phiy,
                                 const int2 *__restrict__ circ, FftDesc fd, int n, int nz,
-                                int nzc, int lgCB, int blocked) {
+                                int nzc, int lgCB) {
   extern __shared__ float2 sm[];  // [a][t]: CB interleaved columns
   const int L = xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
   const int cb = L % gridDim.x, c = L / gridDim.x;
@@ -1090,11 +1097,10 @@ __global__ __launch_bounds__(1024) void k_fr_colfft_adj(const float *__restrict_
   const int n2 = 2 * n, v0 = cb * CB, h = n / 2;
   const int z2 = c + nzc;
   float2 *dst = R + (size_t)c * n2 * n;
-  float2 *blk = dst + (size_t)v0 * n2;  // block cb of the column-blocked layout
   if constexpr (NS > 0) {
     // compiled sizes: first pass from obj (rows outside [1+h, n+h] are
     // zero), last pass straight to R
-    constexpr int LG = col_split(NS) ? split_lg(NS) : col_lg(NS);
+    constexpr int LG = col_split_adj(NS) ? split_lg(NS) : col_lg(NS);
     auto ld = [&](int u, int t) {
       const int ty = u - 1 - h, tx = v0 + t;
       if (ty < 0 || ty >= n || tx >= n) return make_float2(0.f, 0.f);
@@ -1105,10 +1111,9 @@ __global__ __launch_bounds__(1024) void k_fr_colfft_adj(const float *__restrict_
                          (z2 < nz) ? obj[((size_t)z2 * n + ty) * n + tx] * ph : 0.f);
     };
     auto st = [&](int a, int t, float2 x) {
-      (blocked ? blk[(a << LG) + t] : dst[(size_t)a * n + v0 + t]) =
-          (a & 1) ? make_float2(-x.x, -x.y) : x;
+      dst[(size_t)a * n + v0 + t] = (a & 1) ? make_float2(-x.x, -x.y) : x;
     };
-    if constexpr (col_split(NS))
+    if constexpr (col_split_adj(NS))
       fft_c_split<NS, -1, LG, 0, NS>(reinterpret_cast<float *>(sm), fd.tw, tid, nt, ld, st);
     else
       fft_c_global<NS, -1, kFftEPT, LG>(sm, fd.tw, tid, nt, ld, st);
@@ -1146,26 +1151,19 @@ __global__ __launch_bounds__(1024) void k_fr_colfft_adj(const float *__restrict_
 
 template <int NS>
 __global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_rowfft_adj(const float2 *__restrict__ R, float2 *__restrict__ F, FftDesc fd,
-                                int n, int nzc, int lgB) {
+                                int n, int nzc) {
   extern __shared__ float2 sm[];
-  const int L = lgB > 0 ? xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y)
-                        : blockIdx.x + gridDim.x * blockIdx.y;
-  const int a = L % gridDim.x, c = L / gridDim.x;
+  const int a = blockIdx.x, c = blockIdx.y;
   if (c >= nzc) return;
   const int tid = threadIdx.x, nt = blockDim.x;
   const int n2 = 2 * n, h = n / 2;
   const float2 *src = R + ((size_t)c * n2 + a) * n;
-  const float2 *blk = R + (size_t)c * n2 * n + ((size_t)a << lgB);
   if constexpr (NS > 0) {
     float2 *dst = F + ((size_t)c * n2 + a) * n2;
     fft_c_global<NS, -1, kFftEPT, 0>(
         sm, fd.tw, tid, nt,
         [&](int v, int) {
-          const int o = v - h;
-          const float2 x =
-              (o < 0 || o >= n) ? make_float2(0.f, 0.f)
-              : lgB > 0 ? blk[((size_t)(o >> lgB) * n2 << lgB) + (o & ((1 << lgB) - 1))]
-                        : src[o];
+          const float2 x = (v >= h && v < h + n) ? src[v - h] : make_float2(0.f, 0.f);
           return (v & 1) ? make_float2(-x.x, -x.y) : x;
         },
         [&](int b, int, float2 x) { dst[b] = (b & 1) ? make_float2(-x.x, -x.y) : x; });
@@ -1361,6 +1359,8 @@ struct tomo_fr_plan {
   int gridChunk = 0;                     // max list entries per gridding work item
   int rowLds = 0, prepLds = 0, fpLds = 0;
   size_t colLds = 0;
+  int lgCBa = 0, colThreadsA = 256;      // k_fr_colfft_adj's lgCB, colThreads, colLds
+  size_t colLdsA = 0;
   float scale1 = 0.f, K2 = 0.f;
 };
 
@@ -1708,16 +1708,23 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
   P->nsCol = 0;
   if (st2) {
     // (n is a multiple of the columns: 2^8 divides 2n)
-    const bool split = col_split((int)n2);
-    const int lgs = split ? split_lg((int)n2) : col_lg((int)n2);
-    const size_t lds_s = (lds_bytes(true, n2) << lgs) / (split ? 2 : 1);
-    const int thr =
-        fft_threads(P->fft2.rule, (int64_t)n2 << lgs, split ? kFftSplitEPT : kFftEPT);
-    if (lds_s <= maxlds && thr > 0 && thr <= 1024) {
+    auto shape = [&](bool split, int &lgs, size_t &lds, int &thr) {
+      lgs = split ? split_lg((int)n2) : col_lg((int)n2);
+      lds = (lds_bytes(true, n2) << lgs) / (split ? 2 : 1);
+      thr = fft_threads(P->fft2.rule, (int64_t)n2 << lgs, split ? kFftSplitEPT : kFftEPT);
+      return lds <= maxlds && thr > 0 && thr <= 1024;
+    };
+    int lgs = 0, thr = 0, lga = 0, thra = 0;
+    size_t lds_s = 0, lds_a = 0;
+    if (shape(col_split((int)n2), lgs, lds_s, thr) &&
+        shape(col_split_adj((int)n2), lga, lds_a, thra)) {
       P->nsCol = (int)n2;
       P->lgCB = lgs;
       P->colLds = lds_s;
       P->colThreads = thr;
+      P->lgCBa = lga;
+      P->colLdsA = lds_a;
+      P->colThreadsA = thra;
     }
   }
   if (P->nsCol == 0) {
@@ -1727,6 +1734,9 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
       P->lgCB += 1;
     P->colLds = lds_bytes(false, n2) << P->lgCB;
     P->colThreads = fft_rt_threads(P->fft2.d, P->lgCB);
+    P->lgCBa = P->lgCB;
+    P->colLdsA = P->colLds;
+    P->colThreadsA = P->colThreads;
   }
   P->colCB = 1 << P->lgCB;
   const int lg = P->lgCB;
@@ -1770,7 +1780,7 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
     return fail(TOMO_EHIP);
   }
   with_static_size(P->nsCol, [&](auto ns) {
-    lds_attr((const void *)k_fr_colfft_adj<decltype(ns)::value>, P->colLds);
+    lds_attr((const void *)k_fr_colfft_adj<decltype(ns)::value>, P->colLdsA);
   });
   const int rowLds = P->rowLds;
   with_static_size(P->nsRow, [&](auto ns) {
@@ -2205,11 +2215,12 @@ extern "C" int fr_forward(tomo_fr_plan *P, void *data_, const void *obj_, void *
     ProfScope ps_("k_fr_colfft_adj", st);
     with_static_size(P->nsCol, [&](auto ns) {
       constexpr int NS = decltype(ns)::value;
-      hipLaunchKernelGGL(k_fr_colfft_adj<NS>, dim3((unsigned)ceil_div(n, P->colCB), ng * 4),
-                         dim3(P->colThreads), P->colLds, st, obj,
+      hipLaunchKernelGGL(k_fr_colfft_adj<NS>,
+                         dim3((unsigned)ceil_div(n, 1 << P->lgCBa), ng * 4),
+                         dim3(P->colThreadsA), P->colLdsA, st, obj,
                          P->R.as<float2>(),
                          P->phix.as<float>(), P->phiy.as<float>(), P->circ.as<int2>(),
-                         P->fft2.d, n, nz, nzc, P->lgCB, P->lgB > 0 ? 1 : 0);
+                         P->fft2.d, n, nz, nzc, P->lgCBa);
     });
   }
   TOMO_LAUNCH_CHECK();
@@ -2218,7 +2229,7 @@ extern "C" int fr_forward(tomo_fr_plan *P, void *data_, const void *obj_, void *
     with_static_size(P->nsRow, [&](auto ns) {
       hipLaunchKernelGGL(k_fr_rowfft_adj<decltype(ns)::value>, dim3(n2, ng * 4),
                          dim3(P->rowThreads), P->rowLds,
-                         st, P->R.as<float2>(), P->F.as<float2>(), P->fft2.d, n, nzc, P->lgB);
+                         st, P->R.as<float2>(), P->F.as<float2>(), P->fft2.d, n, nzc);
     });
   }
   TOMO_LAUNCH_CHECK();
