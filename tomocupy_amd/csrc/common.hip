@@ -114,10 +114,14 @@ void fft_rt_radices(int N, FftDesc &d) {
   });
 }
 
-int FftPlan::init(int N) {
+int FftPlan::init(int N, bool by_rule) {
   int rc = radices(N, rule);
   if (rc) return rc;
   fft_rt_radices(N, d);
+  if (by_rule) {
+    d.nr = rule.nr;
+    std::copy(rule.r, rule.r + rule.nr, d.r);
+  }
   TOMO_REQUIRE(d.nr > 0 && fft_rt_threads(d, 0) > 0, "FFT length %d has no run-time plan", N);
   std::vector<float> mat;
   size_t off[3] = {0, 0, 0};

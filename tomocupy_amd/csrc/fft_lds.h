@@ -54,7 +54,8 @@ struct FftPlan {
   FftDesc d{};
   FftRule rule{};
   DevBuf tw, pm;
-  int init(int N);  // N <= 16384, prime factors <= kFftMaxPrime
+  // N <= 16384, prime factors <= kFftMaxPrime; by_rule: d has the rule's radices
+  int init(int N, bool by_rule = false);
   // the rule's radix sequence alone (no device memory, no HIP call)
   static int radices(int N, FftRule &r);
   void release() {
@@ -451,12 +452,15 @@ __device__ __forceinline__ void rt_twiddle(float2 *a, TabPtr tw, unsigned base) 
   });
 }
 
-// Butterflies of radix R a thread takes in a pass.
-constexpr int rt_maxb(int R) { return R <= kFftRtVals / 2 ? kFftRtVals / R : 1; }
+// Butterflies of radix R a thread takes in a pass (ten of radix 2 would cost a
+// wave per SIMD: 98 registers).
+constexpr int rt_maxb(int R) { return R == 2 ? 8 : R <= kFftRtVals / 2 ? kFftRtVals / R : 1; }
 
 // One pass of radix R over 2^lgH interleaved transforms of length N (element
-// i of transform t at buf[(i << lgH) + t]); ends with a barrier.
-template <int R, int DIR>
+// i of transform t at buf[(i << lgH) + t]); ends with a barrier.  PAD (lgH = 0):
+// 1 a first pass of radix 2, 4, 8 or 16 that writes element i at lds_pad(i), 2
+// the pass after it.
+template <int R, int DIR, int PAD = 0>
 __device__ __noinline__ void rt_pass(LdsPtr buf, int N_, int Ns_, TabPtr tw, int lgH_, int tid,
                                      int nt_) {
   constexpr int MAXB = rt_maxb(R);
@@ -473,13 +477,14 @@ __device__ __noinline__ void rt_pass(LdsPtr buf, int N_, int Ns_, TabPtr tw, int
     if (g < S) {
       LdsPtr p = buf + g;
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[q][r] = ldf2(p + r * S);
+      for (int r = 0; r < R; ++r) v[q][r] = ldf2(PAD == 2 ? buf + lds_pad(g + r * S) : p + r * S);
       const int j = g >> lgH;
       // j / Ns and j mod Ns: float quotient, corrected
       int jq = (int)((float)j * invNs), k = j - jq * Ns;
       if (k < 0) jq -= 1, k += Ns;
       if (k >= Ns) jq += 1, k -= Ns;
       o[q] = ((jq * Ns * R + k) << lgH) + (g - (j << lgH));
+      if constexpr (PAD == 1) o[q] = lds_pad(g * R);
       if (Ns > 1) rt_twiddle<R, DIR>(v[q], tw, (unsigned)(k * twstep));
       dft<R, DIR>(v[q]);
     }
@@ -585,6 +590,19 @@ __device__ __noinline__ void rt_pass_prime(LdsPtr buf, int N_, int Ns_, int p_, 
   __syncthreads();
 }
 
+// The prime pass with the output pairs a wave takes.
+template <int DIR, bool WIDE>
+__device__ __forceinline__ void rt_prime(LdsPtr buf, int N, int Ns, int R, TabPtr tw,
+                                         const float *pm, int lgH, int tid, int nt) {
+  const int G = rt_prime_pairs((N / R) << lgH, R);
+  if (WIDE && G == 16)
+    rt_pass_prime<16, DIR>(buf, N, Ns, R, tw, pm, lgH, tid, nt);
+  else if (G == 12)
+    rt_pass_prime<12, DIR>(buf, N, Ns, R, tw, pm, lgH, tid, nt);
+  else
+    rt_pass_prime<8, DIR>(buf, N, Ns, R, tw, pm, lgH, tid, nt);
+}
+
 // In-place transform of 2^lgH interleaved sequences of length d.N held in LDS
 // at buf[(i << lgH) + t], with a run-time plan and fft_rt_threads() threads.
 // The caller must __syncthreads() after filling buf; the function ends with a
@@ -607,17 +625,55 @@ __device__ void lds_fft(float2 *buf_, const FftDesc &d, int lgH, int tid, int nt
       TOMO_RT_PASS(12) TOMO_RT_PASS(13) TOMO_RT_PASS(14) TOMO_RT_PASS(15) TOMO_RT_PASS(16)
       TOMO_RT_PASS(17) TOMO_RT_PASS(18) TOMO_RT_PASS(20)
 #undef TOMO_RT_PASS
-      default:
-      {
-        const int G = rt_prime_pairs((N / R) << lgH, R);
-        if (WIDE && G == 16)
-          rt_pass_prime<16, DIR>(buf, N, Ns, R, tw, d.pm[np], lgH, tid, nt);
-        else if (G == 12)
-          rt_pass_prime<12, DIR>(buf, N, Ns, R, tw, d.pm[np], lgH, tid, nt);
-        else
-          rt_pass_prime<8, DIR>(buf, N, Ns, R, tw, d.pm[np], lgH, tid, nt);
-      }
-        ++np;
+      default: rt_prime<DIR, WIDE>(buf, N, Ns, R, tw, d.pm[np++], lgH, tid, nt);
+    }
+    Ns *= R;
+  }
+}
+
+// The same for one transform with a plan of the rule's radices (FftPlan::init
+// by_rule), in LDS of lds_padded_len(N) elements.  Its error is the smaller one
+// where a row is smooth and the result is its high frequencies: the powers of
+// two come first, whose differences of near-equal values are exact, and no
+// radix is a product with factors between.  What is left of the row's mean
+// then sits in one of their outputs.  (Relative error of a ramp-filtered row of
+// ellipses without noise, ne = 1016: 1.5e-5 with fft_rt_radices' order, 127
+// first, against 7.6e-6; 9792 6.6e-5 against 6.0e-5; white rows, ne = 4000:
+// 2.1e-7 against 1.8e-7.)  A first pass of a power of two writes with a pad
+// slot per 16 elements: its writes, R apart, would meet the same banks.
+template <int DIR, bool WIDE>
+__device__ void lds_fft_rule(float2 *buf_, const FftDesc &d, int tid, int nt) {
+  const LdsPtr buf = (LdsPtr)buf_;
+  const TabPtr tw = (TabPtr)d.tw;
+  const int N = d.N;
+  int Ns = 1, np = 0, s = 0;
+  if (d.nr > 1 && d.r[1] <= kFftRegPrime && N % 2 == 0) {
+    switch (d.r[0]) {
+      case 2: rt_pass<2, DIR, 1>(buf, N, 1, tw, 0, tid, nt); break;
+      case 4: rt_pass<4, DIR, 1>(buf, N, 1, tw, 0, tid, nt); break;
+      case 8: rt_pass<8, DIR, 1>(buf, N, 1, tw, 0, tid, nt); break;
+      case 16: rt_pass<16, DIR, 1>(buf, N, 1, tw, 0, tid, nt); break;
+    }
+    Ns = d.r[0];
+    switch (d.r[1]) {
+#define TOMO_RT_PASS(r) \
+  case r: rt_pass<r, DIR, 2>(buf, N, Ns, tw, 0, tid, nt); break;
+      TOMO_RT_PASS(2) TOMO_RT_PASS(3) TOMO_RT_PASS(4) TOMO_RT_PASS(5) TOMO_RT_PASS(7)
+      TOMO_RT_PASS(8) TOMO_RT_PASS(11) TOMO_RT_PASS(13) TOMO_RT_PASS(16) TOMO_RT_PASS(17)
+#undef TOMO_RT_PASS
+    }
+    Ns *= d.r[1];
+    s = 2;
+  }
+  for (; s < d.nr; ++s) {
+    const int R = d.r[s];
+    switch (R) {
+#define TOMO_RT_PASS(r) \
+  case r: rt_pass<r, DIR>(buf, N, Ns, tw, 0, tid, nt); break;
+      TOMO_RT_PASS(2) TOMO_RT_PASS(3) TOMO_RT_PASS(4) TOMO_RT_PASS(5) TOMO_RT_PASS(7)
+      TOMO_RT_PASS(8) TOMO_RT_PASS(11) TOMO_RT_PASS(13) TOMO_RT_PASS(16) TOMO_RT_PASS(17)
+#undef TOMO_RT_PASS
+      default: rt_prime<DIR, WIDE>(buf, N, Ns, R, tw, d.pm[np++], 0, tid, nt);
     }
     Ns *= R;
   }
@@ -628,7 +684,7 @@ __device__ void lds_fft(float2 *buf_, const FftDesc &d, int lgH, int tid, int nt
 // workgroups; N = 2000, row pass, us: 52 with 128 threads, 68 with 256), but
 // for lengths up to 1024, whose launches are short, one butterfly per thread;
 // -1 if more than 1024 would be needed.
-inline int fft_rt_threads(const FftDesc &d, int lgH) {
+inline int fft_rt_threads(const FftDesc &d, int lgH, bool one_each = true) {
   int64_t t = 64, one = 64;
   for (int i = 0; i < d.nr; ++i) {
     const int R = d.r[i];
@@ -639,7 +695,7 @@ inline int fft_rt_threads(const FftDesc &d, int lgH) {
       t = std::max<int64_t>(t, (nb + rt_maxb(R) - 1) / rt_maxb(R));
     if (R <= kFftRtVals && R != 19) one = std::max(one, nb);
   }
-  if (d.N <= 1024 && one <= 512) t = std::max(t, one);
+  if (one_each && d.N <= 1024 && one <= 512) t = std::max(t, one);
   t = (t + 63) / 64 * 64;
   return t > 1024 ? -1 : (int)t;
 }

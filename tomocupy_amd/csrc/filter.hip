@@ -8,9 +8,11 @@
 // The edge-replicate padding of fbp_filter_center
 // (src/tomocupy/reconstruction/backproj_functions.py:97-100) is applied while
 // loading, so the (nz, nproj, ne) temporary of the reference never exists.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -40,12 +42,22 @@ __global__ void k_flt_weights(const float *__restrict__ wfilter, const float *__
   w[(size_t)z * nh + k] = make_float2((float)(a * c), (float)(a * s));
 }
 
+// f(integral_constant<int, ne>) for the lengths whose rows run a compiled
+// transform (none), f(integral_constant<int, 0>) for the others.
+template <typename T, typename F>
+void with_row_size(int ne, F &&f) {
+  f(std::integral_constant<int, 0>());
+}
+
 // mode 0: rows of width ne already padded (cfunc_filter::filter);
-// mode 1: rows of width n, edge-replicate padded on load and cropped on store
-template <int MODE, typename T, bool WIDE>
+// mode 1: rows of width n, edge-replicate padded on load and cropped on store.
+// NS: ne as a compile-time constant; 0: a run-time plan, of the rule's radices
+// for float32 (lds_fft_rule), of few large ones for 16-bit rows.
+template <int MODE, typename T, int NS, bool WIDE>
 __global__ __launch_bounds__(1024) void k_flt_rows(T *__restrict__ g, const float2 *__restrict__ w,
-                                                   FftDesc fd, int ne, int n, int nproj) {
+                                                   FftDesc fd, int ne_, int n, int nproj) {
   extern __shared__ float2 sm[];
+  const int ne = NS > 0 ? NS : ne_;
   const int pp = blockIdx.x, z = blockIdx.y;
   const int tid = threadIdx.x, nt = blockDim.x;
   const int p0 = 2 * pp, p1 = p0 + 1;
@@ -53,16 +65,28 @@ __global__ __launch_bounds__(1024) void k_flt_rows(T *__restrict__ g, const floa
   const int width = MODE == 0 ? ne : n;
   T *r0 = g + ((size_t)z * nproj + p0) * width;
   T *r1 = g + ((size_t)z * nproj + (has1 ? p1 : p0)) * width;
-  const int pad = ne / 2 - n / 2;
-  stage_lds<8, cpx<T>>(
-      ne, tid, nt,
-      [&](int j) {
-        const int src = MODE == 1 ? min(max(j - pad, 0), n - 1) : j;
-        return cpx<T>{r0[src], has1 ? r1[src] : T(0)};
-      },
-      [&](int j, cpx<T> v) { sm[j] = tof2(v); });
-  __syncthreads();
-  lds_fft<-1, WIDE>(sm, fd, 0, tid, nt);
+  const int pad = MODE == 0 ? 0 : ne / 2 - n / 2;
+  auto ld = [&](int j) {
+    const int src = MODE == 1 ? min(max(j - pad, 0), n - 1) : j;
+    return cpx<T>{r0[src], has1 ? r1[src] : T(0)};
+  };
+  auto st = [&](int j, float2 y) {  // j: column of the padded row
+    const int x = j - pad;
+    if (x < 0 || x >= width) return;
+    str(r0 + x, y.x);
+    if (has1) str(r1 + x, y.y);
+  };
+  if constexpr (NS > 0) {
+    fft_c_from_global<NS, -1, kFftEPT, 0>(sm, fd.tw, tid, nt,
+                                          [&](int j, int) { return tof2(ld(j)); });
+  } else {
+    stage_lds<8, cpx<T>>(ne, tid, nt, ld, [&](int j, cpx<T> v) { sm[j] = tof2(v); });
+    __syncthreads();
+    if constexpr (std::is_same<T, float>::value)
+      lds_fft_rule<-1, WIDE>(sm, fd, tid, nt);
+    else
+      lds_fft<-1, WIDE>(sm, fd, 0, tid, nt);
+  }
   const float2 *wz = w + (size_t)z * (ne / 2 + 1);
   const int nh = ne / 2;
   for (int k = tid; k < ne; k += nt) {
@@ -74,22 +98,21 @@ __global__ __launch_bounds__(1024) void k_flt_rows(T *__restrict__ g, const floa
     } else {
       W = cconj(wz[ne - k]);
     }
-    sm[k] = cmul(sm[k], W);
+    sm[lidx<NS>(k)] = cmul(sm[lidx<NS>(k)], W);
   }
   __syncthreads();
-  lds_fft<1, WIDE>(sm, fd, 0, tid, nt);
-  if (MODE == 0) {
-    for (int j = tid; j < ne; j += nt) {
-      const float2 y = sm[j];
-      str(r0 + j, y.x);
-      if (has1) str(r1 + j, y.y);
-    }
+  if constexpr (NS > 0) {
+    using SP = StaticPlan<NS>;
+    constexpr int RL = SP::radix(SP::passes - 1);
+    lds_fft_c<NS, 1, kFftEPT, 0, 0, 1, SP::passes - 1>(sm, fd.tw, tid, nt);
+    fft_pass_c_last<RL, NS / RL, NS, 1, kFftEPT, 0>(
+        sm, fd.tw, tid, nt, [&](int j, int, float2 y) { st(j, y); });
   } else {
-    for (int j = tid; j < n; j += nt) {
-      const float2 y = sm[pad + j];
-      str(r0 + j, y.x);
-      if (has1) str(r1 + j, y.y);
-    }
+    if constexpr (std::is_same<T, float>::value)
+      lds_fft_rule<1, WIDE>(sm, fd, tid, nt);
+    else
+      lds_fft<1, WIDE>(sm, fd, 0, tid, nt);
+    for (int j = pad + tid; j < pad + width; j += nt) st(j, sm[j]);
   }
 }
 
@@ -442,6 +465,18 @@ extern "C" int flt_calc_filter(int64_t ne, const char *name, double *out) {
   return TOMO_OK;
 }
 
+// Threads of a float32 row workgroup with a run-time plan: as few as hold the
+// passes' butterflies where the launch fills the chip, more of them, with fewer
+// butterflies each, where it does not.  us for 100 | 1000 | 4000 workgroups, with
+// as few as possible, 256 and 512 threads: ne = 1152 15.1 11.8 10.8 | 17.6 15.9
+// 24.2 | 42 50 88; 2000 20.8 14.8 12.4 | 24.7 20.3 28.9 | 63 67 104; 4000 (256
+// already) 27.3 | 38.6 | 142 and 19.7 | 48.7 | 177.
+static int rule_threads(const FftDesc &d, int64_t blocks) {
+  const int few = fft_rt_threads(d, 0, false);
+  const int64_t more = blocks <= 256 ? 512 : blocks <= 1024 ? 256 : 0;
+  return few < 0 ? few : (int)std::max<int64_t>(few, std::min(more, ceil_div(d.N, 128) * 64));
+}
+
 extern "C" int flt_create(tomo_flt_plan **plan, int64_t n, int64_t ne, int64_t nproj, int64_t nz,
                           int dtype) {
   clear_error();
@@ -475,7 +510,7 @@ extern "C" int flt_create(tomo_flt_plan **plan, int64_t n, int64_t ne, int64_t n
   P->nproj = nproj;
   P->nz = nz;
   P->dtype = dtype;
-  int rc = P->fft.init((int)ne);
+  int rc = P->fft.init((int)ne, dtype == TOMO_F32);
   if (!rc) rc = P->w.alloc(sizeof(float2) * nz * (ne / 2 + 1));
   if (rc) {
     flt_destroy(P);
@@ -495,23 +530,40 @@ extern "C" int flt_create(tomo_flt_plan **plan, int64_t n, int64_t ne, int64_t n
       return rc;
     }
   }
-  P->threads = fft_rt_threads(P->fft.d, 0);
-  P->lds = sizeof(float2) * (size_t)ne;
+  hipError_t e = hipSuccess;
+  auto shape = [&](auto *t) {
+    using T = typename std::remove_pointer<decltype(t)>::type;
+    with_row_size<T>((int)ne, [&](auto ns) {
+      constexpr int NS = decltype(ns)::value;
+      const bool padded = NS > 0 || std::is_same<T, float>::value;
+      if (NS > 0)
+        P->threads = fft_threads(P->fft.rule, ne);
+      else if (padded)
+        P->threads = rule_threads(P->fft.d, ceil_div(nproj, 2) * nz);
+      else
+        P->threads = fft_rt_threads(P->fft.d, 0);
+      P->lds = sizeof(float2) * (size_t)(padded ? lds_padded_len((int)ne) : ne);
+      if (P->threads <= 0 || P->lds > max_lds_per_block()) return;
+      const void *ks[] = {(const void *)k_flt_rows<0, T, NS, false>,
+                          (const void *)k_flt_rows<1, T, NS, false>,
+                          (const void *)k_flt_rows<0, T, NS, NS == 0>,
+                          (const void *)k_flt_rows<1, T, NS, NS == 0>};
+      for (const void *k : ks)
+        if (e == hipSuccess)
+          e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->lds);
+    });
+  };
+  if (dtype == TOMO_F16)
+    shape((_Float16 *)nullptr);
+  else if (dtype == TOMO_BF16)
+    shape((__bf16 *)nullptr);
+  else
+    shape((float *)nullptr);
   if (P->threads <= 0 || P->lds > max_lds_per_block()) {
     set_error("flt_create: ne=%lld too large for one workgroup", (long long)ne);
     flt_destroy(P);
     return TOMO_EINVAL;
   }
-  const void *rows_kernels[] = {
-      (const void *)k_flt_rows<0, float, false>, (const void *)k_flt_rows<1, float, false>,
-      (const void *)k_flt_rows<0, _Float16, false>, (const void *)k_flt_rows<1, _Float16, false>,
-      (const void *)k_flt_rows<0, __bf16, false>, (const void *)k_flt_rows<1, __bf16, false>,
-      (const void *)k_flt_rows<0, float, true>, (const void *)k_flt_rows<1, float, true>,
-      (const void *)k_flt_rows<0, _Float16, true>, (const void *)k_flt_rows<1, _Float16, true>,
-      (const void *)k_flt_rows<0, __bf16, true>, (const void *)k_flt_rows<1, __bf16, true>};
-  hipError_t e = hipSuccess;
-  for (const void *k : rows_kernels)
-    if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->lds);
   if (e != hipSuccess) {
     set_error("flt_create: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
     flt_destroy(P);
@@ -524,12 +576,17 @@ extern "C" int flt_create(tomo_flt_plan **plan, int64_t n, int64_t ne, int64_t n
 template <int MODE, typename T>
 static void launch_rows(tomo_flt_plan *P, void *g, const float2 *w, hipStream_t st) {
   const dim3 grid((unsigned)ceil_div(P->nproj, 2), (unsigned)P->nz);
-  if (fft_rt_wide(P->fft.d, 0))
-    hipLaunchKernelGGL((k_flt_rows<MODE, T, true>), grid, dim3(P->threads), P->lds, st, (T *)g, w,
-                       P->fft.d, (int)P->ne, (int)P->n, (int)P->nproj);
-  else
-    hipLaunchKernelGGL((k_flt_rows<MODE, T, false>), grid, dim3(P->threads), P->lds, st, (T *)g, w,
-                       P->fft.d, (int)P->ne, (int)P->n, (int)P->nproj);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(P->threads), P->lds, st, (T *)g, w, P->fft.d, (int)P->ne,
+                       (int)P->n, (int)P->nproj);
+  };
+  with_row_size<T>((int)P->ne, [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    if (NS == 0 && fft_rt_wide(P->fft.d, 0))
+      launch(k_flt_rows<MODE, T, NS, NS == 0>);
+    else
+      launch(k_flt_rows<MODE, T, NS, false>);
+  });
 }
 
 template <int MODE>
