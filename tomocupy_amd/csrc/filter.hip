@@ -43,16 +43,37 @@ __global__ void k_flt_weights(const float *__restrict__ wfilter, const float *__
 }
 
 // f(integral_constant<int, ne>) for the lengths whose rows run a compiled
-// transform (none), f(integral_constant<int, 0>) for the others.
+// transform, f(integral_constant<int, 0>) for the others: every power of two from
+// 256, for float32 also those of the usual widths' 4n.  (16-bit rows of these
+// take the run-time plans of few large radices, whose rounding is far below the
+// storage's.)
 template <typename T, typename F>
 void with_row_size(int ne, F &&f) {
+  switch (ne) {
+#define TOMO_SIZE(N) case N: f(std::integral_constant<int, N>()); return;
+    TOMO_SIZE(256) TOMO_SIZE(512) TOMO_SIZE(1024) TOMO_SIZE(2048)
+    TOMO_SIZE(4096) TOMO_SIZE(8192) TOMO_SIZE(16384)
+  }
+  if constexpr (std::is_same<T, float>::value) {
+    switch (ne) {
+      TOMO_SIZE(768) TOMO_SIZE(1280) TOMO_SIZE(1536) TOMO_SIZE(2304) TOMO_SIZE(2560)
+      TOMO_SIZE(3072) TOMO_SIZE(3840) TOMO_SIZE(4608) TOMO_SIZE(5120) TOMO_SIZE(6144)
+      TOMO_SIZE(7680) TOMO_SIZE(9216) TOMO_SIZE(10240) TOMO_SIZE(12288) TOMO_SIZE(15360)
+    }
+  }
+#undef TOMO_SIZE
   f(std::integral_constant<int, 0>());
 }
 
 // mode 0: rows of width ne already padded (cfunc_filter::filter);
 // mode 1: rows of width n, edge-replicate padded on load and cropped on store.
 // NS: ne as a compile-time constant; 0: a run-time plan, of the rule's radices
-// for float32 (lds_fft_rule), of few large ones for 16-bit rows.
+// for float32 (lds_fft_rule), of few large ones for 16-bit rows.  What bounds it is
+// the two transforms' vector arithmetic and LDS.  Unpadded rows, us, compiled and
+// run-time plan (before that plan, per-element passes of the rule's radices): n =
+// 512, 720 angles, 16 slices 40 and 76 (74); 1024, 721, 8 47 and 95 (70); 2048,
+// 1500, 8 238 and 397 (351), float16 256 and 419 (374); 4096, 3000, 2 274 and 471
+// (388).
 template <int MODE, typename T, int NS, bool WIDE>
 __global__ __launch_bounds__(1024) void k_flt_rows(T *__restrict__ g, const float2 *__restrict__ w,
                                                    FftDesc fd, int ne_, int n, int nproj) {
