@@ -71,7 +71,7 @@ void with_row_size(int ne, F &&f) {
 // for float32 (lds_fft_rule), of few large ones for 16-bit rows.  What bounds it is
 // the two transforms' vector arithmetic and LDS.  Unpadded rows, us, compiled and
 // run-time plan (before that plan, per-element passes of the rule's radices): n =
-// 512, 720 angles, 16 slices 40 and 76 (74); 1024, 721, 8 47 and 95 (70); 2048,
+// 512, 720 angles, 16 slices 40 and 69 (74); 1024, 721, 8 47 and 95 (70); 2048,
 // 1500, 8 238 and 397 (351), float16 256 and 419 (374); 4096, 3000, 2 274 and 471
 // (388).
 template <int MODE, typename T, int NS, bool WIDE>
