@@ -82,7 +82,7 @@ void with_ph_size(int N, F &&f) {
 
 // log2 of the columns of a column-pass workgroup: compiled lengths, as many as
 // 512 threads hold in registers, so that two workgroups share a CU and one's
-// loads run under the other's butterflies; run-time lengths, 8
+// loads run under the other's butterflies; run-time lengths, 8 (ph_create)
 constexpr int ph_lg(int N) { return N > 0 ? split_lg(N) - (N > 1024) : 3; }
 // log2 of the columns of a block of the work buffer: 8 or a workgroup's, so
 // that the row passes store and load 128-byte segments (8 columns of 2 rows)
@@ -455,6 +455,14 @@ extern "C" int ph_create(tomo_ph_plan **plan, int64_t dy, int64_t dz, int64_t ba
     P->lgC = ph_lg(decltype(ns)::value);
     P->lgB = ph_lgb(decltype(ns)::value);
   });
+  // Run-time column lengths (below 512): launches of few short columns, which last
+  // as long as a workgroup's chain, so narrow images take 4 columns a workgroup and
+  // all of them many threads.  us for a call, 8 columns with as few threads as hold
+  // the butterflies | 8, 256 threads | 4, 512: 4 images padded to 128 x 128 21.3
+  // 18.7 16.7, 8 to 256 x 256 69.1 54.6 42.4, 8 to 256 x 512 52.2 42.0 33.3, 16 to
+  // 256 x 4096 158 146 208, 32 to 32 x 2048 150 137 183.
+  const bool shortCols = P->Ny < 512, narrow = P->Nx <= 512;
+  if (shortCols && narrow) P->lgC = 2;
   P->Fb = (size_t)std::max(P->Nx / 2, 1 << P->lgB) * dy;
   if (!rc) rc = P->h0.alloc(sizeof(float4) * P->Ny);
   if (!rc) rc = P->F.alloc(sizeof(float2) * (size_t)batch * P->Fb);
@@ -514,6 +522,8 @@ extern "C" int ph_create(tomo_ph_plan **plan, int64_t dy, int64_t dz, int64_t ba
   with_ph_size(P->Nx, [&](auto ns) {
     constexpr int NS = decltype(ns)::value;
     P->rowThreads = NS > 0 ? fft_threads(P->fx.rule, NS) : fft_rt_threads(P->fx.d, 0);
+    if (NS == 0 && P->rowThreads > 0)  // (one value a thread: short rows, as for the columns)
+      P->rowThreads = std::max(P->rowThreads, std::min(256, P->Nx / 64 * 64));
     P->rowLds = sizeof(float2) * (NS > 0 ? lds_padded_len(NS) : P->Nx);
     lds_attr((const void *)k_ph_rows_fwd<NS>, P->rowLds);
     lds_attr((const void *)k_ph_rows_inv<NS>, P->rowLds);
@@ -521,6 +531,9 @@ extern "C" int ph_create(tomo_ph_plan **plan, int64_t dy, int64_t dz, int64_t ba
   with_ph_size(P->Ny, [&](auto ns) {
     constexpr int NS = decltype(ns)::value;
     P->colThreads = NS > 0 ? split_threads(NS, P->lgC) : fft_rt_threads(P->fy.d, P->lgC);
+    if (shortCols && P->colThreads > 0)
+      P->colThreads = std::max(P->colThreads, std::min(narrow ? 512 : 256,
+                                                       (P->Ny << P->lgC) / 128 * 64));
     P->colLds = NS > 0 ? sizeof(float) * ((size_t)lds_padded_len(NS) << P->lgC)
                        : sizeof(float2) * ((size_t)P->Ny << P->lgC);
     lds_attr((const void *)k_ph_cols<NS>, P->colLds);
