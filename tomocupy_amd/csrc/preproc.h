@@ -31,7 +31,7 @@ struct VoBufs {
   }
 };
 
-// Tables and scratch of the Fourier-wavelet stripe removal (stripe.hip),
+// Tables and scratch of the Fourier-wavelet stripe removal's low-rank form (stripe.hip),
 // (re)built when the settings change.
 struct FwPlan {
   std::string name;  // wavelet; empty: nothing built
@@ -51,6 +51,49 @@ struct FwPlan {
     for (DevBuf *b : {&terms, &T, &TS, &A, &P, &B, &row}) b->release();
   }
 };
+
+// One level of the band-by-band form (stripe_bands.hip): analysis input H x W,
+// bands Ho x Wo; the notch keeps nk angular frequencies of the stripe band.
+struct FwLevel {
+  int H = 0, W = 0, Ho = 0, Wo = 0;
+  int nk = 0;
+  int KM = 8;   // notch frequencies a kernel instance holds (8, 16, 32 or 64 >= nk)
+  int R = 4;    // output rows per wave of the column analysis
+  int nrb = 0;  // row blocks of the column analysis
+  DevBuf tw;    // (nk, Ho) float2: cos/sin(2 pi k t / Ho)
+  DevBuf gk;    // (nk,) float: c_k g_k / Ho
+  DevBuf ll;    // (nz, Ho, Wo): low band = input of the next level
+  DevBuf part;  // (nz, nrb, KM, Wo) float2: partial notch DFTs of the stripe band
+  DevBuf X;     // (nz, KM, Wo) float2: notch coefficients, kept until the synthesis
+};
+
+struct FwBands {
+  std::string name;  // wavelet; empty: nothing built
+  int level = 0;
+  double sigma = 0.0;
+  std::vector<FwLevel> lv;
+  DevBuf rowlo, rowhi, synlo, synhi, syn[2];
+  void release() {
+    name.clear();
+    for (auto &l : lv)
+      for (DevBuf *b : {&l.tw, &l.gk, &l.ll, &l.part, &l.X}) b->release();
+    lv.clear();
+    for (DevBuf *b : {&rowlo, &rowhi, &synlo, &synhi, &syn[0], &syn[1]}) b->release();
+  }
+};
+
+// Dark/flat means (k_pre_means output).
+struct DarkFlat {
+  const float *d0, *fa, *fb;
+  int flat_linear;
+};
+
+constexpr int kFwMaxNotch = 64;  // kept notch frequencies per level: sigma up to about 9.8
+
+struct WaveletTaps;
+int fw_bands(tomo_pre_plan *P, const WaveletTaps *wv, double sigma, int level, const void *src,
+             int src_mode, DarkFlat df, void *dst, int dst_mode, int out_dtype, int take_log,
+             hipStream_t st);
 
 // flat0 of a mean flat fa and a mean dark d0: fa * float32(1 + 1e-5) - d0
 // (proc_functions.py:71-72)
@@ -87,6 +130,7 @@ struct tomo_pre_plan {
   int64_t nproj = 0, nz = 0, n = 0, ndark = 0, nflat = 0;
   tomo::DevBuf dark0, flatA, flatB;
   tomo::FwPlan fw;
+  tomo::FwBands fwb;
   tomo::DevBuf outl;  // medians of pre_remove_outliers, allocated on first use
   tomo::DevBuf ti;    // column means and corrections of pre_remove_stripe_ti (first use)
   tomo::VoBufs vo;    // scratch of pre_remove_all_stripe (first use)

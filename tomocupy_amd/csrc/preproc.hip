@@ -373,6 +373,7 @@ extern "C" void pre_destroy(tomo_pre_plan *P) {
   P->flatA.release();
   P->flatB.release();
   P->fw.release();
+  P->fwb.release();
   P->outl.release();
   P->ti.release();
   P->vo.release();

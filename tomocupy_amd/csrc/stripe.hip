@@ -1,5 +1,6 @@
 // Fourier-wavelet stripe removal (tomocupy remove_stripe_fw,
-// src/tomocupy/processing/remove_stripe.py:253-293) for gfx950.
+// src/tomocupy/processing/remove_stripe.py:253-293) for gfx950; scans of few
+// angles take the band-by-band form of stripe_bands.hip (fw_few_angles).
 //
 // Per slice of a (nproj, nz, n) chunk: zero-pad the angles to
 // nproj + nproj/8 (centred), `level` separable DWT levels (detector axis, then
@@ -37,6 +38,7 @@
 // us: 47 + 38 + 52 and 6 for the dark/flat means, against 456 for the filter
 // passes over full-size bands (29 launches); proc_chunk 462 -> 150, whose floor,
 // the counts read and the sinograms written at the rate of a copy, is 29.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -52,7 +54,6 @@ using namespace tomo;
 
 namespace {
 
-constexpr int kMaxNotch = 64;   // kept notch frequencies per level: sigma up to about 9.8
 constexpr int kMaxLevels = 16;
 constexpr int kGroups = 8;      // angle groups (= waves) of a k_fw_project workgroup
 constexpr int kRowTiles = 6;    // 16-term tiles a k_fw_project wave accumulates
@@ -83,12 +84,6 @@ struct AxisLen {
 struct FwTerm {
   int k, q, sin;
   float gk;  // c_q g_q / my
-};
-
-// Dark/flat means (k_pre_means output).
-struct DarkFlat {
-  const float *d0, *fa, *fb;
-  int flat_linear;
 };
 
 // Compile-time filter lengths of the supported wavelets (haar 2, db5 and sym5
@@ -722,16 +717,8 @@ bool orthogonal(const WaveletTaps *wv) {
   return true;
 }
 
-// Tables and scratch for a wavelet, sigma and level count (kept in the plan).
-int setup_fw(tomo_pre_plan *P, const WaveletTaps *wv, double sigma, int level, hipStream_t st) {
-  FwPlan &f = P->fw;
-  if (f.name == wv->name && f.level == level && f.sigma == sigma) return TOMO_OK;
-  const int L = wv->len;
-  const int64_t nz = P->nz, n = P->n, nproj = P->nproj;
-  const int npad = (int)(nproj + nproj / 8);
-  TOMO_REQUIRE(orthogonal(wv), "pre_remove_stripe_fw: wavelet '%s' is not orthogonal", wv->name);
-  const AxisLen H = axis_len(npad, L, level), W = axis_len(n, L, level);
-  std::vector<FwTerm> terms;
+// The terms of a scan whose padded angle axis has the band lengths H.
+int fw_terms(const AxisLen &H, int level, double sigma, std::vector<FwTerm> &terms) {
   for (int k = 0; k < level; ++k) {
     // kept frequencies q <= my/2 with g_q >= 1e-9 (yhat of :276-279)
     const int my = H.N[k + 1];
@@ -748,10 +735,58 @@ int setup_fw(tomo_pre_plan *P, const WaveletTaps *wv, double sigma, int level, h
       terms.push_back(FwTerm{k, q, 0, gk});
       if (!one) terms.push_back(FwTerm{k, q, 1, gk});
     }
-    TOMO_REQUIRE(kept <= kMaxNotch,
+    TOMO_REQUIRE(kept <= kFwMaxNotch,
                  "pre_remove_stripe_fw: sigma=%g keeps %d frequencies at level %d (max %d)", sigma,
-                 kept, k + 1, kMaxNotch);
+                 kept, k + 1, kFwMaxNotch);
   }
+  return TOMO_OK;
+}
+
+// True where the band-by-band form (stripe_bands.hip) is the faster one: scans of
+// few angles and many columns.  Its passes move about S = sum H_k / 2^k rows per
+// column, this form's R terms, each through P and B: with fewer rows than terms
+// the contraction is an expansion.  Both times, in us, are estimated from the
+// counts by a fit to 620 measured calls (8 to 360 angles, 1 to 128 slices of 500 to
+// 11000 columns, sigma 1 to 8, 2 to 7 levels, the three filter lengths), which picks
+// the slower form, by more than 5 %, in 3 % of them; past 360 angles the low-rank
+// form won or tied in all.  Low-rank against bands, sym16, 7 levels: 32 angles, 128
+// slices of 1024, sigma 1 328 against 289, sigma 3 714 against 446; 128 angles, 128 x
+// 2048, sigma 3 1618 against 1267; 24, 8 x 2048, sigma 3 114 against 192; 1500, 8 x
+// 2048, sigma 8 792 against 1758.
+bool fw_few_angles(const tomo_pre_plan *P, const WaveletTaps *wv, double sigma, int level) {
+  if (P->nproj > 360 || P->n > 16000 || P->nz > 65535) return false;  // (a row fits 64 KB)
+  const int L = wv->len;
+  const AxisLen H = axis_len(P->nproj + P->nproj / 8, L, level);
+  std::vector<FwTerm> terms;
+  if (fw_terms(H, level, sigma, terms) != TOMO_OK) return false;  // (setup_fw says why)
+  int kept = 0;
+  for (int k = 0, c = 0; k < level; ++k, kept = std::max(kept, c))
+    c = (int)std::count_if(terms.begin(), terms.end(),
+                           [&](const FwTerm &t) { return t.k == k && !t.sin; });
+  if (terms.empty()) return false;
+  const double R = (double)terms.size(), Rp = (double)(ceil_div((int64_t)R, 32) * 32);
+  const double p = (double)P->nproj, cols = 1e-6 * (double)P->nz * (double)P->n;
+  double S = 0.0;
+  for (int k = 0; k < level; ++k) S += std::ldexp((double)H.N[k], -k);
+  const int KM = kept <= 8 ? 8 : kept <= 16 ? 16 : kept <= 32 ? 32 : 64;
+  const double low = 21 + cols * (17.1 * Rp + 0.028 * Rp * p + 0.158 * R * L + 1.2 * p);
+  const double bands = L == 2    ? 18 + 10 * level + cols * S * (4.0 + 0.223 * KM)
+                       : L == 10 ? 34 + 8.2 * level + cols * (46 + S * (4.6 + 0.348 * KM))
+                                 : 21.5 * level + cols * (337 + S * (3.75 + 0.541 * KM));
+  return bands < low;
+}
+
+// Tables and scratch for a wavelet, sigma and level count (kept in the plan).
+int setup_fw(tomo_pre_plan *P, const WaveletTaps *wv, double sigma, int level, hipStream_t st) {
+  FwPlan &f = P->fw;
+  const int L = wv->len;
+  const int64_t nz = P->nz, n = P->n, nproj = P->nproj;
+  const int npad = (int)(nproj + nproj / 8);
+  TOMO_REQUIRE(orthogonal(wv), "pre_remove_stripe_fw: wavelet '%s' is not orthogonal", wv->name);
+  const AxisLen H = axis_len(npad, L, level), W = axis_len(n, L, level);
+  std::vector<FwTerm> terms;
+  const int rc0 = fw_terms(H, level, sigma, terms);
+  if (rc0) return rc0;
   f.release();
   f.R = (int)terms.size();
   f.Rp = (int)ceil_div(f.R, 32) * 32;
@@ -825,8 +860,19 @@ int fw_run(tomo_pre_plan *P, const WaveletTaps *wv, double sigma, int level, con
            hipStream_t st) {
   TOMO_REQUIRE((src_mode == 0 && dst_mode == 1) || (src_mode == 2 && dst_mode == 2),
                "fw_run: counts to sinograms or the chunk in place");
-  int rc = setup_fw(P, wv, sigma, level, st);
-  if (rc) return rc;
+  int rc;
+  if (!(P->fw.name == wv->name && P->fw.level == level && P->fw.sigma == sigma)) {
+    // new settings, or those of the band-by-band form
+    const FwBands &b = P->fwb;
+    const bool bands = b.name == wv->name && b.level == level && b.sigma == sigma;
+    if (bands || fw_few_angles(P, wv, sigma, level)) {
+      if (!bands) P->fw.release();
+      return fw_bands(P, wv, sigma, level, src, src_mode, df, dst, dst_mode, out_dtype, take_log,
+                      st);
+    }
+    P->fwb.release();
+    if ((rc = setup_fw(P, wv, sigma, level, st))) return rc;
+  }
   const FwPlan &f = P->fw;
   const int L = wv->len, nz = (int)P->nz, nproj = (int)P->nproj, n = (int)P->n;
   hipError_t ea = hipSuccess;
