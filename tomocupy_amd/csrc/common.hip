@@ -66,7 +66,7 @@ double rt_cost(int R) {
 
 }  // namespace
 
-void fft_rt_radices(int N, FftDesc &d) {
+double fft_rt_radices(int N, FftDesc &d, int lgH) {
   d.N = N;
   d.nr = 0;
   // primes above kFftRegPrime first (odd radices: no bank conflicts)
@@ -89,7 +89,7 @@ void fft_rt_radices(int N, FftDesc &d) {
     std::pair<double, int> b{1e30, 0};
     for (int R = 2; R <= kFftRtVals; ++R) {
       if (R == 19 || v % R) continue;
-      if (N / R > 1024 * rt_maxb(R)) continue;
+      if ((N / R) << lgH > 1024 * rt_maxb(R)) continue;
       const auto it = best.find(v / R);
       if (it == best.end()) continue;
       const double c = it->second.first + rt_cost(R);
@@ -99,9 +99,9 @@ void fft_rt_radices(int N, FftDesc &d) {
   }
   for (int v = m; v > 1;) {
     const auto it = best.find(v);
-    if (it == best.end()) {  // not reached for the sizes the callers accept
+    if (it == best.end()) {  // (lgH = 0: not reached for the sizes the callers accept)
       d.nr = 0;
-      return;
+      return 0.0;
     }
     d.r[d.nr++] = it->second.second;
     v /= it->second.second;
@@ -112,6 +112,7 @@ void fft_rt_radices(int N, FftDesc &d) {
     const int la = a & -a, lb = b & -b;
     return la != lb ? la < lb : a > b;
   });
+  return best[m].first;
 }
 
 int FftPlan::init(int N, bool by_rule) {

@@ -64,8 +64,10 @@ struct FftPlan {
   }
 };
 
-// The passes of a run-time plan for length N (no HIP call).
-void fft_rt_radices(int N, FftDesc &d);
+// The cheapest passes of a run-time plan for 2^lgH interleaved transforms of
+// length N (no HIP call, the tables stay); their cost, without the prime passes,
+// or d.nr = 0 where there are none.
+double fft_rt_radices(int N, FftDesc &d, int lgH = 0);
 
 template <int DIR>
 __device__ __forceinline__ float2 mul_i(float2 a) {

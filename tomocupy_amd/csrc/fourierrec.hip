@@ -1359,6 +1359,7 @@ struct tomo_fr_plan {
   int gridChunk = 0;                     // max list entries per gridding work item
   int rowLds = 0, prepLds = 0, fpLds = 0;
   size_t colLds = 0;
+  FftDesc colFft{};                      // the column passes' plan (tables of fft2)
   int lgCBa = 0, colThreadsA = 256;      // k_fr_colfft_adj's lgCB, colThreads, colLds
   size_t colLdsA = 0;
   float scale1 = 0.f, K2 = 0.f;
@@ -1706,6 +1707,7 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
   P->fpLds =
       (int)(P->nsPrep > 0 ? lds_bytes(true, n) << fp_lg((int)n) : lds_bytes(false, n2));
   P->nsCol = 0;
+  P->colFft = P->fft2.d;
   if (st2) {
     // (n is a multiple of the columns: 2^8 divides 2n)
     auto shape = [&](bool split, int &lgs, size_t &lds, int &thr) {
@@ -1732,8 +1734,23 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
     while (P->lgCB < 4 && (lds_bytes(false, n2) << (P->lgCB + 1)) <= maxlds &&
            fft_rt_threads(P->fft2.d, P->lgCB + 1) > 0 && !fft_rt_wide(P->fft2.d, P->lgCB + 1))
       P->lgCB += 1;
+    // Twice the columns, up to 8 (half as many workgroups read a line of R), where
+    // other radices take them at little more arithmetic: one above 10 has one
+    // butterfly a thread, which bars 12, the cheapest, from 2n 2^lgCB = 12289 on.
+    // us for a backprojection and a projection of 4 slices, 40 angles: n = 3456 (2n =
+    // 9 12 8 8 in one column, 18 6 8 8 in two) 2999 and 2478 with one, 2402 and 1892
+    // with two; 1566 536 and 442 with two, 477 and 391 with four.  16 columns for 8
+    // leave too few workgroups: 8 slices of 432 53 against 59.
+    FftDesc more = P->fft2.d, one = P->fft2.d;
+    const double cost = fft_rt_radices((int)n2, one);
+    if (P->lgCB < 3 && (lds_bytes(false, n2) << (P->lgCB + 1)) <= maxlds &&
+        fft_rt_radices((int)n2, more, P->lgCB + 1) <= 1.1 * cost && more.nr > 0 &&
+        fft_rt_threads(more, P->lgCB + 1) > 0 && !fft_rt_wide(more, P->lgCB + 1)) {
+      P->colFft = more;
+      P->lgCB += 1;
+    }
     P->colLds = lds_bytes(false, n2) << P->lgCB;
-    P->colThreads = fft_rt_threads(P->fft2.d, P->lgCB);
+    P->colThreads = fft_rt_threads(P->colFft, P->lgCB);
     P->lgCBa = P->lgCB;
     P->colLdsA = P->colLds;
     P->colThreadsA = P->colThreads;
@@ -1869,7 +1886,7 @@ static int fr_tail_after_grid(tomo_fr_plan *P, T *obj, hipStream_t st) {
                          dim3((unsigned)ceil_div(n, P->colCB), ng * 4),
                          dim3(P->colThreads),
                          P->colLds, st, R, obj, P->phix.as<float>(), P->phiy.as<float>(),
-                         P->circ.as<int2>(), P->fft2.d, n, nz, nzc, P->lgCB, P->lgB > 0 ? 1 : 0);
+                         P->circ.as<int2>(), P->colFft, n, nz, nzc, P->lgCB, P->lgB > 0 ? 1 : 0);
     });
   }
   TOMO_LAUNCH_CHECK();
@@ -2220,7 +2237,7 @@ extern "C" int fr_forward(tomo_fr_plan *P, void *data_, const void *obj_, void *
                          dim3(P->colThreadsA), P->colLdsA, st, obj,
                          P->R.as<float2>(),
                          P->phix.as<float>(), P->phiy.as<float>(), P->circ.as<int2>(),
-                         P->fft2.d, n, nz, nzc, P->lgCBa);
+                         P->colFft, n, nz, nzc, P->lgCBa);
     });
   }
   TOMO_LAUNCH_CHECK();
