@@ -1,6 +1,6 @@
 """Column passes whose run-time plan differs from the row pass's, so that a
 workgroup takes twice the columns (two, four and eight; with and without a large
-prime), against the FP64 oracle.
+prime), and compiled 16-bit ones on a column-blocked array, against the FP64 oracle.
 
 Tolerance: as for every run-time plan, three transforms of at most five passes of
 about 1e-7 of the row's rms each, random: below 1e-6, asserted at 2e-6; float16 six
@@ -19,8 +19,12 @@ def _rel(a, b):
     return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
-@pytest.mark.parametrize('n', [816, 840, 912, 1060, 1560, 1776, 2060, 3096, 3456])
-@pytest.mark.parametrize('dtype', ['float32', 'float16'])
+WIDTHS = [816, 840, 912, 1060, 1560, 1776, 2060, 3096, 3456]
+CASES = [(n, dt) for n in WIDTHS for dt in ('float32', 'float16')]
+CASES += [(n, 'float16') for n in (640, 768, 1152, 1280)]
+
+
+@pytest.mark.parametrize('n,dtype', CASES)
 def test_backprojection_and_projection(n, dtype):
     nproj, nz = 3, 2
     rng = np.random.default_rng(n)

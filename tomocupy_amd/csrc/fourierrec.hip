@@ -1766,21 +1766,23 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
   // R column-blocked (log2 of the block) or row-major, us per chunk of 8
   // slices, row + column pass. The column pass gains contiguous reads, the
   // row pass loses its long stores, so blocks pay where a workgroup's columns
-  // cover less than a 128-byte line of a row and the split column pass reads
-  // them: float32, 8 columns: 2n = 4096 164+147 against 149+174 row-major,
-  // 3840 199+165 against 183+195; 4 columns (32-byte segments): 5120 408+298
-  // against 314+367 and 6144 573+405 against 421+516, so row-major, except at
-  // 8192, where the 2^15-byte row stride puts a column into few memory
-  // channels: 782+533 against 729+1181. 16-bit, 4 or 8 columns: 2n = 2560
-  // 70+60 against 67+71, 4096 170+117 against 160+134, 5120 335+274 against
-  // 305+356, 8192 977+437 against 816+620; 16 columns (2048): 38+31 against
-  // 36+30, so row-major. Without a compiled column pass 16-bit R is blocked
-  // as before.
+  // cover less than a 128-byte line of a row and, in float32, the split column
+  // pass reads them. float32, 8 columns: 2n = 4096 164+147 against 149+174
+  // row-major, 3840 199+165 against 183+195; 4 columns (32-byte segments): 5120
+  // 408+298 against 314+367 and 6144 573+405 against 421+516, so row-major, except
+  // at 8192, where the 2^15-byte row stride puts a column into few memory
+  // channels: 782+533 against 729+1181. 16-bit, 4 or 8 columns: 1280 23+22 against
+  // 23+24, 1536 32+28 against 31+29, 2304 58+42 against 56+48, 2560 69+60 against
+  // 68+70, 4096 170+117 against 160+134, 5120 335+274 against 305+356, 8192 977+437
+  // against 816+620; 16 columns (2048): 38+31 against 36+30, so row-major. Without a
+  // compiled column pass 16-bit R is blocked as before.
   const bool pow2 = (n & (n - 1)) == 0;
-  if (P->nsCol > 0)
-    P->lgB = col_split((int)n2) && lg < 4 && (dtype != TOMO_F32 || lg == 3 || pow2) ? lg : 0;
-  else
+  if (P->nsCol == 0)
     P->lgB = (dtype != TOMO_F32 && n % (1 << lg) == 0) ? lg : 0;
+  else if (dtype != TOMO_F32)
+    P->lgB = lg < 4 ? lg : 0;
+  else
+    P->lgB = col_split((int)n2) && lg < 4 && (lg == 3 || pow2) ? lg : 0;
   hipError_t ea = hipSuccess;
   auto lds_attr = [&](const void *k, size_t bytes) {
     if (ea == hipSuccess)
