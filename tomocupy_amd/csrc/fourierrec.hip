@@ -1585,11 +1585,13 @@ int build_tables(tomo_fr_plan *P, const std::vector<float> &theta) {
 }
 
 
-// Workgroup shapes of the FFT passes for width n, from the radix sequences
-// alone (no HIP call): the detector pass (n points), the row pass (2n) and
-// the column pass (2n, one column per workgroup at least) each need at most
-// 512 threads at their values per thread.  Rejects e.g. n = 4000
-// (2n = 2^6 5^3: 15 values per thread in the radix-5 passes, 576 threads).
+// The accepted widths n, from the rule's radix sequences alone (no HIP call): the
+// detector transform (n points), the row transform (2n) and one column of the
+// column pass (2n) each take at most 512 threads at 16 values per thread (32 in the
+// column pass of 2^a 3^b), 15, 14, 11 or 13 with a radix-3 or 5, 7, 11 or 13 pass.
+// Rejects e.g. n = 4000 (2n = 2^6 5^3, 576 threads).  The compiled transforms have
+// these shapes; the run-time plans have others (fft_rt_threads) and would run the
+// 107 rejected widths of 2838 .. 4096 too, but the set of widths stays.
 int fr_fft_shapes_ok(int64_t n) {
   FftRule d1{}, d2{};
   int rc = FftPlan::radices((int)n, d1);
@@ -1604,8 +1606,8 @@ int fr_fft_shapes_ok(int64_t n) {
               {"column (2n-point)", fft_threads(d2, 2 * n, colEPT)}};
   for (const auto &q : need)
     TOMO_REQUIRE(q.threads > 0 && q.threads <= 512,
-                 "fr_create: n=%lld: the %s FFT pass needs more than 512 threads per workgroup "
-                 "(its radix-3/5/7/11/13 passes cover fewer than 16 values per thread)",
+                 "fr_create: n=%lld is not an accepted width: at 16 values per thread (fewer with "
+                 "a radix-3/5/7/11/13 pass) its %s FFT takes more than 512 threads",
                  (long long)n, q.pass);
   return TOMO_OK;
 }
@@ -1760,8 +1762,12 @@ extern "C" int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int
   }
   P->colCB = 1 << P->lgCB;
   const int lg = P->lgCB;
-  if (P->colThreads <= 0 || P->prepThreads <= 0 || P->rowThreads <= 0 || P->fpThreads <= 0 ||
-      P->colLds > maxlds) {
+  // (the image kernels have no prime passes of 16 pairs: no length up to 8192 needs them)
+  const bool wide = (P->nsPrep == 0 && fft_rt_wide(P->fft1.d, 0)) ||
+                    (P->nsRow == 0 && fft_rt_wide(P->fft2.d, 0)) ||
+                    (P->nsCol == 0 && fft_rt_wide(P->colFft, P->lgCB));
+  if (wide || P->colThreads <= 0 || P->prepThreads <= 0 || P->rowThreads <= 0 ||
+      P->fpThreads <= 0 || P->colLds > maxlds) {
     set_error("fr_create: n=%lld needs more threads or LDS than an FFT workgroup has",
               (long long)n);
     return fail(TOMO_EINVAL);
