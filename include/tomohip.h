@@ -118,9 +118,11 @@ int fr_create(tomo_fr_plan **plan, int64_t n, int64_t nproj, int64_t nz,
  * plan autotuner, tomocupy_amd/autotune.py).  Both options change only the
  * rounding of the results; each configuration is deterministic.
  *   grid_chunk   max sample-list entries per gridding work item: 0 = default
- *                (512), else a multiple of 64 in [64, 8192]
+ *                (128, 256, 512 or 768, by the entries per resident wave), else a
+ *                multiple of 64 in [64, 8192]
  *   fft_generic  1 = run-time radix plans for every FFT, 0 = compiled
- *                size-specialised transforms where 2n is 1024..8192
+ *                size-specialised transforms where 2n is one of the lengths
+ *                2^a 3^b 5^c of with_static_size (csrc/fft_lds.h), 256..8192
  */
 int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int64_t nz,
                    const float *theta, int dtype, int grid_chunk, int fft_generic,

@@ -240,14 +240,6 @@ __device__ __forceinline__ void twiddle(float2 *a, const float2 *__restrict__ tw
     a[2] = cmul(a[2], w2);
     a[3] = cmul(a[3], cmul(w2, w1));
     a[4] = cmul(a[4], w4);
-  } else if constexpr (R == 7) {
-    const float2 w1 = ld(1), w2 = ld(2), w4 = ld(4);
-    a[1] = cmul(a[1], w1);
-    a[2] = cmul(a[2], w2);
-    a[3] = cmul(a[3], cmul(w2, w1));
-    a[4] = cmul(a[4], w4);
-    a[5] = cmul(a[5], cmul(w4, w1));
-    a[6] = cmul(a[6], cmul(w4, w2));
   } else if constexpr (R == 4) {
     const float2 w1 = ld(1), w2 = ld(2);
     a[1] = cmul(a[1], w1);
@@ -282,8 +274,10 @@ __device__ __forceinline__ void twiddle(float2 *a, const float2 *__restrict__ tw
 // one would turn every table read into a FLAT access).  The call's convention
 // spends 87 registers on the 64 a pass needs (5 waves per SIMD); inlined, the
 // switch spilled.  n = 2448 (2n = 17 18 16), 8 slices x 1500 angles, us, row
-// pass / column pass / filter and spectrum: 378 / 528 / 349, against 1211 /
-// 1123 / 1065 with radices 16, 2, 3, 3, 17 and per-element index arithmetic.
+// pass / column pass / filter and spectrum: 378 / 528 / 283, against 1211 /
+// 1123 / 1065 with radices 16, 2, 3, 3, 17 and per-element index arithmetic (of the
+// filter's 1065, 349 were left by the plans, the rest went with its transforms of
+// 2n points).
 
 typedef float f2v __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) f2v *LdsPtr;
@@ -1006,7 +1000,7 @@ __device__ __forceinline__ void chain_last(const float2 *buf, const float2 *__re
 constexpr int kFftSplitEPT = 32;
 
 // log2 of the sequences a split workgroup takes: as many as 1024 threads hold,
-// at most 16 (15 of a thread's values in the radix-3 and 5 passes).
+// at most 16 (30 of a thread's values in the radix-3 and 5 passes).
 constexpr int split_lg(int N) {
   return ilog2c(1024 * kFftSplitEPT / N) > 4 ? 4 : ilog2c(1024 * kFftSplitEPT / N);
 }

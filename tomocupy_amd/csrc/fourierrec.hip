@@ -51,7 +51,7 @@ constexpr int kColEPT = 32;     // column-pass values per thread in the width ru
 // as fit 512 threads at kColEPT values each (and the LDS), at most 16
 constexpr int col_lg(int N) { return ilog2c(16384 / N) > 4 ? 4 : ilog2c(16384 / N); }
 // 2n = N whose column passes run fft_c_split (split_lg(N) columns): the sizes
-// where the split gives a workgroup twice the columns and at least 24 waves'
+// where the split gives a workgroup twice the columns and at least 12 waves'
 // worth of values (row + column pass, us per chunk of 8 slices, float32, split
 // against fft_c_global: 2n = 2048 39+37 against 39+41, 3072 109+103 against
 // 99+123, 8192 782+533 against 729+1181; 2304, whose 8 columns are 18432
@@ -1059,19 +1059,16 @@ __global__ __launch_bounds__(1024) void k_fr_colfft(const cpx<T> *__restrict__ R
         [&](int idx, cpx<T> v) {
           const int a = idx >> lgCB, t = idx & (CB - 1);
           const float2 x = tof2(v);
-          sm[(lidx<NS>(a) << lgCB) + t] = (a & 1) ? make_float2(-x.x, -x.y) : x;
+          sm[(a << lgCB) + t] = (a & 1) ? make_float2(-x.x, -x.y) : x;
         });
     __syncthreads();
-    if constexpr (NS > 0)
-      lds_fft_c<NS, 1, kFftEPT, col_lg(NS)>(sm, fd.tw, tid, nt);
-    else
-      lds_fft<1>(sm, fd, lgCB, tid, nt);
+    lds_fft<1>(sm, fd, lgCB, tid, nt);
     for (int idx = tid; idx < CB * n; idx += nt) {
       const int ty = idx >> lgCB, t = idx & (CB - 1);
       const int tx = v0 + t;
       if (tx >= n) continue;
       const int u = ty + 1 + h;
-      float2 x = sm[(lidx<NS>(u) << lgCB) + t];
+      float2 x = sm[(u << lgCB) + t];
       const int2 ci = circ[ty];
       const float ph = (tx >= ci.x && tx < ci.y) ? phix[tx] * phiy[ty] * ((u & 1) ? -1.f : 1.f) : 0.f;
       str(obj + ((size_t)c * n + ty) * n + tx, x.x * ph);

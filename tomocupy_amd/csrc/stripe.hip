@@ -32,7 +32,7 @@
 //   k_fw_detector  P_r -> B_r, one workgroup per term and slice, all levels
 //   k_fw_apply     x_0 + A B, a matrix product with K = terms, fused with the
 //                  dark/flat correction, -log and the swap to sinograms
-// At sigma = 1 and 7 levels there are 92 terms; the two products are 9 GFLOP
+// At sigma = 1 and 7 levels there are 83 terms (96 padded); the products are 9 GFLOP
 // per 8 slices of 2048 x 1500, far below what the matrix cores take for the
 // bytes of x_0.  Measured, 8 slices of 2048 x 1500 (sym16, 7 levels, sigma 1),
 // us: 47 + 38 + 52 and 6 for the dark/flat means, against 456 for the filter
@@ -64,7 +64,7 @@ constexpr int kApplyCols = 128; // columns of a k_fw_apply workgroup (32 per wav
 // low-pass (as given, DWTInverse, :221-225) is a too, and both high-passes are
 // b[j] = (-1)^j a[L - 1 - j].  One set of taps, 64 scalar registers, stays
 // resident through k_fw_detector (four sets spilled to vector lanes: 50 us
-// against 46 at 92 terms x 8 slices x 2048).
+// against 46 at 83 terms x 8 slices x 2048).
 struct Taps {
   double a[32];
 };
@@ -446,7 +446,7 @@ __device__ __forceinline__ void synthesis2(const double *x, const Taps &t, int q
 // parts in matrix-operand order [z][part][r / 8][nPad][r % 8]; terms past the
 // last one are zero.  Bound by the chain of up to 2 (k + 1) dependent passes:
 // the mirrored margins are written with the bands, so that a pass is one round
-// of constant-offset LDS reads and one barrier (38 us at 92 terms x 8 slices x
+// of constant-offset LDS reads and one barrier (38 us at 83 terms x 8 slices x
 // 2048 columns; 63 with the reflection worked out per read).
 template <int L, bool GLOB>
 __global__ __launch_bounds__(256) void k_fw_detector(const double *__restrict__ P,
