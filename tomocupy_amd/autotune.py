@@ -5,11 +5,11 @@ backprojection (``fr_filter_backprojection``) under each candidate plan
 configuration on synthetic data of that shape and returns the fastest:
 
 * ``grid_chunk``: the longest sample list one gridding wave walks before the
-  tile is split into partial tiles that a reduction pass sums (64..2048
+  tile is split into partial tiles that a reduction pass sums (128..2048
   entries); short chunks balance the heavily loaded tiles near the spectrum's
   centre, long ones avoid partial-tile traffic;
-* ``fft``: compiled size-specialised transforms (``'static'``, power-of-two
-  sizes 1024..8192) or run-time radix plans (``'generic'``).
+* ``fft``: compiled size-specialised transforms (``'static'``, where 2n is one
+  of the compiled lengths 2^a 3^b 5^c up to 8192) or run-time radix plans (``'generic'``).
 
 Both options change only the rounding of the results (the order in which the
 partial sums of a heavy tile are added, the radix sequence of a transform);
@@ -22,7 +22,7 @@ import os
 
 from . import _lib
 
-GRID_CHUNKS = (128, 256, 512, 1024, 2048)
+GRID_CHUNKS = (128, 256, 512, 768, 1024, 2048)  # the defaults fr_create chooses from, and longer
 FFTS = ('static', 'generic')
 
 
