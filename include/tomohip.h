@@ -129,6 +129,15 @@ int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int64_t nz,
                    void *stream);
 
 /*
+ * Says that the plan's launches run at the same time as others (a batch, several
+ * streams; no counterpart in the reference): rows is the number of sinogram rows of
+ * this width, angles times pairs of slices, in all of them together, 0 = the plan's
+ * own.  Kernels chosen for launches that leave the chip idle are then not taken.
+ * Changes only the rounding of the results.
+ */
+int fr_share(tomo_fr_plan *plan, int64_t rows);
+
+/*
  * Replaces FourierRec.backprojection(obj, data, stream)
  * (fourierrec.py:61-68) and cfunc_fourierrec::backprojection
  * (cfunc_fourierrec.cu:67-93).

@@ -207,7 +207,10 @@ __global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_prep(const T *__rest
 // reconstruction, WIDE minus register form: n = 256 and 512 -3.7 and -10.4 at
 // 200 rows, -3.0 and -3.7 at 1800, +3.4 and +3.9 at 3600; n = 768 and 1024 -4.5
 // and -3.7 at 200, -4.3 and -2.8 at 1200, +1.6 and +3.5 at 1800; n = 1280 -0.6
-// at 200 and 1536 -2.3, +11.8 and +11.7 at 1200, so not beyond 1024.
+// at 200 and 1536 -2.3, +11.8 and +11.7 at 1200, so not beyond 1024.  Launches that
+// run at the same time fill the chip together, so their rows count together
+// (fr_share; 16 requests of n = 512, 500 angles, 8 slices: 1014 us with the 256-thread
+// form, 927 without).
 constexpr int kFpWideMax = 1024, kFpWideThreads = 256;
 inline bool fp_wide(int n, int64_t rows) {
   return n <= kFpWideMax && rows <= (n <= 512 ? 2304 : 1536);
@@ -1357,6 +1360,7 @@ struct tomo_fr_plan {
   int nsRow = 0, nsCol = 0, nsPrep = 0;  // compiled FFT sizes in use (0 = run-time sizes)
   int lgB = 0;                           // column-blocked R (see k_fr_rowfft)
   int gridChunk = 0;                     // max list entries per gridding work item
+  int64_t shareRows = 0;                 // fr_share
   int rowLds = 0, prepLds = 0, fpLds = 0;
   size_t colLds = 0;
   FftDesc colFft{};                      // the column passes' plan (tables of fft2)
@@ -1929,7 +1933,7 @@ static int fr_head(tomo_fr_plan *P, tomo_flt_plan *F, const T *data, hipStream_t
                          F->HR.as<float>(), F->fft2n.d.tw, P->fft1.d, n, nproj, nz, nzc,
                          P->scale1, P->gmax.as<float>());
     };
-    const bool wide = fp_wide(n, (int64_t)nproj * nzc);
+    const bool wide = fp_wide(n, std::max((int64_t)nproj * nzc, P->shareRows));
     with_static_size(P->nsPrep, [&](auto ns) {
       constexpr int NS = decltype(ns)::value;
       if constexpr (NS > 0 && NS <= kFpWideMax) {
@@ -2310,6 +2314,14 @@ extern "C" void fr_destroy(tomo_fr_plan *P) {
   P->fft1.release();
   P->fft2.release();
   delete P;
+}
+
+extern "C" int fr_share(tomo_fr_plan *P, int64_t rows) {
+  clear_error();
+  TOMO_REQUIRE(P != nullptr, "fr_share: plan is NULL");
+  TOMO_REQUIRE(rows >= 0, "fr_share: rows < 0");
+  P->shareRows = rows;
+  return TOMO_OK;
 }
 
 extern "C" int fr_get_sizes(const tomo_fr_plan *P, int64_t *n, int64_t *nproj, int64_t *nz) {
