@@ -124,7 +124,7 @@ int FftPlan::init(int N, bool by_rule) {
     std::copy(rule.r, rule.r + rule.nr, d.r);
   }
   TOMO_REQUIRE(d.nr > 0 && fft_rt_threads(d, 0) > 0, "FFT length %d has no run-time plan", N);
-  std::vector<float> mat;
+  std::vector<double> mat;
   size_t off[3] = {0, 0, 0};
   int np = 0;
   for (int i = 0; i < d.nr; ++i) {
@@ -137,21 +137,24 @@ int FftPlan::init(int N, bool by_rule) {
     if (np > 0 && d.r[np - 1] == p) {
       off[np] = off[np - 1];
     } else {
-      mat.resize(mat.size() + (size_t)2 * h * hp, 0.f);
+      mat.resize(mat.size() + (size_t)2 * h * hp, 0.0);
       for (int j = 1; j <= h; ++j)
         for (int q = 1; q <= h; ++q) {
           const double ang = 2.0 * M_PI * (double)((j * q) % p) / (double)p;
-          float *e = &mat[off[np] + 2 * ((size_t)(j - 1) * hp + q - 1)];
-          e[0] = (float)std::cos(ang);
-          e[1] = (float)std::sin(ang);
+          double *e = &mat[off[np] + 2 * (size_t)(j - 1) * hp];
+          e[by_rule ? q - 1 : 2 * (q - 1)] = std::cos(ang);
+          e[by_rule ? hp + q - 1 : 2 * (q - 1) + 1] = std::sin(ang);
         }
     }
     ++np;
   }
   if (!mat.empty()) {
-    if ((rc = pm.alloc(sizeof(float) * mat.size()))) return rc;
-    TOMO_HIP(hipMemcpy(pm.p, mat.data(), sizeof(float) * mat.size(), hipMemcpyHostToDevice));
-    for (int i = 0; i < np; ++i) d.pm[i] = pm.as<float>() + off[i];
+    const std::vector<float> single(mat.begin(), mat.end());
+    const size_t sz = by_rule ? sizeof(double) : sizeof(float);
+    if ((rc = pm.alloc(sz * mat.size()))) return rc;
+    TOMO_HIP(hipMemcpy(pm.p, by_rule ? (const void *)mat.data() : single.data(), sz * mat.size(),
+                       hipMemcpyHostToDevice));
+    for (int i = 0; i < np; ++i) d.pm[i] = pm.as<char>() + sz * off[i];
   }
   std::vector<float2> h(N);
   for (int k = 0; k < N; ++k) {

@@ -38,7 +38,8 @@ struct FftDesc {
   int nr;
   int r[kFftMaxRadices];
   const float2 *tw;    // device, N entries
-  const float *pm[3];  // cosine/sine matrices of the primes above kFftRegPrime, in pass order
+  const void *pm[3];  // cosine/sine matrices of the primes above kFftRegPrime, in pass order
+                      // (float pairs; FftPlan::init by_rule: columns of double)
 };
 
 // The radix sequence of the compiled sizes; for every size the sequence by
@@ -283,6 +284,7 @@ typedef float f2v __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) f2v *LdsPtr;
 typedef const __attribute__((address_space(1))) f2v *TabPtr;
 typedef const __attribute__((address_space(4))) float *ScalarPtr;
+typedef const __attribute__((address_space(4))) double *ScalarPtr64;
 
 __device__ __forceinline__ float2 ldf2(LdsPtr p) {
   const f2v v = *p;
@@ -586,17 +588,123 @@ __device__ __noinline__ void rt_pass_prime(LdsPtr buf, int N_, int Ns_, int p_, 
   __syncthreads();
 }
 
-// The prime pass with the output pairs a wave takes.
+// The same in 64 bits between the LDS reads and writes, for one transform: P_j and
+// M_j are rounded once, the sums too, and the cosines and sines are doubles (`pm`:
+// row j has hp cosines, then hp sines).  Roundings of each step, and of the (p-1)/2
+// constants, whose error all terms share, show where the result is what is left of
+// much larger inputs, the high frequencies of a smooth row: noisy sinogram rows of
+// ellipses, ramp, ne = 2840 (71), 2.7e-6 with floats, 2.4e-6 as one sum with the
+// length's table, 2.15e-6 now.  What bounds it is the multiply-adds, at
+// the rate of float ones; the cosine sums are finished before the sine sums begin
+// (a third fewer registers).  8 x 720 rows of ne = 2840: 175 us with floats, 998 as
+// one sum, 212 now.
+template <int G, int DIR>
+__device__ __noinline__ void rt_pass_prime64(LdsPtr buf, int N_, int Ns_, int p_, TabPtr tw,
+                                             const double *pm_, int tid, int nt_) {
+  const int N = __builtin_amdgcn_readfirstlane(N_), Ns = __builtin_amdgcn_readfirstlane(Ns_);
+  const int p = __builtin_amdgcn_readfirstlane(p_), nt = __builtin_amdgcn_readfirstlane(nt_);
+  const uintptr_t pa = (uintptr_t)pm_;
+  const unsigned plo = __builtin_amdgcn_readfirstlane((unsigned)pa);
+  const unsigned phi = __builtin_amdgcn_readfirstlane((unsigned)(pa >> 32));
+  const ScalarPtr64 pm = (ScalarPtr64)(((uintptr_t)phi << 32) | plo);
+  const int h = (p - 1) / 2, hp = rt_prime_cols(p);
+  const int nb = N / p, twstep = nb / Ns;
+  for (int e = tid; e < nb * h; e += nt) {
+    const int jj = e / nb, g = e - jj * nb, kt = g % Ns * twstep;
+    const LdsPtr x = buf + g + (jj + 1) * nb, y = buf + g + (p - 1 - jj) * nb;
+    const float2 u = ldf2(x), v = ldf2(y);
+    float2 wu = ldf2(tw + kt * (jj + 1)), wv = ldf2(tw + kt * (p - 1 - jj));
+    if (DIR > 0) wu.y = -wu.y, wv.y = -wv.y;
+    const double ux = (double)u.x * wu.x - (double)u.y * wu.y;
+    const double uy = (double)u.x * wu.y + (double)u.y * wu.x;
+    const double vx = (double)v.x * wv.x - (double)v.y * wv.y;
+    const double vy = (double)v.x * wv.y + (double)v.y * wv.x;
+    stf2(x, make_float2((float)(ux + vx), (float)(uy + vy)));
+    stf2(y, make_float2((float)(ux - vx), (float)(uy - vy)));
+  }
+  __syncthreads();
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int nblk = (nb + 63) / 64, grp = w / nblk;
+  const int g = (w - grp * nblk) * 64 + lane;
+  const bool live = grp * G < h && g < nb;
+  float2 re[G], y0;
+  double Sx[G], Sy[G];
+  if (live) {
+    const float2 a0 = ldf2(buf + g);
+    double y0x = a0.x, y0y = a0.y;
+#pragma unroll
+    for (int u = 0; u < G; ++u) Sx[u] = a0.x, Sy[u] = a0.y;
+#pragma unroll 1
+    for (int j = 0; j < h; ++j) {
+      const float2 P = ldf2(buf + g + (j + 1) * nb);
+      const double px = P.x, py = P.y;
+      const ScalarPtr64 m = pm + 2 * j * hp + grp * G;
+      y0x += px;
+      y0y += py;
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+        Sx[u] = fma(m[u], px, Sx[u]);
+        Sy[u] = fma(m[u], py, Sy[u]);
+      }
+    }
+    y0 = make_float2((float)y0x, (float)y0y);
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      re[u] = make_float2((float)Sx[u], (float)Sy[u]);
+      Sx[u] = Sy[u] = 0.0;
+    }
+#pragma unroll 1
+    for (int j = 0; j < h; ++j) {
+      const float2 M = ldf2(buf + g + (p - 1 - j) * nb);
+      const double mx = M.x, my = M.y;
+      const ScalarPtr64 m = pm + (2 * j + 1) * hp + grp * G;
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+        Sx[u] = fma(m[u], mx, Sx[u]);
+        Sy[u] = fma(m[u], my, Sy[u]);
+      }
+    }
+  }
+  __syncthreads();
+  if (live) {
+    const int jq = g / Ns, k = g - jq * Ns;
+    LdsPtr o = buf + jq * Ns * p + k;
+    if (grp == 0) stf2(o, y0);
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      const int q = grp * G + u + 1;
+      if (q > h) break;
+      const float2 mi = mul_i<DIR>(make_float2((float)Sx[u], (float)Sy[u]));
+      stf2(o + q * Ns, cadd(re[u], mi));
+      stf2(o + (p - q) * Ns, csub(re[u], mi));
+    }
+  }
+  __syncthreads();
+}
+
+// The prime passes with the output pairs a wave takes.
 template <int DIR, bool WIDE>
 __device__ __forceinline__ void rt_prime(LdsPtr buf, int N, int Ns, int R, TabPtr tw,
-                                         const float *pm, int lgH, int tid, int nt) {
+                                         const void *pm, int lgH, int tid, int nt) {
   const int G = rt_prime_pairs((N / R) << lgH, R);
   if (WIDE && G == 16)
-    rt_pass_prime<16, DIR>(buf, N, Ns, R, tw, pm, lgH, tid, nt);
+    rt_pass_prime<16, DIR>(buf, N, Ns, R, tw, (const float *)pm, lgH, tid, nt);
   else if (G == 12)
-    rt_pass_prime<12, DIR>(buf, N, Ns, R, tw, pm, lgH, tid, nt);
+    rt_pass_prime<12, DIR>(buf, N, Ns, R, tw, (const float *)pm, lgH, tid, nt);
   else
-    rt_pass_prime<8, DIR>(buf, N, Ns, R, tw, pm, lgH, tid, nt);
+    rt_pass_prime<8, DIR>(buf, N, Ns, R, tw, (const float *)pm, lgH, tid, nt);
+}
+
+template <int DIR, bool WIDE>
+__device__ __forceinline__ void rt_prime64(LdsPtr buf, int N, int Ns, int R, TabPtr tw,
+                                           const void *pm, int tid, int nt) {
+  const int G = rt_prime_pairs(N / R, R);
+  if (WIDE && G == 16)
+    rt_pass_prime64<16, DIR>(buf, N, Ns, R, tw, (const double *)pm, tid, nt);
+  else if (WIDE && G == 12)
+    rt_pass_prime64<12, DIR>(buf, N, Ns, R, tw, (const double *)pm, tid, nt);
+  else
+    rt_pass_prime64<8, DIR>(buf, N, Ns, R, tw, (const double *)pm, tid, nt);
 }
 
 // In-place transform of 2^lgH interleaved sequences of length d.N held in LDS
@@ -634,9 +742,10 @@ __device__ void lds_fft(float2 *buf_, const FftDesc &d, int lgH, int tid, int nt
 // radix is a product with factors between.  What is left of the row's mean
 // then sits in one of their outputs.  (Relative error of a ramp-filtered row of
 // ellipses without noise, ne = 1016: 1.5e-5 with fft_rt_radices' order, 127
-// first, against 7.6e-6; 9792 6.6e-5 against 6.0e-5; white rows, ne = 4000:
+// first, against 7.6e-6, 6.6e-6 with its pass in 64 bits; 9792 6.6e-5 against 6.0e-5; white rows, ne = 4000:
 // 2.1e-7 against 1.8e-7.)  A first pass of a power of two writes with a pad
-// slot per 16 elements: its writes, R apart, would meet the same banks.
+// slot per 16 elements: its writes, R apart, would meet the same banks.  WIDE: also
+// the prime passes of 12 and 16 pairs a wave (120 registers against 85).
 template <int DIR, bool WIDE>
 __device__ void lds_fft_rule(float2 *buf_, const FftDesc &d, int tid, int nt) {
   const LdsPtr buf = (LdsPtr)buf_;
@@ -669,7 +778,7 @@ __device__ void lds_fft_rule(float2 *buf_, const FftDesc &d, int tid, int nt) {
       TOMO_RT_PASS(2) TOMO_RT_PASS(3) TOMO_RT_PASS(4) TOMO_RT_PASS(5) TOMO_RT_PASS(7)
       TOMO_RT_PASS(8) TOMO_RT_PASS(11) TOMO_RT_PASS(13) TOMO_RT_PASS(16) TOMO_RT_PASS(17)
 #undef TOMO_RT_PASS
-      default: rt_prime<DIR, WIDE>(buf, N, Ns, R, tw, d.pm[np++], 0, tid, nt);
+      default: rt_prime64<DIR, WIDE>(buf, N, Ns, R, tw, d.pm[np++], tid, nt);
     }
     Ns *= R;
   }
@@ -696,12 +805,13 @@ inline int fft_rt_threads(const FftDesc &d, int lgH, bool one_each = true) {
   return t > 1024 ? -1 : (int)t;
 }
 
-// True if the plan has a prime pass of 16 pairs a wave (lds_fft's WIDE).
-inline bool fft_rt_wide(const FftDesc &d, int lgH) {
+// True if the plan has a prime pass of `pairs` pairs a wave or more: 16 for lds_fft's
+// WIDE, 12 for lds_fft_rule's.
+inline bool fft_rt_wide(const FftDesc &d, int lgH, int pairs = 16) {
   bool wide = false;
   for (int i = 0; i < d.nr; ++i) {
     const int R = d.r[i];
-    wide |= (R > kFftRtVals || R == 19) && rt_prime_pairs((d.N / R) << lgH, R) == 16;
+    wide |= (R > kFftRtVals || R == 19) && rt_prime_pairs((d.N / R) << lgH, R) >= pairs;
   }
   return wide;
 }

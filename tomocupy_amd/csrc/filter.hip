@@ -603,7 +603,7 @@ static void launch_rows(tomo_flt_plan *P, void *g, const float2 *w, hipStream_t 
   };
   with_row_size<T>((int)P->ne, [&](auto ns) {
     constexpr int NS = decltype(ns)::value;
-    if (NS == 0 && fft_rt_wide(P->fft.d, 0))
+    if (NS == 0 && fft_rt_wide(P->fft.d, 0, std::is_same<T, float>::value ? 12 : 16))
       launch(k_flt_rows<MODE, T, NS, NS == 0>);
     else
       launch(k_flt_rows<MODE, T, NS, false>);
