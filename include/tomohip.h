@@ -129,10 +129,10 @@ int fr_create_opts(tomo_fr_plan **plan, int64_t n, int64_t nproj, int64_t nz,
                    void *stream);
 
 /*
- * Says that the plan's launches run at the same time as others (a batch, several
- * streams; no counterpart in the reference): rows is the number of sinogram rows of
- * this width, angles times pairs of slices, in all of them together, 0 = the plan's
- * own.  Kernels chosen for launches that leave the chip idle are then not taken.
+ * Says that the plan's launches run beside others (a batch, several streams; no
+ * counterpart in the reference): the choice of kernels then counts rows, angles times
+ * pairs of slices, instead of the plan's own if they are more; 0 = the plan's own.
+ * Kernels chosen for launches that leave the chip idle are then taken less often.
  * Changes only the rounding of the results.
  */
 int fr_share(tomo_fr_plan *plan, int64_t rows);

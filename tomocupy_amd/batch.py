@@ -70,13 +70,15 @@ class BatchRec:
                 'data': torch.zeros((nz, nproj, n), dtype=td, device='cuda'),
                 'obj': torch.zeros((nz, n, n), dtype=td, device='cuda'),
                 'cost': request_bytes(n, nproj, nz, dtype)})
-        # Two requests' filters run at the same time on average (four streams, between
-        # other kernels): 16 of n = 512, 2000 rows each, 1014 us as if alone, 927 with
-        # the kernels of long launches; 8 of 720 rows 330 as if alone, 347 with those.
-        pair = (min(2, len(self.items)) * sum(it['n'] * it['nproj'] * ((it['nz'] + 1) // 2)
-                                              for it in self.items)) // len(self.items)
-        for it in self.items:
-            _lib.check(_lib.lib().fr_share(it['bf'].cl_rec._handle(), pair // it['n']), 'fr_share')
+        # Requests' filters run beside other requests' kernels (four streams), so the line
+        # between the two forms of the filter lies at fewer rows than for one alone: 7/4
+        # times its rows count.  12 equal requests of 8 slices, us with the 256-thread form
+        # and without: n = 512, 1000 rows 569 and 573, 1400 657 and 624, 2000 787 and 727;
+        # n = 768, 700 rows 1044 and 1042, 900 1092 and 1070; n = 1024, 900 rows 1511 and
+        # 1490, 1140 1573 and 1533.
+        for it in self.items if len(self.items) > 1 else ():
+            rows = it['nproj'] * ((it['nz'] + 1) // 2)
+            _lib.check(_lib.lib().fr_share(it['bf'].cl_rec._handle(), rows * 7 // 4), 'fr_share')
         self.streams = [torch.cuda.Stream() for _ in range(max(1, int(streams)))]
         # longest processing time first onto the least loaded stream
         load = [0] * len(self.streams)

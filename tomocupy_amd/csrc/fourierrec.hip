@@ -207,10 +207,9 @@ __global__ __launch_bounds__(NS > 0 ? 512 : 1024) void k_fr_prep(const T *__rest
 // reconstruction, WIDE minus register form: n = 256 and 512 -3.7 and -10.4 at
 // 200 rows, -3.0 and -3.7 at 1800, +3.4 and +3.9 at 3600; n = 768 and 1024 -4.5
 // and -3.7 at 200, -4.3 and -2.8 at 1200, +1.6 and +3.5 at 1800; n = 1280 -0.6
-// at 200 and 1536 -2.3, +11.8 and +11.7 at 1200, so not beyond 1024.  Launches that
-// run at the same time fill the chip together, so their rows count together
-// (fr_share; 16 requests of n = 512, 500 angles, 8 slices: 1014 us with the 256-thread
-// form, 927 without).
+// at 200 and 1536 -2.3, +11.8 and +11.7 at 1200, so not beyond 1024.  Beside other
+// launches the line lies at fewer rows (fr_share; 16 requests of n = 512, 500 angles,
+// 8 slices on streams: 974 us with the 256-thread form, 883 without).
 constexpr int kFpWideMax = 1024, kFpWideThreads = 256;
 inline bool fp_wide(int n, int64_t rows) {
   return n <= kFpWideMax && rows <= (n <= 512 ? 2304 : 1536);
