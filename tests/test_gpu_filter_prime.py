@@ -78,3 +78,22 @@ def test_no_worse_than_the_sum(p):
     got = np.linalg.norm(d.cpu().numpy().astype(np.float64) - ref)
     print('p=%d error %.3g of the sum %.3g' % (p, got, emulated))
     assert got <= 1.05 * emulated
+
+
+@pytest.mark.parametrize('ne', [9804, 10184, 14964, 15544, 15776, 16376])
+def test_twelve_and_sixteen_pairs(ne):
+    """Lengths whose prime passes take 12 or 16 output pairs a wave, white rows.  Two
+    transforms of at most five passes, each about 1e-7 of the values: 1e-7 sqrt(10)."""
+    from tomocupy_amd.fbp_filter import FBPFilter
+    rng = np.random.default_rng(ne)
+    rows = rng.standard_normal((2, 5, ne)).astype(F4)
+    gain = rng.uniform(0.5, 1, ne // 2 + 1) * np.exp(1j * rng.uniform(-3, 3, ne // 2 + 1))
+    gain[0] = gain[-1] = 1
+    gain = gain.astype(C8)
+    ref = np.fft.irfft(np.fft.rfft(rows.astype(np.float64)) * gain, n=ne) * ne
+    flt = FBPFilter(ne, 5, 2, n_unpadded=ne // 8 * 2)
+    d = torch.from_numpy(rows).cuda()
+    flt.filter(d, torch.from_numpy(gain).cuda().expand(2, -1).contiguous())
+    err = np.linalg.norm(d.cpu().numpy() - ref) / np.linalg.norm(ref)
+    print('ne=%d error %.3g' % (ne, err))
+    assert err <= 1e-7 * np.sqrt(10)

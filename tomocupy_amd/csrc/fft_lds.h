@@ -594,10 +594,9 @@ __device__ __noinline__ void rt_pass_prime(LdsPtr buf, int N_, int Ns_, int p_, 
 // constants, whose error all terms share, show where the result is what is left of
 // much larger inputs, the high frequencies of a smooth row: noisy sinogram rows of
 // ellipses, ramp, ne = 2840 (71), 2.7e-6 with floats, 2.4e-6 as one sum with the
-// length's table, 2.15e-6 now.  What bounds it is the multiply-adds, at
-// the rate of float ones; the cosine sums are finished before the sine sums begin
-// (a third fewer registers).  8 x 720 rows of ne = 2840: 175 us with floats, 998 as
-// one sum, 212 now.
+// length's table, 2.15e-6 now.  What bounds it is the multiply-adds, at the rate of
+// float ones; the cosine sums are finished before the sine sums begin (a third fewer
+// registers).  8 x 720 rows of ne = 2840: 175 us with floats, 998 as one sum, 212 now.
 template <int G, int DIR>
 __device__ __noinline__ void rt_pass_prime64(LdsPtr buf, int N_, int Ns_, int p_, TabPtr tw,
                                              const double *pm_, int tid, int nt_) {
@@ -741,11 +740,11 @@ __device__ void lds_fft(float2 *buf_, const FftDesc &d, int lgH, int tid, int nt
 // two come first, whose differences of near-equal values are exact, and no
 // radix is a product with factors between.  What is left of the row's mean
 // then sits in one of their outputs.  (Relative error of a ramp-filtered row of
-// ellipses without noise, ne = 1016: 1.5e-5 with fft_rt_radices' order, 127
-// first, against 7.6e-6, 6.6e-6 with its pass in 64 bits; 9792 6.6e-5 against 6.0e-5; white rows, ne = 4000:
-// 2.1e-7 against 1.8e-7.)  A first pass of a power of two writes with a pad
-// slot per 16 elements: its writes, R apart, would meet the same banks.  WIDE: also
-// the prime passes of 12 and 16 pairs a wave (120 registers against 85).
+// ellipses without noise, ne = 1016: 1.5e-5 with fft_rt_radices' order, 127 first,
+// against 7.6e-6, 6.6e-6 with its pass in 64 bits; 9792 6.6e-5 against 6.0e-5; white
+// rows, ne = 4000: 2.1e-7 against 1.8e-7.)  A first pass of a power of two writes
+// with a pad slot per 16 elements: its writes, R apart, would meet the same banks.
+// WIDE: also the prime passes of 12 and 16 pairs a wave (120 registers against 85).
 template <int DIR, bool WIDE>
 __device__ void lds_fft_rule(float2 *buf_, const FftDesc &d, int tid, int nt) {
   const LdsPtr buf = (LdsPtr)buf_;
@@ -822,11 +821,11 @@ inline bool fft_rt_wide(const FftDesc &d, int lgH, int pairs = 16) {
 // N = 2^k 3^a 5^b with 2^k >= 256.  The radices are those FftPlan::radices
 // picks: radix 16 passes, one radix 8/4/2 pass for the remaining power of
 // two, then the radix-3 and radix-5 passes, so every sub-transform length Ns
-// is 1 or a multiple of 16 (its index splits are divisions by constants).  With one pad slot per 16 elements, the R reads of a butterfly
-// (stride N/R, a multiple of 16) and its R writes (stride Ns, a multiple of
-// 16, or consecutive when Ns = 1) sit at constant offsets from one base
-// address, so a pass costs one address computation per butterfly instead of
-// one per element.
+// is 1 or a multiple of 16 (its index splits are divisions by constants).  With one
+// pad slot per 16 elements, the R reads of a butterfly (stride N/R, a multiple of
+// 16) and its R writes (stride Ns, a multiple of 16, or consecutive when Ns = 1) sit
+// at constant offsets from one base address, so a pass costs one address
+// computation per butterfly instead of one per element.
 constexpr int ilog2c(int x) { return x <= 1 ? 0 : 1 + ilog2c(x / 2); }
 
 constexpr int count_factor(int x, int p) { return x % p == 0 ? 1 + count_factor(x / p, p) : 0; }
