@@ -257,9 +257,9 @@ struct ColumnFlat {
 // the six products down to 2^-16 of a product.
 //
 // What bounds it (47 us per 8 slices of 2048 x 1500; 26 with one tile pair
-// instead of six, so half is the loads' latency and the split): vector work
-// (the quotient and the split, about 12 instructions per value) plus matrix
-// work (11 us), with the 49 MB of counts beside them; T is re-read from L2 for each
+// instead of six): vector work (the quotient and the split, about 12 instructions per
+// value) for 36 % of the cycles, matrix work (11 us) for 24 %, which do not overlap,
+// and between them the loads' latency; T is re-read from L2 for each
 // 16 CT columns.  CT = 4 (half the reads of T, but 2 waves per SIMD instead of
 // 4) measured 52 us against 46.
 template <int SRC, int CT>
